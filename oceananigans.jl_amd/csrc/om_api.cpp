@@ -451,10 +451,12 @@ template <class T> struct ModelT : ModelBase {
         // the Fourier–tridiagonal plan serves the FT solver and, on stretched z, the CG preconditioner
         P.tridiagonal = (c.pressure_solver == OM_SOLVER_FOURIER_TRIDIAGONAL ||
                          (c.pressure_solver == OM_SOLVER_CONJUGATE_GRADIENT && hg.stretched)) ? 1 : 0;
-        P.zmode = g.tz != OM_BOUNDED ? 0 : (g.Nz % 2 == 0 ? 1 : 2);
-        P.Lz_line = P.zmode == 2 ? 2 * g.Nz : g.Nz;
+        P.zmode = g.tz == OM_BOUNDED ? 1 : 0;
         P.Lz_norm = g.tz == OM_BOUNDED ? 2 * g.Nz : g.Nz;
-        P.tw_z = upload(twiddles<T>(P.Lz_line));
+        P.tw_z = upload(twiddles<T>(g.Nz));
+        P.st_x = upload(fft_stages(xline));
+        P.st_y = upload(fft_stages(g.Ny));
+        P.st_z = upload(fft_stages(g.Nz));
         {
             std::vector<typename Vec2<T>::type> c(g.Nz);
             for (int k = 0; k < g.Nz; ++k) {
@@ -618,7 +620,7 @@ template <class T> struct ModelT : ModelBase {
             PhaseScope ps(this, OM_PHASE_HALOS);
             for (int f = 0; f < 3; ++f) launch_mask(g, s.U[f], f + 1, st);
         }
-        if (defer && !cg && !tune_refine && g.tz == OM_BOUNDED && poisson_source_reads_no_halo(P, ctx()))
+        if (defer && !cg && !tune_refine && poisson_source_reads_no_halo(ctx()))
             u_halo_pending = true;
         else
             halos_prognostic(0x7u, true);
@@ -651,8 +653,7 @@ template <class T> struct ModelT : ModelBase {
         // periodic x and y without an immersed bottom or a refinement pass: the correction reads
         // p's neighbours across the edges by wrapped index, and p's halo fill joins the next
         // halo launch (update_state's), one launch fewer per substage
-        const bool wrap = !tune_refine && !g.kbot && g.tx == OM_PERIODIC && g.ty == OM_PERIODIC &&
-                          (g.tz == OM_BOUNDED || g.tz == OM_PERIODIC);
+        const bool wrap = !tune_refine && !g.kbot && g.tx == OM_PERIODIC && g.ty == OM_PERIODIC;
         if (!wrap) halos_aux({s.pNHS});
         { PhaseScope ps(this, OM_PHASE_CORRECTION); launch_correct(ctx(), dtp, 0, st, wrap ? 1 : 0); }
         p_halo_pending = wrap;
@@ -1657,7 +1658,7 @@ int om_autotune(om_model_t *m, int32_t *kchunk) {
 // overlap another's compute-bound ones.
 struct BatchGroup {
     std::vector<size_t> members;      // indices into the ensemble's member list
-    std::vector<void *> tables;       // device argument tables, one per position
+    std::vector<void *> tables;       // device argument tables, one per position and variant
     hipGraphExec_t exec = nullptr;
     hipStream_t st = nullptr;
 };
@@ -1750,34 +1751,45 @@ void build_plan(om_ensemble *e, double dt) {
     for (BatchGroup &grp : P.groups) {
         HIPCHECK(hipStreamCreateWithFlags(&grp.st, hipStreamNonBlocking));
         const int gn = (int)grp.members.size();
-        std::vector<uint32_t> blocks(npos);
-        std::vector<size_t> lds(npos);
+        // the launches of the sequence: one per position and variant of its kernel
+        struct Launch {
+            const LaunchRec *r;
+            void *table;
+            int n;
+            uint32_t blocks;
+            size_t lds;
+        };
+        std::vector<Launch> launches;
         for (size_t p = 0; p < npos; ++p) {
-            const size_t es = rec[0].recs[p].entry_size;
-            std::vector<unsigned char> host(es * gn);
-            uint64_t begin = 0;
-            size_t l = 0;
-            for (int q = 0; q < gn; ++q) {
-                const LaunchRec &r = rec[grp.members[q]].recs[p];
-                const uint64_t nb = (uint64_t)r.grid.x * r.grid.y * r.grid.z;
-                r.fill(host.data() + q * es, r, (uint32_t)begin);
-                begin += (nb + 7) & ~uint64_t(7);   // member ranges start on a multiple of 8 (XCD residue kept)
-                l = std::max(l, r.lds);
+            std::vector<char> done(gn, 0);
+            for (int first = 0; first < gn; ++first) {
+                if (done[first]) continue;
+                const LaunchRec &r0 = rec[grp.members[first]].recs[p];
+                const size_t es = r0.entry_size;
+                std::vector<unsigned char> host(es * gn);
+                uint64_t begin = 0;
+                size_t l = 0;
+                int n = 0;
+                for (int q = first; q < gn; ++q) {
+                    const LaunchRec &r = rec[grp.members[q]].recs[p];
+                    if (done[q] || r.launch_many != r0.launch_many) continue;
+                    done[q] = 1;
+                    const uint64_t nb = (uint64_t)r.grid.x * r.grid.y * r.grid.z;
+                    r.fill(host.data() + n++ * es, r, (uint32_t)begin);
+                    begin += (nb + 7) & ~uint64_t(7);   // member ranges start on a multiple of 8 (XCD residue kept)
+                    l = std::max(l, r.lds);
+                }
+                if (begin > 0x7fffffffull) throw ArgError{"the ensemble's launch has more than 2^31 blocks"};
+                void *t = nullptr;
+                HIPCHECK(hipMalloc(&t, n * es));
+                grp.tables.push_back(t);
+                HIPCHECK(hipMemcpy(t, host.data(), n * es, hipMemcpyHostToDevice));
+                launches.push_back(Launch{&r0, t, n, (uint32_t)begin, l});
             }
-            if (begin > 0x7fffffffull) throw ArgError{"the ensemble's launch has more than 2^31 blocks"};
-            void *t = nullptr;
-            HIPCHECK(hipMalloc(&t, host.size()));
-            grp.tables.push_back(t);
-            HIPCHECK(hipMemcpy(t, host.data(), host.size(), hipMemcpyHostToDevice));
-            blocks[p] = (uint32_t)begin;
-            lds[p] = l;
         }
         hipGraph_t gr = nullptr;
         HIPCHECK(hipStreamBeginCapture(grp.st, hipStreamCaptureModeThreadLocal));
-        for (size_t p = 0; p < npos; ++p) {
-            const LaunchRec &r = rec[grp.members[0]].recs[p];
-            r.launch_many(grp.tables[p], gn, blocks[p], r.block, lds[p], grp.st);
-        }
+        for (const Launch &L : launches) L.r->launch_many(L.table, L.n, L.blocks, L.r->block, L.lds, grp.st);
         HIPCHECK(hipStreamEndCapture(grp.st, &gr));
         const hipError_t ei = hipGraphInstantiate(&grp.exec, gr, nullptr, nullptr, 0);
         (void)hipGraphDestroy(gr);

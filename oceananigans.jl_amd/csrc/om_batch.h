@@ -18,6 +18,7 @@
 #include <stdint.h>
 
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace om {
@@ -55,7 +56,7 @@ __global__ void __launch_bounds__(K::kThreads, K::kMinBlocks) k_many(const Batch
 // recording
 // ---------------------------------------------------------------------------------------------
 struct LaunchRec {
-    const void *kind;                                  // identifies (K, A): &launch_many<K, A>
+    const void *kind;                                  // identifies K's family and A
     dim3 grid, block;
     size_t lds;
     std::vector<unsigned char> args;                   // the A bytes
@@ -83,10 +84,17 @@ template <class K, class A> void batch_launch_many(const void *tab, int n, uint3
     hipLaunchKernelGGL((k_many<K, A>), dim3(blocks), block, lds, st, static_cast<const BatchEntry<A> *>(tab), n);
 }
 
+// A kernel kind may name a family (`using Family = …`): variants that do the same work of the step on
+// members of different sizes.  Members whose recorded launches agree in kind share a position of a
+// batch; launch_many tells the variants apart, and each variant is one launch of that position.
+template <class K, class = void> struct KindFamily { using type = K; };
+template <class K> struct KindFamily<K, std::void_t<typename K::Family>> { using type = typename K::Family; };
+template <class F, class A> inline const char kind_tag = 0;
+
 template <class K, class A> void launch_k(dim3 grid, dim3 block, size_t lds, hipStream_t st, const A &a) {
     if (Recorder *R = thread_recorder()) {
         LaunchRec r;
-        r.kind = reinterpret_cast<const void *>(&batch_launch_many<K, A>);
+        r.kind = &kind_tag<typename KindFamily<K>::type, A>;
         r.grid = grid; r.block = block; r.lds = lds;
         r.args.resize(sizeof(A));
         std::memcpy(r.args.data(), &a, sizeof(A));

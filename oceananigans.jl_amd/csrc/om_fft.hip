@@ -6,11 +6,11 @@
 //   X-forward  : source term (∇·U* formed on the fly, optionally ×Δzᶜ) → real-to-complex FFT
 //   Y-forward  : complex FFT along y                    (skipped when y is the last axis)
 //   last axis  : forward transform · eigenvalue division · backward transform in one kernel
-//                (Bounded z: DCT-II / DCT-III pair through one complex FFT of length Nz, or the
-//                 2Nz-point even extension for odd Nz; Fourier–tridiagonal: Thomas algorithm)
+//                (Bounded z: DCT-II / DCT-III pair through one complex FFT of length Nz;
+//                 Fourier–tridiagonal: Thomas algorithm)
 //   Y-backward, X-backward (complex-to-real, written into the pressure field's interior)
 // Each line transform is an in-place radix-4 Stockham FFT in LDS for power-of-two lengths and a
-// direct DFT otherwise; the global loads that stage the lines are batched per thread.  Reference: src/Solvers/fft_based_poisson_solver.jl:94-124,
+// mixed-radix Stockham FFT between two LDS buffers otherwise; the global loads that stage the lines are batched per thread.  Reference: src/Solvers/fft_based_poisson_solver.jl:94-124,
 // src/Solvers/fourier_tridiagonal_poisson_solver.jl:231-260, src/Solvers/batched_tridiagonal_solver.jl:211-243.
 #include <hip/hip_runtime.h>
 
@@ -51,19 +51,142 @@ __device__ __forceinline__ void staged_copy(int count, Get get, Put put) {
     }
 }
 
-// R lines of length n, row r at a + r·ld; tw (in LDS) holds exp(-2πi m / n), m < n.
-// Power-of-two n: in-place Stockham stages of radix 4 (one radix-2 stage first when log2 n is
-// odd).  A radix-R stage at sub-length m maps a[kk + jj·m + p·n/R] (p < R) to
+// Butterfly of P points, P odd: y_q = Σ_p c_p e^{∓2πi pq/P}, from the sums and differences of the
+// pairs (c_k, c_{P−k}): y_q, y_{P−q} = A ∓ iB (forward) with A = c_0 + Σ_k cos(2πkq/P) (c_k + c_{P−k}) and
+// B = Σ_k sin(2πkq/P) (c_k − c_{P−k}).  cs, sn: cos and sin of 2πm/P, m = 0 .. P−1.
+template <int P> struct OddTable;
+template <> struct OddTable<3> {
+    static constexpr double cs[3] = {1.0, -0.5, -0.5};
+    static constexpr double sn[3] = {0.0, 0.86602540378443864676, -0.86602540378443864676};
+};
+template <> struct OddTable<5> {
+    static constexpr double cs[5] = {1.0, 0.30901699437494742410, -0.80901699437494742410, -0.80901699437494742410, 0.30901699437494742410};
+    static constexpr double sn[5] = {0.0, 0.95105651629515357212, 0.58778525229247312917, -0.58778525229247312917, -0.95105651629515357212};
+};
+template <> struct OddTable<7> {
+    static constexpr double cs[7] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624,
+                                     -0.90096886790241912624, -0.22252093395631440429, 0.62348980185873353053};
+    static constexpr double sn[7] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048,
+                                     -0.43388373911755812048, -0.97492791218182360702, -0.78183148246802980871};
+};
+template <class T, int P> __device__ __forceinline__ void butterfly(C2<T> (&c)[P], bool inverse) {
+    if constexpr (P == 2) {
+        const C2<T> t = csub<T>(c[0], c[1]);
+        c[0] = cadd<T>(c[0], c[1]);
+        c[1] = t;
+    } else if constexpr (P == 4) {
+        const C2<T> t0 = cadd<T>(c[0], c[2]), t1 = csub<T>(c[0], c[2]), t2 = cadd<T>(c[1], c[3]), d = csub<T>(c[1], c[3]);
+        const C2<T> t3 = inverse ? cmk<T>(-d.y, d.x) : cmk<T>(d.y, -d.x);   // ±i·(c1 − c3)
+        c[0] = cadd<T>(t0, t2);
+        c[1] = cadd<T>(t1, t3);
+        c[2] = csub<T>(t0, t2);
+        c[3] = csub<T>(t1, t3);
+    } else {
+        constexpr int H = (P - 1) / 2;
+        C2<T> sp[H], dm[H];
+#pragma unroll
+        for (int k = 1; k <= H; ++k) {
+            sp[k - 1] = cadd<T>(c[k], c[P - k]);
+            dm[k - 1] = csub<T>(c[k], c[P - k]);
+        }
+        const C2<T> c0 = c[0];
+#pragma unroll
+        for (int k = 0; k < H; ++k) c[0] = cadd<T>(c[0], sp[k]);
+#pragma unroll
+        for (int q = 1; q <= H; ++q) {
+            C2<T> A = c0, B = cmk<T>(T(0), T(0));
+#pragma unroll
+            for (int k = 1; k <= H; ++k) {
+                const T cs = T(OddTable<P>::cs[k * q % P]), sn = T(OddTable<P>::sn[k * q % P]);
+                A.x += cs * sp[k - 1].x;
+                A.y += cs * sp[k - 1].y;
+                B.x += sn * dm[k - 1].x;
+                B.y += sn * dm[k - 1].y;
+            }
+            if (inverse) B = cmk<T>(-B.x, -B.y);
+            c[q] = cmk<T>(A.x + B.y, A.y - B.x);       // A − iB
+            c[P - q] = cmk<T>(A.x - B.y, A.y + B.x);   // A + iB
+        }
+    }
+}
+
+// One Stockham stage of radix P on R lines of length n, a → b: at sub-length m the butterfly
+// bf = kk + jj·m (kk < m) of a line takes a[bf + p·n/P] to b[kk + (jj·P + q)·m], times w^{q·jj·m}.
+// The butterflies of all lines are one flat range; bf and jj come from multiplications by the
+// stage's reciprocals (exact for the ranges here, see FftStage).
+template <class T, int P>
+__device__ __forceinline__ void fft_stage(const C2<T> *a, C2<T> *b, int R, int n, int ld, const C2<T> *tw, bool inverse,
+                                          const FftStage &S) {
+    const int nb = n / P, m = (int)S.m;
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));   // keeps each radix's index arithmetic inside its own case
+#pragma unroll 1
+    for (; t < R * nb; t += blockDim.x) {
+        const int row = nb == 1 ? t : (int)__umulhi((uint32_t)t, S.mul_b), bf = t - row * nb;
+        const int jj = m == 1 ? bf : (int)__umulhi((uint32_t)bf, S.mul_m), kk = bf - jj * m;
+        const C2<T> *src = a + row * ld + bf;
+        C2<T> c[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) c[p] = src[p * nb];
+        butterfly<T, P>(c, inverse);
+        C2<T> *dst = b + row * ld + kk + jj * P * m;
+        const int e = jj * m;
+        dst[0] = c[0];
+#pragma unroll
+        for (int q = 1; q < P; ++q) {
+            C2<T> w = tw[q * e];
+            if (inverse) w.y = -w.y;
+            dst[q * m] = cmul<T>(w, c[q]);
+        }
+    }
+}
+
+// The same stage for any radix: one output per thread, a direct sum over the P inputs.
+template <class T>
+__device__ __forceinline__ void fft_stage_any(const C2<T> *a, C2<T> *b, int R, int n, int ld, const C2<T> *tw, bool inverse,
+                                              const FftStage &S) {
+    const int P = (int)S.radix, nb = n / P, m = (int)S.m;
+#pragma unroll 1
+    for (int t = threadIdx.x; t < R * n; t += blockDim.x) {
+        const int row = t / n, o = t - row * n;
+        const int v = o / m, kk = o - v * m, jj = v / P, q = v - jj * P;
+        const C2<T> *src = a + row * ld + kk + jj * m;
+        C2<T> s = src[0];
+        int f = 0;
+#pragma unroll 2
+        for (int p = 1; p < P; ++p) {
+            f += q;
+            if (f >= P) f -= P;
+            C2<T> w = tw[f * nb];
+            if (inverse) w.y = -w.y;
+            s = cadd<T>(s, cmul<T>(src[p * nb], w));
+        }
+        C2<T> w = tw[q * jj * m];
+        if (inverse) w.y = -w.y;
+        b[row * ld + o] = cmul<T>(w, s);
+    }
+}
+
+// R lines of length n, row r at a + r·ld; tw (in LDS) holds exp(-2πi m / n), m < n.  Returns the
+// buffer that holds the (unnormalised) transform.
+// MIXED = false, power-of-two n: in-place Stockham stages of radix 4 (one radix-2 stage first when
+// log2 n is odd).  A radix-R stage at sub-length m maps a[kk + jj·m + p·n/R] (p < R) to
 // a[kk + R·jj·m + q·m] = w^{q·jj·m} Σ_p c_p e^{∓2πi pq/R}; every thread reads its butterflies'
 // inputs into registers, the block synchronises, and the outputs overwrite the same buffer, so
 // one buffer serves every stage.  Each thread holds at most 2 radix-4 (4 radix-2) butterflies:
 // R·n ≤ 8·blockDim.x.  Index splits are shifts and masks.
-// Other n: a direct DFT into b.  Returns the buffer that holds the (unnormalised) transform.
-template <class T>
-__device__ C2<T> *lds_fft(C2<T> *a, C2<T> *b, int R, int n, int ld, const C2<T> *tw, bool inverse) {
+// MIXED = true, other n: the stages of the plan (radices 7, 5, 3, then any prime above 7 as a direct
+// sum of that length, then 4 and 2), each from one buffer to the other.  LDS traffic and barriers
+// bound it (an FP32 y pass of 192 × 192 × 96 takes 14 µs, 3.9 TB/s, against 318 µs as direct sums of
+// 192 terms; the z pass of 150 × 100 × 75 12 µs against 284 as a 150-point even extension).
+// The two are separate kernels: in one, the radix-7 butterfly's registers would halve the blocks a
+// CU holds of the power-of-two passes too (98 VGPRs against 54).
+template <class T, bool MIXED>
+__device__ __forceinline__ C2<T> *lds_fft(C2<T> *a, C2<T> *b, int R, int n, int ld, const C2<T> *tw, bool inverse,
+                       const FftStage *__restrict__ stages) {
     const int nt = blockDim.x;
     const int tid = threadIdx.x;
-    if ((n & (n - 1)) == 0) {
+    if constexpr (!MIXED) {
         const int lg = __builtin_ctz((unsigned)n);
         int lm = 0;   // log2 of the current sub-length m
         if (lg & 1) {
@@ -130,25 +253,32 @@ __device__ C2<T> *lds_fft(C2<T> *a, C2<T> *b, int R, int n, int ld, const C2<T> 
             __syncthreads();
         }
         return a;
-    }
-    for (int t = tid; t < R * n; t += nt) {
-        const int r = t / n, ko = t - r * n;
-        C2<T> s = cmk<T>(T(0), T(0));
-        for (int q = 0; q < n; ++q) {
-            C2<T> w = tw[(int)(((int64_t)ko * q) % n)];
-            if (inverse) w.y = -w.y;
-            s = cadd<T>(s, cmul<T>(a[r * ld + q], w));
+    } else {
+#pragma unroll 1
+        for (int q = 0;; ++q) {
+            const FftStage S = stages[q];
+            switch (S.radix) {
+                case 0: return a;
+                case 2: fft_stage<T, 2>(a, b, R, n, ld, tw, inverse, S); break;
+                case 3: fft_stage<T, 3>(a, b, R, n, ld, tw, inverse, S); break;
+                case 4: fft_stage<T, 4>(a, b, R, n, ld, tw, inverse, S); break;
+                case 5: fft_stage<T, 5>(a, b, R, n, ld, tw, inverse, S); break;
+                case 7: fft_stage<T, 7>(a, b, R, n, ld, tw, inverse, S); break;
+                default: fft_stage_any<T>(a, b, R, n, ld, tw, inverse, S);
+            }
+            __syncthreads();
+            C2<T> *t = a;
+            a = b;
+            b = t;
         }
-        b[r * ld + ko] = s;
     }
-    __syncthreads();
-    return b;
 }
 
 template <class T> __device__ __forceinline__ void load_table(C2<T> *dst, const C2<T> *src, int n) {
     staged_copy<4>(n, [&](int t) { return src[t]; }, [&](int t, C2<T> v) { dst[t] = v; });
 }
 
+constexpr int kXFwdBatch = 4;      // elements per thread and batch of loads of the X-forward source
 constexpr int kFftThreads = 512;   // threads per block of the line kernels (a multiple of R ≤ 16)
 
 // Line staging geometry, chosen on the host: R lines per block, row stride ld (n + 1 when R > 1,
@@ -168,15 +298,22 @@ template <class T> struct XFwdArgs {
     const T *src;
     C2<T> *S;
     const C2<T> *tw;      // length Nx/2 table (for the half-length complex FFT), Nx when Nx is odd
+    const FftStage *stages;   // of the line length of tw
     const C2<T> *post;    // exp(-2πi k / Nx), k = 0 .. Nx/2
     int scale_dzc;
+    // FP32: form the cancelling sum of the divergence with its rounding errors (cancelling_sum).  The
+    // velocity differences of a nearly divergence-free flow cancel to a small part of each;
+    // rounded term by term they leave white noise of ε|U|/Δx, which the inverse Laplacian amplifies
+    // at the longest waves: most of the FP32 pressure's error (1.1e-5 against 2e-6 of FP64 at
+    // 192 × 192 × 96 stretched).  On for grids with a line that is not a power of two; where all are,
+    // the sum stays as it was and so do the results, bit for bit.
+    int compensated;
     LineGeom L;
     FastDiv fNy, fMx;
     int Ms;
 };
 
-template <class T> __device__ __forceinline__ T source_at(const Ctx<T> &C, const T *src, int i, int j, int k) {
-    if (src) return src[(int64_t)i + (int64_t)C.g.Nx * ((int64_t)j + (int64_t)C.g.Ny * k)];
+template <class T> __device__ __forceinline__ T source_at(const Ctx<T> &C, int i, int j, int k) {
     // divergence with periodic index wrap in x and y (halos of U* are not needed)
     const int ip = (i + 1 == C.g.Nx) ? 0 : i + 1;
     const int jp = (j + 1 == C.g.Ny) ? 0 : j + 1;
@@ -190,11 +327,38 @@ template <class T> __device__ __forceinline__ T source_at(const Ctx<T> &C, const
     return C.iVc(k) * ((sx + sy) + sz);
 }
 
-template <class T> struct KXFwd {
+// A₁(a₁ − b₁) + A₂(a₂ − b₂) + A₃(a₃ − b₃) rounded (nearly) once: each difference and product with its
+// rounding error (Knuth's two-sum; the product's by FMA), the errors summed beside the values.
+__device__ __forceinline__ float cancelling_sum(float A1, float a1, float b1, float A2, float a2, float b2, float A3, float a3, float b3) {
+    auto two_sum = [](float x, float y, float &err) {
+        const float s = x + y, yy = s - x;
+        err += (x - (s - yy)) + (y - yy);
+        return s;
+    };
+    float err = 0.0f;
+    auto term = [&](float A, float a, float b) {
+        float e = 0.0f;
+        const float d = two_sum(a, -b, e), t = A * d;
+        err += fmaf(A, e, fmaf(A, d, -t));
+        return t;
+    };
+    const float t1 = term(A1, a1, b1), t2 = term(A2, a2, b2), t3 = term(A3, a3, b3);
+    const float s12 = two_sum(t1, t2, err), s = two_sum(s12, t3, err);
+    return s + err;
+}
+__device__ __forceinline__ double cancelling_sum(double, double, double, double, double, double, double, double, double) { return 0.0; }
+
+// SRC: where the source comes from.  kSrcVelocity: ∇·U without an immersed bottom, read without halos
+// (poisson_source_reads_no_halo); kSrcDense: the dense array; kSrcGeneral: ∇·U with every topology
+// and bottom test per element.  Variants of one kernel, since the general source alone is
+// thousands of instructions that the others would carry.
+enum { kSrcGeneral = 0, kSrcVelocity = 1, kSrcDense = 2 };
+template <class T, bool MIXED, int SRC> struct KXFwd {
+    using Family = KXFwd<T, false, kSrcGeneral>;
     static constexpr int kThreads = kFftThreads, kMinBlocks = 1;
     static __device__ __forceinline__ void run(const XFwdArgs<T> &A, const Blk &B);
 };
-template <class T> __device__ __forceinline__ void KXFwd<T>::run(const XFwdArgs<T> &A, const Blk &B) {
+template <class T, bool MIXED, int SRC> __device__ __forceinline__ void KXFwd<T, MIXED, SRC>::run(const XFwdArgs<T> &A, const Blk &B) {
     extern __shared__ unsigned char smem_raw[];
     const Ctx<T> &C = A.C;
     const int Nx = C.g.Nx, Ny = C.g.Ny;
@@ -209,65 +373,69 @@ template <class T> __device__ __forceinline__ void KXFwd<T>::run(const XFwdArgs<
     const int nrows = Ny * C.g.Nz;
     load_table<T>(twl, A.tw, M);
     T *ap = reinterpret_cast<T *>(a);
-    // without an immersed bottom the source is ∇·U of three non-Flat axes on a whole row: each
-    // thread forms its (at most kFastX) elements from loads all issued before any arithmetic,
-    // with no per-element branch (the general path below tests the topology per element).  Its
-    // neighbours across the x and y edges are read by wrapped index, and a Bounded z's boundary
-    // faces of w as the zero the impenetrable fill writes there, so it reads no halo
-    // (poisson_source_reads_no_halo is the same test on the host)
-    constexpr int kFastX = kXFwdFastElems;
-    const bool fast = !A.src && !C.g.kbot && !C.flx() && !C.fly() && !C.flz() && half && !A.scale_dzc &&
-                      Nx <= kFastX * (int)(blockDim.x >> A.L.lgR);
-    if (fast) {
-        const int lgt = __builtin_ctz((unsigned)blockDim.x) - A.L.lgR;   // log2 of threads per row
-        const int tpr = 1 << lgt;
-        const int r = threadIdx.x >> lgt, l = threadIdx.x & (tpr - 1);
-        const int row = row0 + r;
-        const bool live = row < nrows;
-        const int k = live ? (int)fdiv((uint32_t)row, A.fNy) : 0, j = live ? row - k * Ny : 0;
+    // blockDim.x / R threads per row: a thread's row (j, k), its metric factors and addresses are
+    // fixed, and its elements i = l, l + tpr, … differ by constant offsets.  Rows past the last stage
+    // zeros.
+    const int lgt = __builtin_ctz((unsigned)blockDim.x) - A.L.lgR;   // log2 of threads per row
+    const int tpr = 1 << lgt;
+    const int r = threadIdx.x >> lgt, l = threadIdx.x & (tpr - 1);
+    const int row = row0 + r;
+    const bool live = row < nrows;
+    const int k = live ? (int)fdiv((uint32_t)row, A.fNy) : 0, j = live ? row - k * Ny : 0;
+    const T zs = A.scale_dzc && live ? C.g.dzc[k] : T(1);
+    auto put = [&](int i, T x) {
+        if (half) ap[2 * (r * ld + (i >> 1)) + (i & 1)] = x;
+        else a[r * ld + i] = cmk<T>(x, T(0));
+    };
+    if constexpr (SRC == kSrcVelocity) {
+        // each thread forms kXFwdBatch elements at a time from loads all issued before any arithmetic,
+        // with no per-element branch.  Its neighbours across periodic edges are read by wrapped
+        // index, and a Bounded z's boundary faces of w as the zero the impenetrable fill writes
+        // there, so it reads no halo.
         const int jp = (j + 1 == Ny) ? 0 : j + 1;
         const int64_t o = C.at(0, j, k);
         const T *u = C.s.U[0] + o, *v = C.s.U[1] + o, *w = C.s.U[2] + o;
-        const T *vp = C.s.U[1] + C.at(0, jp, k), *wp = w + C.g.sz;
+        const bool flat = C.flz();   // (w's differences are zero then)
+        const int kp = flat || (C.g.tz == OM_PERIODIC && k + 1 == C.g.Nz) ? 0 : k + 1;
+        const T *vp = C.s.U[1] + C.at(0, jp, k), *wp = C.s.U[2] + C.at(0, j, kp);
         const bool wb = C.g.tz == OM_BOUNDED && k == 0, wt = C.g.tz == OM_BOUNDED && k == C.g.Nz - 1;
-        T su[kFastX], sq[kFastX], sv[kFastX], svp[kFastX], sw[kFastX], swp[kFastX];
-#pragma unroll
-        for (int e = 0; e < kFastX; ++e) {
-            const int i = l + e * tpr;
-            const bool in = live && i < Nx;
-            const int ii = in ? i : 0;
-            const int ip = (ii + 1 == Nx) ? 0 : ii + 1;
-            su[e] = in ? u[ii] : T(0);
-            sq[e] = in ? u[ip] : T(0);
-            sv[e] = in ? v[ii] : T(0);
-            svp[e] = in ? vp[ii] : T(0);
-            sw[e] = in && !wb ? w[ii] : T(0);
-            swp[e] = in && !wt ? wp[ii] : T(0);
-        }
         const T Ax = C.Axc(k), Ay = C.Ayc(k), Az = C.g.Az, iV = C.iVc(k);
+        for (int i0 = l; i0 < Nx; i0 += kXFwdBatch * tpr) {
+            T su[kXFwdBatch], sq[kXFwdBatch], sv[kXFwdBatch], svp[kXFwdBatch], sw[kXFwdBatch], swp[kXFwdBatch];
 #pragma unroll
-        for (int e = 0; e < kFastX; ++e) {
-            const int i = l + e * tpr;
-            if (i < Nx) {
-                // Ctx::divU's expression (source_at), in its order of operations
-                const T sx = Ax * sq[e] - Ax * su[e];
-                const T sy = Ay * svp[e] - Ay * sv[e];
-                const T sz = Az * swp[e] - Az * sw[e];
-                ap[2 * (r * ld + (i >> 1)) + (i & 1)] = iV * ((sx + sy) + sz);
+            for (int e = 0; e < kXFwdBatch; ++e) {
+                const int i = i0 + e * tpr;
+                const bool in = live && i < Nx;
+                const int ii = in ? i : 0;
+                const int ip = (ii + 1 == Nx) ? 0 : ii + 1;
+                su[e] = in ? u[ii] : T(0);
+                sq[e] = in ? u[ip] : T(0);
+                sv[e] = in ? v[ii] : T(0);
+                svp[e] = in ? vp[ii] : T(0);
+                sw[e] = in && !wb ? w[ii] : T(0);
+                swp[e] = in && !wt ? wp[ii] : T(0);
+            }
+#pragma unroll
+            for (int e = 0; e < kXFwdBatch; ++e) {
+                const int i = i0 + e * tpr;
+                if (i < Nx) {
+                    T d;
+                    if (sizeof(T) == 4 && A.compensated) {
+                        d = iV * cancelling_sum(Ax, sq[e], su[e], Ay, svp[e], sv[e], Az, swp[e], sw[e]);
+                    } else {
+                        // Ctx::divU's expression (source_at), in its order of operations
+                        const T sx = Ax * sq[e] - Ax * su[e];
+                        const T sy = Ay * svp[e] - Ay * sv[e];
+                        const T sz = flat ? T(0) : Az * swp[e] - Az * sw[e];
+                        d = iV * ((sx + sy) + sz);
+                    }
+                    put(i, A.scale_dzc ? zs * d : d);
+                }
             }
         }
     } else {
-        // blockDim.x / R threads per row: a thread's row (j, k), its metric factors and addresses are
-        // fixed, and its elements i = l, l + tpr, … differ by constant offsets; the loads of four
-        // elements are issued before their LDS stores.  Rows past the last stage zeros.
-        const int lgt = __builtin_ctz((unsigned)blockDim.x) - A.L.lgR;   // log2 of threads per row
-        const int tpr = 1 << lgt;
-        const int r = threadIdx.x >> lgt, l = threadIdx.x & (tpr - 1);
-        const int row = row0 + r;
-        const bool live = row < nrows;
-        const int k = live ? (int)fdiv((uint32_t)row, A.fNy) : 0, j = live ? row - k * Ny : 0;
-        const T zs = A.scale_dzc && live ? C.g.dzc[k] : T(1);
-        constexpr int NB = 4;
+        constexpr int NB = SRC == kSrcDense ? kXFwdBatch : 4;
+        const T *dense = A.src + (int64_t)Nx * (live ? row : 0);
         for (int i0 = l; i0 < Nx; i0 += NB * tpr) {
             T x[NB];
 #pragma unroll
@@ -275,22 +443,19 @@ template <class T> __device__ __forceinline__ void KXFwd<T>::run(const XFwdArgs<
                 const int i = i0 + u * tpr;
                 x[u] = T(0);
                 if (live && i < Nx) {
-                    x[u] = source_at<T>(C, A.src, i, j, k);
+                    x[u] = SRC == kSrcDense ? dense[i] : source_at<T>(C, i, j, k);
                     if (A.scale_dzc) x[u] = zs * x[u];
                 }
             }
 #pragma unroll
             for (int u = 0; u < NB; ++u) {
                 const int i = i0 + u * tpr;
-                if (i < Nx) {
-                    if (half) ap[2 * (r * ld + (i >> 1)) + (i & 1)] = x[u];
-                    else a[r * ld + i] = cmk<T>(x[u], T(0));
-                }
+                if (i < Nx) put(i, x[u]);
             }
         }
     }
     __syncthreads();
-    const C2<T> *Z = lds_fft<T>(a, b, R, M, ld, twl, false);
+    const C2<T> *Z = lds_fft<T, MIXED>(a, b, R, M, ld, twl, false, A.stages);
     for (int t = threadIdx.x; t < R * Mx; t += blockDim.x) {
         const int r = (int)fdiv((uint32_t)t, A.fMx), kk = t - r * Mx;
         const int row = row0 + r;
@@ -312,21 +477,29 @@ template <class T> __device__ __forceinline__ void KXFwd<T>::run(const XFwdArgs<
 template <class T> struct XBwdArgs {
     DevGrid<T> g;
     const C2<T> *S;
-    const C2<T> *tw, *post;
+    const C2<T> *tw;
+    const FftStage *stages;
+    const C2<T> *post;
     T *out;            // field interior view (strided) or dense array
     int dense;
     T scale;           // 1 / (Nx · Ny · Nz-normalisations)
     T divisor;         // the written value is (x · scale) / divisor
+    // even Nx: take X_0 and X_{Nx/2} as real, which they are but for rounding.  Their imaginary parts
+    // hold the forward passes' rounding, amplified at the longest y and z waves by the inverse
+    // Laplacian, and would enter the output as a ±1 wave along x (a u error of 4e-6 of max |u| at
+    // 16 × 16 × 300 in FP32, 5e-7 without).  On with XFwdArgs::compensated.
+    int real_ends;
     LineGeom L;
     FastDiv fNy;
     int Ms;
 };
 
-template <class T> struct KXBwd {
+template <class T, bool MIXED> struct KXBwd {
+    using Family = KXBwd<T, false>;   // one kernel of the step: a batch may hold both variants
     static constexpr int kThreads = kFftThreads, kMinBlocks = 1;
     static __device__ __forceinline__ void run(const XBwdArgs<T> &A, const Blk &B);
 };
-template <class T> __device__ __forceinline__ void KXBwd<T>::run(const XBwdArgs<T> &A, const Blk &B) {
+template <class T, bool MIXED> __device__ __forceinline__ void KXBwd<T, MIXED>::run(const XBwdArgs<T> &A, const Blk &B) {
     extern __shared__ unsigned char smem_raw[];
     const int Nx = A.g.Nx, Ny = A.g.Ny;
     const bool half = (Nx & 1) == 0;
@@ -358,8 +531,9 @@ template <class T> __device__ __forceinline__ void KXBwd<T>::run(const XBwdArgs<
                     if (!half) {
                         Zk = kk < Mx ? Srow[kk] : cconj<T>(Srow[Nx - kk]);
                     } else {
-                        const C2<T> Xk = Srow[kk];
-                        const C2<T> Xc = cconj<T>(Srow[M - kk]);
+                        C2<T> Xk = Srow[kk];
+                        C2<T> Xc = cconj<T>(Srow[M - kk]);
+                        if (kk == 0 && A.real_ends) Xk.y = Xc.y = T(0);
                         const C2<T> E = cmk<T>(T(0.5) * (Xk.x + Xc.x), T(0.5) * (Xk.y + Xc.y));
                         const C2<T> d = csub<T>(Xk, Xc);
                         // O = (Xk - conj(X_{M-k})) · e^{+2πik/N} / 2 ;  Z = E + i O
@@ -377,7 +551,7 @@ template <class T> __device__ __forceinline__ void KXBwd<T>::run(const XBwdArgs<
         }
     }
     __syncthreads();
-    const C2<T> *z = lds_fft<T>(a, b, R, M, ld, twl, true);
+    const C2<T> *z = lds_fft<T, MIXED>(a, b, R, M, ld, twl, true, A.stages);
     if (live) {
         const int k = (int)fdiv((uint32_t)row, A.fNy), j = row - k * Ny;
         T *dst = A.dense ? A.out + (int64_t)Nx * ((int64_t)j + (int64_t)Ny * k) : A.out + idx3(0, j, k, A.g.sy, A.g.sz);
@@ -405,6 +579,7 @@ template <class T> struct YArgs {
     DevGrid<T> g;
     C2<T> *S;
     const C2<T> *tw;
+    const FftStage *stages;
     int Mx, Ms;
     int inverse;
     int fused_divide;
@@ -413,11 +588,12 @@ template <class T> struct YArgs {
     FastDiv fMs;        // division by the row stride Ms
 };
 
-template <class T> struct KYPass {
+template <class T, bool MIXED> struct KYPass {
+    using Family = KYPass<T, false>;   // one kernel of the step: a batch may hold both variants
     static constexpr int kThreads = kFftThreads, kMinBlocks = 1;
     static __device__ __forceinline__ void run(const YArgs<T> &A, const Blk &B);
 };
-template <class T> __device__ __forceinline__ void KYPass<T>::run(const YArgs<T> &A, const Blk &B) {
+template <class T, bool MIXED> __device__ __forceinline__ void KYPass<T, MIXED>::run(const YArgs<T> &A, const Blk &B) {
     extern __shared__ unsigned char smem_raw[];
     const int Ny = A.g.Ny, Mx = A.Mx, R = A.L.R, lgR = A.L.lgR, ld = A.L.ld;
     C2<T> *twl = reinterpret_cast<C2<T> *>(smem_raw);
@@ -436,7 +612,7 @@ template <class T> __device__ __forceinline__ void KYPass<T>::run(const YArgs<T>
         [&](int t) { return valid ? col[(int64_t)(t >> lgR) * Ms] : cmk<T>(T(0), T(0)); },
         [&](int t, C2<T> v) { a[r * ld + (t >> lgR)] = v; });
     __syncthreads();
-    C2<T> *res = lds_fft<T>(a, b, R, Ny, ld, twl, A.inverse != 0);
+    C2<T> *res = lds_fft<T, MIXED>(a, b, R, Ny, ld, twl, A.inverse != 0, A.stages);
     if (A.fused_divide) {
         C2<T> *other = (res == a) ? b : a;
         for (int t = threadIdx.x; t < R * Ny; t += blockDim.x) {
@@ -444,7 +620,7 @@ template <class T> __device__ __forceinline__ void KYPass<T>::run(const YArgs<T>
             if (valid) res[r * ld + j] = eig_divide<T>(res[r * ld + j], A.lx[kx] + A.ly[j], kx == 0 && j == 0);
         }
         __syncthreads();
-        res = lds_fft<T>(res, other, R, Ny, ld, twl, true);
+        res = lds_fft<T, MIXED>(res, other, R, Ny, ld, twl, true, A.stages);
     }
     if (!valid) return;
     for (int t = threadIdx.x; t < R * Ny; t += blockDim.x) {
@@ -459,31 +635,33 @@ template <class T> __device__ __forceinline__ void KYPass<T>::run(const YArgs<T>
 // S[k·Ny·Ms + ℓ], so a block reads R contiguous values per level; lines with kx ≥ Mx are row
 // padding and are skipped.
 //   zmode 0 (Periodic z): FFT of length Nz.
-//   zmode 1 (Bounded z, Nz even): the DCT-II of length N = Nz through one complex FFT of length N
-//     (Makhoul 1980): v = (x0, x2, …, x_{N−2}, x_{N−1}, …, x3, x1), V = FFT(v),
+//   zmode 1 (Bounded z): the DCT-II of length N = Nz through one complex FFT of length N
+//     (Makhoul 1980): v = (x0, x2, x4, …, x5, x3, x1), V = FFT(v),
 //     X_k = c_k V_k + c̄_k V_{N−k} with c_k = e^{−iπk/2N}; after the division the inverse is
 //     V'_k = c̄_k (Φ_k − i Φ_{N−k}) (Φ_N = 0), v' = IFFT(V'), x read back through the same
 //     permutation.  Each thread handles the pair (k, N−k).  The result equals the inverse
-//     transform of the 2N-point even extension, so it shares that normalisation (1 / 2N).
-//   zmode 2 (Bounded z, Nz odd): FFT of the 2N-point even extension, mirrored in LDS.
+//     transform of the 2N-point even extension, so it shares that normalisation (1 / 2N).  For odd
+//     N every k > 0 has a partner other than itself.
 // ---------------------------------------------------------------------------------------------
 template <class T> struct ZArgs {
     DevGrid<T> g;
     C2<T> *S;
-    const C2<T> *tw;         // table for the FFT length L
+    const C2<T> *tw;         // table for the FFT length Nz
+    const FftStage *stages;
     const C2<T> *dct;        // c_k, k < Nz (zmode 1)
-    int Mx, Ms, L, zmode;    // L = Nz (zmodes 0, 1) or 2Nz (zmode 2); Ms: row stride of S
+    int Mx, Ms, zmode;       // Ms: row stride of S
     const T *lx, *ly, *lz;   // lz: Nz entries (Periodic), 2Nz (Bounded, symmetric)
     LineGeom G;
 };
 
-template <class T> struct KZPass {
+template <class T, bool MIXED> struct KZPass {
+    using Family = KZPass<T, false>;   // one kernel of the step: a batch may hold both variants
     static constexpr int kThreads = kFftThreads, kMinBlocks = 1;
     static __device__ __forceinline__ void run(const ZArgs<T> &A, const Blk &B);
 };
-template <class T> __device__ __forceinline__ void KZPass<T>::run(const ZArgs<T> &A, const Blk &B) {
+template <class T, bool MIXED> __device__ __forceinline__ void KZPass<T, MIXED>::run(const ZArgs<T> &A, const Blk &B) {
     extern __shared__ unsigned char smem_raw[];
-    const int Ny = A.g.Ny, Nz = A.g.Nz, Mx = A.Mx, L = A.L, zmode = A.zmode;
+    const int Ny = A.g.Ny, Nz = A.g.Nz, L = Nz, Mx = A.Mx, zmode = A.zmode;
     const int R = A.G.R, lgR = A.G.lgR, ld = A.G.ld;
     C2<T> *twl = reinterpret_cast<C2<T> *>(smem_raw);
     C2<T> *dctl = twl + L;
@@ -503,14 +681,10 @@ template <class T> __device__ __forceinline__ void KZPass<T>::run(const ZArgs<T>
         [&](int t) { return valid ? col[(int64_t)(t >> lgR) * plane] : cmk<T>(T(0), T(0)); },
         [&](int t, C2<T> v) {
             const int k = t >> lgR;
-            if (zmode == 1) a[r * ld + ((k & 1) ? Nz - ((k + 1) >> 1) : (k >> 1))] = v;
-            else {
-                a[r * ld + k] = v;
-                if (zmode == 2) a[r * ld + (L - 1 - k)] = v;
-            }
+            a[r * ld + (zmode == 1 ? ((k & 1) ? Nz - ((k + 1) >> 1) : (k >> 1)) : k)] = v;
         });
     __syncthreads();
-    C2<T> *res = lds_fft<T>(a, b, R, L, ld, twl, false);
+    C2<T> *res = lds_fft<T, MIXED>(a, b, R, L, ld, twl, false, A.stages);
     C2<T> *other = (res == a) ? b : a;
     const T lxy = valid ? A.lx[kx] + A.ly[j] : T(1);
     const bool zero_col = kx == 0 && j == 0;
@@ -536,7 +710,7 @@ template <class T> __device__ __forceinline__ void KZPass<T>::run(const ZArgs<T>
         }
     }
     __syncthreads();
-    res = lds_fft<T>(res, other, R, L, ld, twl, true);
+    res = lds_fft<T, MIXED>(res, other, R, L, ld, twl, true, A.stages);
     if (!valid) return;
     for (int t = threadIdx.x; t < R * Nz; t += blockDim.x) {
         const int k = t >> lgR;
@@ -748,18 +922,28 @@ template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C,
     const int Mx = Nx / 2 + 1;
     const int nrows = Ny * Nz;
     size_t lds = 0;
+    auto p2 = [](int n) { return (n & (n - 1)) == 0; };
+    const int compensated = !(p2(M) && p2(Ny) && (P.tridiagonal || p2(Nz)));
+    // one of a kernel's two variants by its line length
+    auto by_length = [&](auto plain, auto mixed, int n, int blocks, size_t shared, const auto &A) {
+        if (p2(n)) launch_k<decltype(plain)>(dim3(blocks), dim3(kFftThreads), shared, st, A);
+        else launch_k<decltype(mixed)>(dim3(blocks), dim3(kFftThreads), shared, st, A);
+    };
     {
         const LineGeom L = line_geom(M, M, e, lds);
-        XFwdArgs<T> A{C, src, P.S, P.tw_xh, P.post, P.tridiagonal, L, make_fastdiv((uint32_t)Ny), make_fastdiv((uint32_t)Mx), P.Ms};
-        launch_k<KXFwd<T>>(dim3((nrows + L.R - 1) / L.R), dim3(kFftThreads), lds, st, A);
+        XFwdArgs<T> A{C, src, P.S, P.tw_xh, P.st_x, P.post, P.tridiagonal, compensated, L, make_fastdiv((uint32_t)Ny), make_fastdiv((uint32_t)Mx), P.Ms};
+        const int blocks = (nrows + L.R - 1) / L.R;
+        if (src) by_length(KXFwd<T, false, kSrcDense>(), KXFwd<T, true, kSrcDense>(), M, blocks, lds, A);
+        else if (poisson_source_reads_no_halo(C)) by_length(KXFwd<T, false, kSrcVelocity>(), KXFwd<T, true, kSrcVelocity>(), M, blocks, lds, A);
+        else by_length(KXFwd<T, false, kSrcGeneral>(), KXFwd<T, true, kSrcGeneral>(), M, blocks, lds, A);
     }
     const bool z_active = g.tz != OM_FLAT;
     const LineGeom Ly = line_geom(Ny, Ny, e, lds);
     const size_t lds_y = lds;
     const int ygrid = (P.Ms * Nz + Ly.R - 1) / Ly.R;
     {
-        YArgs<T> A{g, P.S, P.tw_y, Mx, P.Ms, 0, z_active ? 0 : 1, P.lx, P.ly, Ly, make_fastdiv((uint32_t)P.Ms)};
-        launch_k<KYPass<T>>(dim3(ygrid), dim3(kFftThreads), lds_y, st, A);
+        YArgs<T> A{g, P.S, P.tw_y, P.st_y, Mx, P.Ms, 0, z_active ? 0 : 1, P.lx, P.ly, Ly, make_fastdiv((uint32_t)P.Ms)};
+        by_length(KYPass<T, false>(), KYPass<T, true>(), Ny, ygrid, lds_y, A);
     }
     T scale = T(1) / (T(M) * T(Ny));
     if (z_active) {
@@ -775,31 +959,22 @@ template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C,
             hipLaunchKernelGGL(k_tridiag<T>, dim3((unsigned)((ncol + bw - 1) / bw)), dim3(bw), (size_t)Nz * bw * sizeof(T), st, A,
                                P.S, g.dzc, g.idzf);
         } else {
-            const LineGeom Lz = line_geom(P.Lz_line, P.Lz_line + (P.zmode == 1 ? Nz : 0), e, lds);
-            ZArgs<T> A{g, P.S, P.tw_z, P.tw_dct, Mx, P.Ms, P.Lz_line, P.zmode, P.lx, P.ly, P.lz, Lz};
-            launch_k<KZPass<T>>(dim3((P.Ms * Ny + Lz.R - 1) / Lz.R), dim3(kFftThreads), lds, st, A);
+            const LineGeom Lz = line_geom(Nz, Nz + (P.zmode == 1 ? Nz : 0), e, lds);
+            ZArgs<T> A{g, P.S, P.tw_z, P.st_z, P.tw_dct, Mx, P.Ms, P.zmode, P.lx, P.ly, P.lz, Lz};
+            by_length(KZPass<T, false>(), KZPass<T, true>(), Nz, (P.Ms * Ny + Lz.R - 1) / Lz.R, lds, A);
             scale = T(1) / ((T(M) * T(Ny)) * T(P.Lz_norm));
         }
-        YArgs<T> A{g, P.S, P.tw_y, Mx, P.Ms, 1, 0, P.lx, P.ly, Ly, make_fastdiv((uint32_t)P.Ms)};
-        launch_k<KYPass<T>>(dim3(ygrid), dim3(kFftThreads), lds_y, st, A);
+        YArgs<T> A{g, P.S, P.tw_y, P.st_y, Mx, P.Ms, 1, 0, P.lx, P.ly, Ly, make_fastdiv((uint32_t)P.Ms)};
+        by_length(KYPass<T, false>(), KYPass<T, true>(), Ny, ygrid, lds_y, A);
     }
     {
         const LineGeom L = line_geom(M, M, e, lds);
-        XBwdArgs<T> A{g, P.S, P.tw_xh, P.post, out, dense_out, scale, divisor, L, make_fastdiv((uint32_t)Ny), P.Ms};
-        launch_k<KXBwd<T>>(dim3((nrows + L.R - 1) / L.R), dim3(kFftThreads), lds, st, A);
+        XBwdArgs<T> A{g, P.S, P.tw_xh, P.st_x, P.post, out, dense_out, scale, divisor, compensated, L, make_fastdiv((uint32_t)Ny), P.Ms};
+        by_length(KXBwd<T, false>(), KXBwd<T, true>(), M, (nrows + L.R - 1) / L.R, lds, A);
     }
 }
 
-template <class T> bool poisson_source_reads_no_halo(const PoissonPlan<T> &P, const Ctx<T> &C) {
-    const DevGrid<T> &g = C.g;
-    if (g.kbot || g.tx == OM_FLAT || g.ty == OM_FLAT || g.tz == OM_FLAT || (g.Nx & 1) || P.tridiagonal) return false;
-    const int M = g.Nx / 2;
-    const int R = fft_lines_per_block(M, M, sizeof(C2<T>));
-    return R >= 1 && g.Nx <= kXFwdFastElems * (kFftThreads / R);
-}
-
 #ifndef OM_ONLY_DOUBLE
-template bool poisson_source_reads_no_halo<float>(const PoissonPlan<float> &, const Ctx<float> &);
 template void launch_poisson_residual<float>(const Ctx<float> &, const RefineOp &, const float *, int64_t, int64_t,
                                              const double *, double, float *, hipStream_t);
 template void launch_add_correction<float>(const DevGrid<float> &, float *, int64_t, int64_t, const float *, hipStream_t);
@@ -807,7 +982,6 @@ template void launch_poisson<float>(const PoissonPlan<float> &, const Ctx<float>
                                     hipStream_t);
 #endif
 #ifndef OM_ONLY_FLOAT
-template bool poisson_source_reads_no_halo<double>(const PoissonPlan<double> &, const Ctx<double> &);
 template void launch_poisson_residual<double>(const Ctx<double> &, const RefineOp &, const double *, int64_t, int64_t,
                                               const double *, double, double *, hipStream_t);
 template void launch_add_correction<double>(const DevGrid<double> &, double *, int64_t, int64_t, const double *, hipStream_t);

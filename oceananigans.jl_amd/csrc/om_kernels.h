@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <vector>
 
 #include "om_internal.h"
 
@@ -647,6 +648,37 @@ template <class T> struct RKArgs {
     int nfields;
 };
 
+// One stage of a mixed-radix line transform of length n (not a power of two): its radix, the
+// product m of the radices before it, and ⌈2³²/m⌉, ⌈2³²/(n/radix)⌉.  The high word of t·⌈2³²/d⌉ is
+// ⌊t/d⌋ whenever t·(d − 1) < 2³²; here t < 4096 and d ≤ 4096 (R·n ≤ 4096 elements per block);
+// the stages treat d = 1 apart.
+struct FftStage {
+    uint32_t radix, m, mul_m, mul_b;
+};
+// the stages of a line of length n, ended by radix 0.  The odd radices come first: their stages then
+// run at odd sub-lengths, whose output strides spread over the LDS banks.
+inline std::vector<FftStage> fft_stages(int n) {
+    std::vector<FftStage> st;
+    uint32_t m = 1;
+    auto mul = [](uint32_t d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
+    auto add = [&](uint32_t r) {
+        st.push_back(FftStage{r, m, mul(m), mul((uint32_t)n / r)});
+        m *= r;
+    };
+    int rest = n;
+    for (int r : {7, 5, 3}) for (; rest % r == 0; rest /= r) add((uint32_t)r);
+    int twos = 0;
+    for (; rest % 2 == 0; rest /= 2) ++twos;
+    for (int r = 11; rest > 1; r += 2) {
+        if (r * r > rest) r = rest;
+        for (; rest % r == 0; rest /= r) add((uint32_t)r);
+    }
+    for (; twos >= 2; twos -= 2) add(4);
+    if (twos) add(2);
+    st.push_back(FftStage{0, 0, 0, 0});
+    return st;
+}
+
 // Poisson solver plan: spectral storage and per-axis tables (device pointers).
 template <class T> struct PoissonPlan {
     typename Vec2<T>::type *S;          // complex spectral array, Ms · Ny · Nz (x rows padded to Ms)
@@ -654,11 +686,11 @@ template <class T> struct PoissonPlan {
     const typename Vec2<T>::type *tw_xh; // twiddles for the x line (length Nx/2 when Nx is even, Nx otherwise)
     const typename Vec2<T>::type *post;  // exp(-2πi k / Nx), k = 0 .. Nx/2
     const typename Vec2<T>::type *tw_y;  // length Ny
-    const typename Vec2<T>::type *tw_z;  // length Lz_line
+    const typename Vec2<T>::type *tw_z;  // length Nz
+    const FftStage *st_x, *st_y, *st_z;  // stages of the x, y and z lines (lengths as the tables')
     const typename Vec2<T>::type *tw_dct; // exp(-iπk / 2Nz), k < Nz (zmode 1)
     const T *lx, *ly, *lz;               // eigenvalues (lz: Nz entries, 2·Nz for Bounded z)
-    int zmode;                           // 0 Periodic z, 1 Bounded z via a length-Nz DCT, 2 Bounded z, odd Nz, 2Nz extension
-    int Lz_line;                         // FFT length along z: Nz (zmodes 0, 1), 2·Nz (zmode 2)
+    int zmode;                           // 0 Periodic z, 1 Bounded z via a length-Nz DCT
     int Lz_norm;                         // normalisation of the z transform pair: Nz (Periodic), 2·Nz (Bounded)
     int tridiagonal;                     // Fourier–tridiagonal z solve (stretched z)
     T eps10;                             // 10·eps(FT): the Thomas pivot guard
@@ -666,7 +698,7 @@ template <class T> struct PoissonPlan {
 
 // Lines of the FFT passes staged per block: the largest power of two R ≤ 16 with R·n ≤ 4096 whose
 // R rows (stride n + 1 when R > 1) and `tables` complex table entries fit in 64 KiB of LDS, with a
-// second buffer when n is not a power of two (direct DFT).  0: not even one line fits.
+// second buffer when n is not a power of two (mixed radix).  0: not even one line fits.
 inline int fft_lines_per_block(int n, int tables, size_t elem) {
     const bool p2 = (n & (n - 1)) == 0;
     for (int R = 16; R >= 1; R >>= 1) {
@@ -775,10 +807,10 @@ template <class T> void launch_divergence(const Ctx<T> &C, T *out, hipStream_t s
 template <class T> void launch_halos(const DevGrid<T> &g, const HaloJob<T> &J, hipStream_t st);
 // Solve ∇²ϕ = source; writes ϕ / divisor into `out` (the nonhydrostatic pressure p/Δt when
 // called from the pressure correction, divisor = 1 otherwise).
-// elements per thread of the X-forward pass's halo-free source path
-constexpr int kXFwdFastElems = 8;
-// whether the X-forward pass forms ∇·U of the state without reading a halo (its fast path)
-template <class T> bool poisson_source_reads_no_halo(const PoissonPlan<T> &P, const Ctx<T> &C);
+// whether the X-forward pass forms ∇·U of the state without reading a halo
+template <class T> bool poisson_source_reads_no_halo(const Ctx<T> &C) {
+    return !C.g.kbot && C.g.tx != OM_FLAT && C.g.ty != OM_FLAT;
+}
 template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C, const T *src, T *out, int dense_out,
                                        T divisor, hipStream_t st);
 
