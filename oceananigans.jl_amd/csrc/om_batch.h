@@ -32,8 +32,30 @@ template <class A> struct BatchEntry {
     uint32_t gx, gy, gz, begin;
 };
 
+// The arguments of a kind that declares kArgsInMemory are read where the launch put them (the
+// kernel-argument segment, or the batch's table), in the constant address space, so that the kind may
+// read them again (ConstArgs) instead of holding them all in scalar registers.
+#define OM_CONSTANT __attribute__((address_space(4)))
+template <class K, class = void> struct ArgsInMemory { static constexpr bool value = false; };
+template <class K> struct ArgsInMemory<K, std::enable_if_t<K::kArgsInMemory>> { static constexpr bool value = true; };
+
+template <class A> struct ConstArgs {
+    const OM_CONSTANT A *p;
+    __device__ __forceinline__ explicit ConstArgs(const A &a) : p((const OM_CONSTANT A *)&a) {}
+    // the arguments, read anew from here on: what was loaded before need not stay in registers
+    __device__ __forceinline__ const A &again() const {
+        const OM_CONSTANT A *q = p;
+        asm volatile("" : "+s"(q));
+        return *(const A *)q;
+    }
+};
+
 template <class K, class A> __global__ void __launch_bounds__(K::kThreads, K::kMinBlocks) k_one(A a) {
-    K::run(a, Blk{blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, gridDim.z});
+    const Blk B{blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, gridDim.z};
+    if constexpr (ArgsInMemory<K>::value)   // (the only argument: the segment starts with it)
+        K::run(*(const A *)(const OM_CONSTANT A *)__builtin_amdgcn_kernarg_segment_ptr(), B);
+    else
+        K::run(a, B);
 }
 
 template <class K, class A>
@@ -45,7 +67,7 @@ __global__ void __launch_bounds__(K::kThreads, K::kMinBlocks) k_many(const Batch
         if (tab[mid].begin <= id) lo = mid;
         else hi = mid - 1;
     }
-    const BatchEntry<A> &E = tab[lo];
+    const BatchEntry<A> &E = tab[__builtin_amdgcn_readfirstlane(lo)];
     const uint32_t local = id - E.begin;
     if (local >= E.gx * E.gy * E.gz) return;
     const uint32_t x = local % E.gx, r = local / E.gx;

@@ -8,6 +8,11 @@
 // of from L1/L2.  Each thread keeps its column's tracers at k-1 .. k+1 in registers for the
 // vertical gradients.  The expressions and their operand order are those of k_closure
 // (om_kernels.hip), so the two kernels give identically rounded results.
+//
+// VALU issue and latency bound it.  The two closures are separate kernels, the staging offsets are
+// formed once per block and the arguments read again from constant memory at each level: 127 → 93
+// VGPRs for AMD with one tracer (5 waves per SIMD instead of 4), 76 for Smagorinsky–Lilly with two,
+// which took 143 as one kernel (512 × 512 × 256: 876 → 712 µs; AMD 256 × 256 × 128: 112.5 → 111 µs).
 #include <hip/hip_runtime.h>
 
 #include "om_batch.h"
@@ -39,18 +44,21 @@ template <class T> struct ClosureTiledArgs {
     int kchunk, ntx;
 };
 
-template <class T, int NT> struct KClosureTiled {
+template <class T, int NT, bool SMAG> struct KClosureTiled {
+    using Family = KClosureTiled<T, NT, false>;
     static constexpr int kThreads = 256, kMinBlocks = 1;
+    static constexpr bool kArgsInMemory = true;
     static __device__ __forceinline__ void run(const ClosureTiledArgs<T> &A, const Blk &B);
 };
 
-template <class T, int NT>
-__device__ __forceinline__ void KClosureTiled<T, NT>::run(const ClosureTiledArgs<T> &A, const Blk &B) {
+template <class T, int NT, bool SMAG>
+__device__ __forceinline__ void KClosureTiled<T, NT, SMAG>::run(const ClosureTiledArgs<T> &A0, const Blk &B) {
     __shared__ ClosureSmem<T, NT> S;
+    const ConstArgs<ClosureTiledArgs<T>> args(A0);
+    const ClosureTiledArgs<T> &A = args.again();
     const Ctx<T> &C = A.C;
     const int kchunk = A.kchunk, ntx = A.ntx;
     const DevGrid<T> &g = C.g;
-    const DevPhysics<T> &ph = C.ph;
     const int tid = threadIdx.x;
     const int a = tid & (CT - 1), b = tid >> 4;
     // work item → (z chunk, tile): the chunks of one tile are consecutive, tiles in row order
@@ -62,10 +70,9 @@ __device__ __forceinline__ void KClosureTiled<T, NT>::run(const ClosureTiledArgs
     const int k0 = chunk * kchunk;
     const int k1 = min(k0 + kchunk, g.Nz);
     const int i = i0 + a, j = j0 + b;
-    const bool colok = i <= g.Nx + g.Hx - 1 && j <= g.Ny + g.Hy - 1;
     const bool cell = i < g.Nx && j < g.Ny;
-    const int64_t col = idx3(i, j, 0, g.sy, g.sz);
-    const bool smag = ph.closure == OM_CLOSURE_SMAGORINSKY_LILLY;
+    // (held inside the field: threads past its last halo point read a column nobody uses)
+    const int64_t col = idx3(min(i, g.Nx + g.Hx - 1), min(j, g.Ny + g.Hy - 1), 0, g.sy, g.sz);
 
     auto P = [&](const T *p, int dx, int dy) -> T { return p[(b + 1 + dy) * CW + (a + 1 + dx)]; };
     auto slot3 = [](int level) { return ((level % 3) + 3) % 3; };
@@ -75,7 +82,7 @@ __device__ __forceinline__ void KClosureTiled<T, NT>::run(const ClosureTiledArgs
     const uint32_t colb0 = (uint32_t)(col * (int64_t)sizeof(T));
     uint32_t colb = colb0;
     auto ldcol = [&](const T *f, int k) -> T {
-        return colok ? *reinterpret_cast<const T *>(reinterpret_cast<const char *>(f + (int64_t)k * g.sz) + colb) : T(0);
+        return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(f + (int64_t)k * g.sz) + colb);
     };
 
     // own-column tracers at levels kk-1, kk, kk+1 ([0], [1], [2])
@@ -90,32 +97,29 @@ __device__ __forceinline__ void KClosureTiled<T, NT>::run(const ClosureTiledArgs
 
     const T half = T(0.5);
     // The planes a level adds (u, v, w at k + 1, the tracers at k) are loaded into registers while
-    // the previous level is evaluated, so their memory latency is hidden behind that work; the
-    // plane shares are rebuilt for each load from an opaque copy of tid.
+    // the previous level is evaluated, so their memory latency is hidden behind that work.
+    const PlaneShare<T, CW> ps(g, i0, j0, 1, tid);
     T ru[2], rv[2], rw[2], rc[NT > 0 ? NT : 1][2];
-    auto load_level = [&](int k) {
-        int otid = tid;
-        asm volatile("" : "+v"(otid));
-        const PlaneShare<T, CW> ps(g, i0, j0, 1, otid);
-        ps.load(ru, ps.origin(C.s.U[0], g, i0, j0, 1, k + 1));
-        ps.load(rv, ps.origin(C.s.U[1], g, i0, j0, 1, k + 1));
-        ps.load(rw, ps.origin(C.s.U[2], g, i0, j0, 1, k + 1));
+    auto load_level = [&](const Ctx<T> &C, int k) {
+        const DevGrid<T> &g = C.g;
+        const uint32_t o0 = ps.off0, o1 = ps.off1();
+        ps.load(ru, ps.origin(C.s.U[0], g, i0, j0, 1, k + 1), o0, o1);
+        ps.load(rv, ps.origin(C.s.U[1], g, i0, j0, 1, k + 1), o0, o1);
+        ps.load(rw, ps.origin(C.s.U[2], g, i0, j0, 1, k + 1), o0, o1);
 #pragma unroll
-        for (int n = 0; n < NT; ++n) ps.load(rc[n], ps.origin(C.s.U[3 + n], g, i0, j0, 1, k));
+        for (int n = 0; n < NT; ++n) ps.load(rc[n], ps.origin(C.s.U[3 + n], g, i0, j0, 1, k), o0, o1);
     };
-    load_level(k0);
+    load_level(C, k0);
     // AMD: the x-z and y-z gradients at level k + 1 of one level are those at level k of the next
     // (same expressions on the same planes and ratios), so they are carried instead of recomputed
     T c_xw[2], c_zu[2], c_ywx[2], c_yw[2], c_zv[2];
     bool carried = false;
     for (int k = k0; k < k1; ++k) {
-        int otid = tid;
-        asm volatile("" : "+v"(otid));
         colb = colb0;
         asm volatile("" : "+v"(colb));
-        const PlaneShare<T, CW> ps(g, i0, j0, 1, otid);
+        const Ctx<T> &Cw = args.again().C;
 #pragma unroll
-        for (int n = 0; n < NT; ++n) { cw[n][0] = cw[n][1]; cw[n][1] = cw[n][2]; cw[n][2] = ldcol(C.s.U[3 + n], k + 1); }
+        for (int n = 0; n < NT; ++n) { cw[n][0] = cw[n][1]; cw[n][1] = cw[n][2]; cw[n][2] = ldcol(Cw.s.U[3 + n], k + 1); }
         __syncthreads();   // previous level's readers are done
         ps.store(S.u[slot3(k + 1)], ru, tid);
         ps.store(S.v[slot3(k + 1)], rv, tid);
@@ -123,8 +127,11 @@ __device__ __forceinline__ void KClosureTiled<T, NT>::run(const ClosureTiledArgs
 #pragma unroll
         for (int n = 0; n < NT; ++n) ps.store(S.c[n], rc[n], tid);
         __syncthreads();
-        if (k + 1 < k1) load_level(k + 1);
+        if (k + 1 < k1) load_level(args.again().C, k + 1);
         if (!cell) continue;
+        const Ctx<T> &C = args.again().C;
+        const DevGrid<T> &g = C.g;
+        const DevPhysics<T> &ph = C.ph;
 
         const T *Um = S.u[slot3(k - 1)], *U0 = S.u[slot3(k)], *Up = S.u[slot3(k + 1)];
         const T *Vm = S.v[slot3(k - 1)], *V0 = S.v[slot3(k)], *Vp = S.v[slot3(k + 1)];
@@ -142,7 +149,7 @@ __device__ __forceinline__ void KClosureTiled<T, NT>::run(const ClosureTiledArgs
         auto dz_v = [&](const T *Vl, const T *Vlm, int dj, int kk) { return (P(Vl, 0, dj) - P(Vlm, 0, dj)) * g.idzf[kk]; };
         auto at = [&](T *f) -> T & { return *reinterpret_cast<T *>(reinterpret_cast<char *>(f + (int64_t)k * g.sz) + colb); };
 
-        if (smag) {
+        if constexpr (SMAG) {
             auto S12 = [&](int di, int dj) { return half * (dy_u(di, dj) + dx_v(di, dj)); };
             T s12[4] = {S12(0, 0), S12(1, 0), S12(0, 1), S12(1, 1)};
             T s13[4] = {half * (dz_u(U0, Um, 0, k) + dx_w(W0, 0)), half * (dz_u(U0, Um, 1, k) + dx_w(W0, 1)),
@@ -180,9 +187,7 @@ __device__ __forceinline__ void KClosureTiled<T, NT>::run(const ClosureTiledArgs
             T s2 = T(1) - fmin(T(1), cb * N2p / S2);
             T sig = (S2 == T(0)) ? T(0) : sqrt(s2);
             at(C.s.nu) = (sig * (c0 * c0)) * (Df * Df) * sqrt(T(2) * S2);
-            continue;
-        }
-
+        } else {
         // ---- AMD (the level ratios come from the grid's table: same values, no per-thread division)
         const T Dfx = T(2) * g.dx, Dfy = T(2) * g.dy;
         const T Dfz0 = T(2) * g.dzc[k], Dfz1 = T(2) * g.dzc[k + 1];
@@ -275,6 +280,7 @@ __device__ __forceinline__ void KClosureTiled<T, NT>::run(const ClosureTiledArgs
             at(C.s.kap[n]) = fmax(T(0), kap);
         }
 #undef A4
+        }
     }
 }
 
@@ -292,10 +298,15 @@ template <class T> void launch_closure_tiled(const Ctx<T> &C, int kchunk, hipStr
     const int nch = (g.Nz + kchunk - 1) / kchunk;
     const dim3 grid(ntx * nty * nch), blk(CT * CT);
     const ClosureTiledArgs<T> A{C, kchunk, ntx};
+    auto by_closure = [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        if (C.ph.closure == OM_CLOSURE_SMAGORINSKY_LILLY) launch_k<KClosureTiled<T, NT, true>>(grid, blk, 0, st, A);
+        else launch_k<KClosureTiled<T, NT, false>>(grid, blk, 0, st, A);
+    };
     switch (C.ph.n_tracers) {
-        case 0: launch_k<KClosureTiled<T, 0>>(grid, blk, 0, st, A); break;
-        case 1: launch_k<KClosureTiled<T, 1>>(grid, blk, 0, st, A); break;
-        default: launch_k<KClosureTiled<T, 2>>(grid, blk, 0, st, A); break;
+        case 0: by_closure(std::integral_constant<int, 0>()); break;
+        case 1: by_closure(std::integral_constant<int, 1>()); break;
+        default: by_closure(std::integral_constant<int, 2>());
     }
 }
 

@@ -205,38 +205,37 @@ __device__ __forceinline__ int xcd_work_item(int id, int nb) {
 }
 
 // A thread's share of a W × W plane staged into LDS by a 256-thread block: plane elements tid and
-// tid + 256 (row-major, origin (i0 − h, j0 − h)).  Their byte offsets from the plane origin and
-// their validity are computed once per block, so staging a level costs one scalar origin per
-// field and a load per element, and every load of a level can be issued before the first LDS
-// store.  Elements beyond the field's last halo point in x or y are staged as 0.
+// tid + 256 (row-major, origin (i0 − h, j0 − h)).  The byte offset of the first from the plane origin
+// is computed once per block and the second's follows from it (256 elements further on: a fixed
+// number of rows and columns, and one row more where the column wraps), so staging a level costs one
+// scalar origin per field and a load per element, and every load of a level can be issued before the
+// first LDS store.  Offsets are held inside the level's plane, so no load is predicated: what the
+// elements beyond the field's last halo point (or past the W × W elements) read is never used.
 template <class T, int W> struct PlaneShare {
-    uint32_t off[2];
-    bool in1;       // element tid + 256 lies inside the plane (element tid always does: W² ≥ 256)
-    bool ok[2];     // inside the plane and the field
+    uint32_t off0, step, wrapstep, most;   // (the last three are the same for the whole block)
+    bool wraps;
     __device__ __forceinline__ PlaneShare(const DevGrid<T> &g, int i0, int j0, int h, int tid) {
         static_assert(W * W >= 256 && W * W <= 512, "two elements per thread");
-        const int imax = g.Nx + g.Hx - 1, jmax = g.Ny + g.Hy - 1;
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = tid + 256 * u;
-            const int y = e / W, x = e - y * W;
-            const bool in = e < W * W;
-            ok[u] = in && i0 - h + x <= imax && j0 - h + y <= jmax;
-            off[u] = (uint32_t)(((int64_t)y * g.sy + x) * (int64_t)sizeof(T));
-            if (u == 1) in1 = in;
-        }
+        constexpr uint32_t e = sizeof(T);
+        const int y = tid / W, x = tid - y * W;
+        most = (uint32_t)(g.sz - 1 - ((int64_t)(j0 - h + g.Hy) * g.sy + (i0 - h + g.Hx))) * e;
+        step = ((uint32_t)(256 / W) * (uint32_t)g.sy + 256 % W) * e;
+        wrapstep = step + ((uint32_t)g.sy - W) * e;
+        off0 = min(((uint32_t)y * (uint32_t)g.sy + x) * e, most);
+        wraps = x + 256 % W >= W;
     }
     // plane origin of field f at level k (uniform across the block)
     __device__ __forceinline__ static const char *origin(const T *f, const DevGrid<T> &g, int i0, int j0, int h, int k) {
         return reinterpret_cast<const char *>(f + idx3(i0 - h, j0 - h, k, g.sy, g.sz));
     }
-    __device__ __forceinline__ void load(T (&v)[2], const char *base) const {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) v[u] = ok[u] ? *reinterpret_cast<const T *>(base + off[u]) : T(0);
+    __device__ __forceinline__ uint32_t off1() const { return min(off0 + (wraps ? wrapstep : step), most); }
+    __device__ __forceinline__ static void load(T (&v)[2], const char *base, uint32_t o0, uint32_t o1) {
+        v[0] = *reinterpret_cast<const T *>(base + o0);
+        if (threadIdx.x < W * W - 256) v[1] = *reinterpret_cast<const T *>(base + o1);
     }
-    __device__ __forceinline__ void store(T *dst, const T (&v)[2], int tid) const {
+    __device__ __forceinline__ static void store(T *dst, const T (&v)[2], int tid) {
         dst[tid] = v[0];
-        if (in1) dst[tid + 256] = v[1];
+        if (tid < W * W - 256) dst[tid + 256] = v[1];
     }
 };
 
