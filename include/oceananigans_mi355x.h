@@ -290,7 +290,7 @@ int om_last_step_timing(const om_model_t *m, double *ms_total, double *ms_per_ph
  * them: every tendency kernel gives identically rounded tendencies. */
 #define OM_TUNE_TENDENCY_KERNEL 0   /* 0: z-marching LDS-tiled tendency and closure kernels where supported
                                        (default); 1: thread-per-cell kernels */
-#define OM_TUNE_KCHUNK          1   /* z levels marched by one block of the tiled kernels (default 16;
+#define OM_TUNE_KCHUNK          1   /* z levels marched by one block of the tiled kernels (default: by the grid's size;
                                        om_autotune may choose different ones for the two kernels) */
 #define OM_TUNE_LEARNED_ITERATIONS 2 /* leading iterations of each CG solve that apply the learned
                                         correction (0: all); later iterations use the FFT

@@ -211,8 +211,10 @@ template <class T> struct ModelT : ModelBase {
     std::vector<double> snap_isz;
     // launch-shape choices (om_set_tuning)
     int tune_tendency_kernel = 0;      // 0: tiled z-marching kernel where supported, 1: thread per cell
-    int tune_kchunk = 16;              // z levels per block of the tiled tendency kernel
-    int tune_kchunk_closure = 16;      // z levels per block of the tiled closure kernel
+    int tune_kchunk = 0;               // z levels per block of the tiled tendency kernel (set by choose_chunks)
+    int tune_kchunk_closure = 0;       // z levels per block of the tiled closure kernel
+    bool chunks_chosen = false;        // by the caller or the autotuner: choose_chunks leaves them
+    int cus = 256;                     // compute units of the device
     int tune_learned_iterations = 0;   // leading CG iterations that apply the learned correction (0: all)
     int tune_step_graphs = 1;          // om_time_step replays captured two-step graphs
     int tune_refine = 0;               // FP64 iterative refinement of FFT / Fourier–tridiagonal solves
@@ -294,6 +296,7 @@ template <class T> struct ModelT : ModelBase {
         nf = 3 + nt;
         make_grid(hg, c);
         HIPCHECK(hipGetDevice(&device));
+        HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
         HIPCHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
         HIPCHECK(hipEventCreate(&ev0));
         HIPCHECK(hipEventCreate(&ev1));
@@ -301,6 +304,7 @@ template <class T> struct ModelT : ModelBase {
         g.Nx = hg.N[0]; g.Ny = hg.N[1]; g.Nz = hg.N[2];
         g.Hx = hg.H[0]; g.Hy = hg.H[1]; g.Hz = hg.H[2];
         g.tx = hg.topo[0]; g.ty = hg.topo[1]; g.tz = hg.topo[2];
+        choose_chunks({tend_grid()}, {closure_grid()});
         pnx = g.Nx + 2 * g.Hx; pny = g.Ny + 2 * g.Hy; pnz = g.Nz + 2 * g.Hz + 1;
         {
             const int line = (int)(128 / sizeof(T));   // elements per 128-byte line
@@ -572,6 +576,14 @@ template <class T> struct ModelT : ModelBase {
     uint32_t all_mask() const { return (1u << nf) - 1u; }
 
     // ---- phases
+    MarchGrid tend_grid() const { return MarchGrid{march_tiles(g.Nx, g.Ny, kTendTile), g.Nz}; }
+    MarchGrid closure_grid() const { return MarchGrid{march_tiles(g.Nx, g.Ny, kClosureTile), g.Nz}; }
+    // the tiled kernels' chunks for launches over the given grids (this model's, or a batch's)
+    void choose_chunks(const std::vector<MarchGrid> &tend, const std::vector<MarchGrid> &closure) {
+        if (chunks_chosen) return;
+        tune_kchunk = march_chunk(tend, cus, tend_march_cost(sizeof(T), nt));
+        tune_kchunk_closure = march_chunk(closure, cus, closure_march_cost(sizeof(T)));
+    }
     void compute_tendencies() {
         PhaseScope ps(this, OM_PHASE_TENDENCIES);
         const Ctx<T> C = ctx();
@@ -982,7 +994,8 @@ template <class T> struct ModelT : ModelBase {
     // recorded into R instead of run.  The model's stream is captured meanwhile, so a launch that
     // has no member-table form (it bypasses the recorder) lands in the captured graph, not on the
     // device, and is reported.
-    void record_two_steps(double dt, Recorder &R) {
+    // tend, closure: the batch's grids, for the tiled kernels' chunks.
+    void record_two_steps(double dt, Recorder &R, const std::vector<MarchGrid> &tend, const std::vector<MarchGrid> &closure) {
         if (!capturable()) throw ArgError{"the conjugate-gradient solver's steps read scalars on the host"};
         if (iteration == 0) throw ArgError{"a model's first step is not recorded (it begins with update_state)"};
         HIPCHECK(hipStreamSynchronize(st));
@@ -992,6 +1005,7 @@ template <class T> struct ModelT : ModelBase {
         HIPCHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         thread_recorder() = &R;
         bool threw = false;
+        choose_chunks(tend, closure);
         try {
             step_launches(dt);
             step_launches(dt);
@@ -999,6 +1013,7 @@ template <class T> struct ModelT : ModelBase {
             threw = true;
         }
         thread_recorder() = nullptr;
+        choose_chunks({tend_grid()}, {closure_grid()});
         phase_timing = pt;
         const hipError_t ec = hipStreamEndCapture(st, &gr);
         size_t nodes = 0;
@@ -1039,6 +1054,7 @@ template <class T> struct ModelT : ModelBase {
         if (clo) tune_kchunk_closure = fastest([&](int kc) { launch_closure_tiled(C, kc, st); });
         if (clo && g.kbot) launch_closure(C, st, true);
         tune_kchunk = fastest([&](int kc) { launch_tend_tiled(C, kc, st); });
+        chunks_chosen = true;
         if (g.kbot) launch_tendencies(C, st, true);
         drop_graph();
         return tune_kchunk;
@@ -1712,10 +1728,16 @@ void build_plan(om_ensemble *e, double dt) {
     const size_t n = e->members.size();
     std::vector<Recorder> rec(n);
     int device = -1;
+    std::vector<MarchGrid> tend, closure;
+    for (size_t q = 0; q < n; ++q)
+        (void)WITH_MODEL(e->members[q], { tend.push_back(M->tend_grid()); closure.push_back(M->closure_grid()); });
     for (size_t q = 0; q < n; ++q) {
         om_model_t *m = e->members[q];
         int dev = -1;
-        const int rc = WITH_MODEL(m, { M->record_two_steps(dt, rec[q]); dev = M->device; });
+        const int rc = WITH_MODEL(m, {
+            M->record_two_steps(dt, rec[q], tend, closure);
+            dev = M->device;
+        });
         if (rc != OM_OK) throw ArgError{"member " + std::to_string(q) + ": " + m->err};
         if (q == 0) device = dev;
         else if (dev != device) throw ArgError{"member " + std::to_string(q) + " lives on another device"};
@@ -1951,7 +1973,7 @@ int om_set_tuning(om_model_t *m, int32_t key, int32_t value) {
     if (!known_tuning_key(key)) return OM_EINVAL;
     return WITH_MODEL(m, {
         if (key == OM_TUNE_TENDENCY_KERNEL) M->tune_tendency_kernel = value;
-        else if (key == OM_TUNE_KCHUNK) M->tune_kchunk = M->tune_kchunk_closure = value;
+        else if (key == OM_TUNE_KCHUNK) { M->tune_kchunk = M->tune_kchunk_closure = value; M->chunks_chosen = true; }
         else if (key == OM_TUNE_LEARNED_ITERATIONS) M->tune_learned_iterations = value;
         else if (key == OM_TUNE_STEP_GRAPHS) M->tune_step_graphs = value;
         else if (key == OM_TUNE_CONV_TILED) M->net.tiled_conv = value;

@@ -20,7 +20,7 @@
 
 namespace om {
 
-constexpr int CT = 16;              // cells (and threads) per tile edge
+constexpr int CT = kClosureTile;    // cells (and threads) per tile edge
 constexpr int CW = CT + 2;          // staged plane width: i0-1 .. i0+16
 constexpr int CA = CW * CW;
 

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "om_internal.h"
@@ -707,6 +708,50 @@ inline int fft_lines_per_block(int n, int tables, size_t elem) {
     }
     return 0;
 }
+
+// Levels per block (the z chunk) of a kernel whose blocks march up a tile of columns.  With n =
+// tiles · chunks blocks, m = n / CUs of them per CU and `occ` resident at once, a level of a full CU
+// costs each block one unit of VALU time, a level of a lone block `lat` units of latency, and a block
+// `over` levels beyond its chunk (the state below it; `over_lat` where latency rules).  The last,
+// partly filled round of blocks adds up to a lone block's time:
+//   cost(chunk) = max((chunk + over) (m + lat (1 − frac q) / max(1, ⌊q⌋)), (chunk + over_lat) lat),  q = m / occ.
+// The constants are fits of measured launches of 32³ to 512 × 512 × 256 cells at chunks of 1 to 128
+// (tendencies of 32³ FP32: 103 µs at the former fixed chunk of 16, 16 at 1; 128³ 110 → 99;
+// 256 × 256 × 128 369 → 350).  Chunks do not change results.
+struct MarchCost {
+    int occ;
+    double lat, over, over_lat;
+};
+// The chunk for one launch over the given grids (a batch's members share one: a member with longer
+// chunks than the rest would end the launch alone).
+struct MarchGrid {
+    int tiles, Nz;
+};
+inline int march_chunk(const std::vector<MarchGrid> &grids, int cus, const MarchCost &M) {
+    int best = 1, most = 1;
+    for (const MarchGrid &g : grids) most = std::max(most, std::min(g.Nz, 64));
+    double least = INFINITY, before = 0;
+    for (int kc = 1; kc <= most; ++kc) {
+        double blocks = 0;
+        for (const MarchGrid &g : grids) blocks += (double)g.tiles * ((g.Nz + kc - 1) / kc);
+        if (blocks == before) continue;   // the same chunks, less evenly filled
+        before = blocks;
+        const double m = blocks / cus, q = m / M.occ, f = q - std::floor(q);
+        const double tail = f > 0 ? M.lat * (1.0 - f) / std::max(1.0, std::floor(q)) : 0.0;
+        const double c = std::max((kc + M.over) * (m + tail), (kc + M.over_lat) * M.lat);
+        if (c < 0.999 * least) { least = c; best = kc; }
+    }
+    return best;
+}
+inline MarchCost tend_march_cost(size_t elem, int n_tracers) {
+    if (elem == 8) return MarchCost{2, 1.4, 0.65, 1.6};
+    return n_tracers <= 1 ? MarchCost{5, 2.4, 0.65, 1.6} : MarchCost{4, 2.1, 0.65, 1.6};
+}
+inline MarchCost closure_march_cost(size_t elem) {
+    return elem == 8 ? MarchCost{3, 1.6, 0.8, 2.9} : MarchCost{5, 2.0, 0.8, 2.9};
+}
+constexpr int kTendTile = 15, kClosureTile = 16;   // cells per tile edge of the two kernels
+inline int march_tiles(int Nx, int Ny, int edge) { return ((Nx + edge - 1) / edge) * ((Ny + edge - 1) / edge); }
 
 // The generic kernels over every cell, or (fixup) only over the cells below kfix of an immersed
 // grid, after the tiled kernels have covered the rest

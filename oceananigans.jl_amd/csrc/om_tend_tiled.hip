@@ -32,7 +32,7 @@
 namespace om {
 
 constexpr int TT = 16;            // threads per tile edge
-constexpr int TC = 15;            // cells per tile edge
+constexpr int TC = kTendTile;     // cells per tile edge
 constexpr int PW = TT + 5;        // staged plane width: i0-3 .. i0+17
 constexpr int PA = PW * PW;
 constexpr int NWD = TT + 1;       // ν / κ plane width: i0-1 .. i0+15
