@@ -576,12 +576,15 @@ template <class T> struct ModelT : ModelBase {
     uint32_t all_mask() const { return (1u << nf) - 1u; }
 
     // ---- phases
-    MarchGrid tend_grid() const { return MarchGrid{march_tiles(g.Nx, g.Ny, kTendTile), g.Nz}; }
-    MarchGrid closure_grid() const { return MarchGrid{march_tiles(g.Nx, g.Ny, kClosureTile), g.Nz}; }
+    MarchGrid tend_grid() const {
+        return cfg.advection == OM_ADV_CENTERED2 ? MarchGrid{march_tiles(g.Nx, g.Ny, kCenteredX, kCenteredY), g.Nz}
+                                                 : MarchGrid{march_tiles(g.Nx, g.Ny, kTendTile, kTendTile), g.Nz};
+    }
+    MarchGrid closure_grid() const { return MarchGrid{march_tiles(g.Nx, g.Ny, kClosureTile, kClosureTile), g.Nz}; }
     // the tiled kernels' chunks for launches over the given grids (this model's, or a batch's)
     void choose_chunks(const std::vector<MarchGrid> &tend, const std::vector<MarchGrid> &closure) {
         if (chunks_chosen) return;
-        tune_kchunk = march_chunk(tend, cus, tend_march_cost(sizeof(T), nt));
+        tune_kchunk = march_chunk(tend, cus, cfg.advection == OM_ADV_CENTERED2 ? centered_march_cost(sizeof(T)) : tend_march_cost(sizeof(T), nt));
         tune_kchunk_closure = march_chunk(closure, cus, closure_march_cost(sizeof(T)));
     }
     void compute_tendencies() {
@@ -590,6 +593,8 @@ template <class T> struct ModelT : ModelBase {
         if (tune_tendency_kernel == 0 && tiled_tendencies_supported(C)) {
             launch_tend_tiled(C, tune_kchunk, st);
             if (g.kbot) launch_tendencies(C, st, true);   // cells within reach of the immersed bottom
+        } else if (tune_tendency_kernel == 0 && centered_tendencies_supported(C)) {
+            launch_tend_centered(C, tune_kchunk, st);
         } else {
             launch_tendencies(C, st);
         }

@@ -205,18 +205,18 @@ __device__ __forceinline__ int xcd_work_item(int id, int nb) {
     return (id & 7) * per + (id >> 3);
 }
 
-// A thread's share of a W × W plane staged into LDS by a 256-thread block: plane elements tid and
+// A thread's share of a plane of R rows of W, staged into LDS by a 256-thread block: plane elements tid and
 // tid + 256 (row-major, origin (i0 − h, j0 − h)).  The byte offset of the first from the plane origin
 // is computed once per block and the second's follows from it (256 elements further on: a fixed
 // number of rows and columns, and one row more where the column wraps), so staging a level costs one
 // scalar origin per field and a load per element, and every load of a level can be issued before the
 // first LDS store.  Offsets are held inside the level's plane, so no load is predicated: what the
-// elements beyond the field's last halo point (or past the W × W elements) read is never used.
-template <class T, int W> struct PlaneShare {
+// elements beyond the field's last halo point read is never used.
+template <class T, int W, int R = W> struct PlaneShare {
     uint32_t off0, step, wrapstep, most;   // (the last three are the same for the whole block)
     bool wraps;
     __device__ __forceinline__ PlaneShare(const DevGrid<T> &g, int i0, int j0, int h, int tid) {
-        static_assert(W * W >= 256 && W * W <= 512, "two elements per thread");
+        static_assert(W * R >= 256 && W * R <= 512, "two elements per thread");
         constexpr uint32_t e = sizeof(T);
         const int y = tid / W, x = tid - y * W;
         most = (uint32_t)(g.sz - 1 - ((int64_t)(j0 - h + g.Hy) * g.sy + (i0 - h + g.Hx))) * e;
@@ -232,11 +232,11 @@ template <class T, int W> struct PlaneShare {
     __device__ __forceinline__ uint32_t off1() const { return min(off0 + (wraps ? wrapstep : step), most); }
     __device__ __forceinline__ static void load(T (&v)[2], const char *base, uint32_t o0, uint32_t o1) {
         v[0] = *reinterpret_cast<const T *>(base + o0);
-        if (threadIdx.x < W * W - 256) v[1] = *reinterpret_cast<const T *>(base + o1);
+        if (threadIdx.x < W * R - 256) v[1] = *reinterpret_cast<const T *>(base + o1);
     }
     __device__ __forceinline__ static void store(T *dst, const T (&v)[2], int tid) {
         dst[tid] = v[0];
-        if (tid < W * W - 256) dst[tid + 256] = v[1];
+        if (tid < W * R - 256) dst[tid + 256] = v[1];
     }
 };
 
@@ -747,18 +747,23 @@ inline MarchCost tend_march_cost(size_t elem, int n_tracers) {
     if (elem == 8) return MarchCost{2, 1.4, 0.65, 1.6};
     return n_tracers <= 1 ? MarchCost{5, 2.4, 0.65, 1.6} : MarchCost{4, 2.1, 0.65, 1.6};
 }
+inline MarchCost centered_march_cost(size_t elem) { return elem == 8 ? MarchCost{4, 2.0, 0.5, 3.0} : MarchCost{6, 2.5, 0.5, 3.0}; }
 inline MarchCost closure_march_cost(size_t elem) {
     return elem == 8 ? MarchCost{3, 1.6, 0.8, 2.9} : MarchCost{5, 2.0, 0.8, 2.9};
 }
 constexpr int kTendTile = 15, kClosureTile = 16;   // cells per tile edge of the two kernels
-inline int march_tiles(int Nx, int Ny, int edge) { return ((Nx + edge - 1) / edge) * ((Ny + edge - 1) / edge); }
+constexpr int kCenteredX = 32, kCenteredY = 8;     // and of the centered tendency kernel's tile
+inline int march_tiles(int Nx, int Ny, int ex, int ey) { return ((Nx + ex - 1) / ex) * ((Ny + ey - 1) / ey); }
 
 // The generic kernels over every cell, or (fixup) only over the cells below kfix of an immersed
 // grid, after the tiled kernels have covered the rest
 constexpr int kImmersedReach = 5;   // farthest offset of an immersed-boundary query from its cell, plus one
 constexpr int kGenericBlockX = 64, kGenericBlockY = 4;   // block shape of k_tendencies / k_closure
 template <class T> void launch_tendencies(const Ctx<T> &C, hipStream_t st, bool fixup = false);
-// z-marching LDS-tiled tendency kernel (om_tend_tiled.hip) and the configurations it covers
+// z-marching tendency kernels: WENO(order=5) (om_tend_tiled.hip) and Centered(order=2) with constant or
+// no diffusivity (om_tend_centered.hip), and the configurations they cover
+template <class T> bool centered_tendencies_supported(const Ctx<T> &C);
+template <class T> void launch_tend_centered(const Ctx<T> &C, int kchunk, hipStream_t st);
 template <class T> bool tiled_tendencies_supported(const Ctx<T> &C);
 template <class T> void launch_tend_tiled(const Ctx<T> &C, int kchunk, hipStream_t st);
 template <class T> void launch_closure(const Ctx<T> &C, hipStream_t st, bool fixup = false);
