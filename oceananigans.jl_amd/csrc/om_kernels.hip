@@ -267,50 +267,60 @@ template <class T> __global__ void __launch_bounds__(256) k_closure(Ctx<T> C, in
 // ----------------------------------------------------------------------------------------
 // Hydrostatic pressure anomaly: downward column integral (update_hydrostatic_pressure.jl:11-21)
 // ----------------------------------------------------------------------------------------
+// FP64, in the reference's order: the column sum cancels between neighbouring columns when ∂x pHY′ is
+// formed, so it is accumulated from the top down without FMA contraction.  A block takes 64 columns of a
+// row and slabs of kHySlab levels: its eight waves form the slab's terms ½(b(k) + b(k+1))·Δzᶠ(k+1) in
+// parallel into LDS, one wave runs the serial sum down them, and all waves store the result.  The
+// serial part is additions from LDS only (128³: 33.8 µs with the loads in the
+// chain of one thread per column, 256 waves on the device, → 14.3 µs).
+constexpr int kHySlab = 64, kHyWaves = 8;
 template <class T> struct KHydrostatic {
-    static constexpr int kThreads = 256, kMinBlocks = 1;
+    static constexpr int kThreads = 64 * kHyWaves, kMinBlocks = 1;
     static __device__ __forceinline__ void run(const CtxArgs<T> &A, const Blk &B);
 };
 template <class T> __device__ __forceinline__ void KHydrostatic<T>::run(const CtxArgs<T> &A, const Blk &Bk) {
-    // The column sum cancels between neighbouring columns when ∂x pHY′ is formed; it is
-    // accumulated without FMA contraction, in the reference's order.
 #pragma clang fp contract(off)
+    __shared__ T term[kHySlab][64];
     const Ctx<T> &C = A.C;
-    const int i = Bk.x * blockDim.x + threadIdx.x;
-    const int j = Bk.y * blockDim.y + threadIdx.y;
-    if (i >= C.g.Nx || j >= C.g.Ny) return;
+    const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int i = Bk.x * 64 + lane, j = Bk.y;
+    const bool col = i < C.g.Nx;
     const int Nz = C.g.Nz;
-    T bk = C.buoy(i, j, Nz);                      // halo value b[Nz+1] (0-based index Nz)
-    T bkm = C.buoy(i, j, Nz - 1);
-    T p = -(T(0.5) * (bkm + bk)) * C.g.dzf[Nz];
-    C.s.pHY[C.at(i, j, Nz - 1)] = p;
-    // One thread per column gives one wave per SIMD, so the memory latency is hidden within each
-    // thread: the buoyancy is loaded in batches of B levels, double-buffered, the next batch's
-    // loads issued before the current batch is integrated (a load placed after a store to pHY′
-    // cannot be moved above it, as the arrays might alias).
-    constexpr int B = sizeof(T) == 4 ? 32 : 16;
-    T ba[B], bb[B];
-    auto load = [&](T (&buf)[B], int top) {
+    constexpr int per = kHySlab / kHyWaves;
+    T p = T(0);   // (wave 0: the sum so far)
+    for (int top = Nz - 1; top >= 0; top -= kHySlab) {
+        // this wave's levels of the slab: top − wave·per − q
+        const int t0 = top - wave * per;
+        if (col) {
+            T b[per + 1];
 #pragma unroll
-        for (int q = 0; q < B; ++q) buf[q] = top - q >= 0 ? C.buoy(i, j, top - q) : T(0);
-    };
-    auto integrate = [&](const T (&buf)[B], int top) {
+            for (int q = 0; q <= per; ++q) b[q] = C.buoy(i, j, max(t0 + 1 - q, 0));
 #pragma unroll
-        for (int q = 0; q < B; ++q) {
-            if (top - q < 0) break;
-            bk = bkm;
-            bkm = buf[q];
-            p -= (T(0.5) * (bkm + bk)) * C.g.dzf[top - q + 1];
-            C.s.pHY[C.at(i, j, top - q)] = p;
+            for (int q = 0; q < per; ++q)
+                if (t0 - q >= 0) term[wave * per + q][lane] = (T(0.5) * (b[q + 1] + b[q])) * C.g.dzf[t0 - q + 1];
         }
-    };
-    int k = Nz - 2;
-    load(ba, k);
-    for (; k >= 0; k -= 2 * B) {
-        load(bb, k - B);
-        integrate(ba, k);
-        load(ba, k - 2 * B);
-        integrate(bb, k - B);
+        __syncthreads();
+        if (wave == 0) {
+            // (rows past the column's lowest level hold stale terms; their sums are not stored)
+            constexpr int U = 8;
+            for (int q0 = 0; q0 < kHySlab; q0 += U) {
+                T t[U];
+#pragma unroll
+                for (int q = 0; q < U; ++q) t[q] = term[q0 + q][lane];
+#pragma unroll
+                for (int q = 0; q < U; ++q) {
+                    p = top == Nz - 1 && q0 + q == 0 ? -t[q] : p - t[q];
+                    term[q0 + q][lane] = p;
+                }
+            }
+        }
+        __syncthreads();
+        if (col) {
+#pragma unroll
+            for (int q = 0; q < per; ++q)
+                if (t0 - q >= 0) C.s.pHY[C.at(i, j, t0 - q)] = term[wave * per + q][lane];
+        }
+        __syncthreads();
     }
 }
 
@@ -327,7 +337,10 @@ template <class T> __device__ __forceinline__ void KHydrostatic<T>::run(const Ct
 // the segment totals are exchanged through LDS, and p(m) = −(terms of the segments above + the
 // running sum at m).  KHydrostaticSeg (any Nz, four segments): the same in two passes, the first
 // for the totals, the second recomputing the terms.  Both associate the reference's sequential sum
-// in segments, so FP32 results differ from the sequential order by rounding only.
+// in segments, so FP32 results differ from the sequential order by rounding only.  Memory latency
+// bounds the scan: with every load of a segment issued first and none under a condition, from scalar
+// level origins, 58 → 36 µs at 256 × 256 × 128 (3.7 TB/s of its 134 MB), 687 → 487 µs at 512 × 512 × 256
+// with temperature and salinity (2.8 TB/s).
 constexpr int kHyLevels = 16;
 
 template <class T, int S> struct KHydrostaticReg {
@@ -343,57 +356,92 @@ template <class T, int S> __device__ __forceinline__ void KHydrostaticReg<T, S>:
     const int item = xcd_work_item((int)B.x, (int)B.gx);
     const int i = (item % nbx) * 64 + threadIdx.x;
     const int j = item / nbx;
-    const int seg = threadIdx.y, nseg = blockDim.y;
+    const int seg = __builtin_amdgcn_readfirstlane(threadIdx.y), nseg = blockDim.y;   // (a wave is one segment)
     const int Nz = C.g.Nz;
     const int per = (Nz + nseg - 1) / nseg;
-    const int lo = seg * per, hi = min(Nz, lo + per);   // levels lo .. hi-1 of this segment
+    const int lo = min(seg * per, Nz), hi = min(Nz, lo + per);   // levels lo .. hi-1 of this segment
     const bool col = i < C.g.Nx;
     const bool diff = C.s.dxpHY != nullptr;
-    T tp[kHyLevels], tx[kHyLevels], ty[kHyLevels];
-    T rp = T(0), rx = T(0), ry = T(0);
+    // this thread's columns through scalar level origins one row and one column back (so that no
+    // offset is negative): its own, that of row j − 1 and that of column i − 1
+    const int64_t back = C.g.sy + 1;
+    const uint32_t here = (uint32_t)((idx3(i, j, 0, C.g.sy, C.g.sz) + back) * (int64_t)sizeof(T));
+    const uint32_t below = here - (uint32_t)(C.g.sy * (int64_t)sizeof(T)), left = here - (uint32_t)sizeof(T);
+    auto at = [](const T *f, int64_t lev, uint32_t off) { return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(f + lev) + off); };
+    // b, b(i) − b(i−1) and b(j) − b(j−1) at levels hi − q (q = 0 the level above the segment; below it
+    // the lowest level again, unused): every load of the segment is issued before the first sum, none
+    // under a condition
+    T bq[kHyLevels + 1], xq[kHyLevels + 1], yq[kHyLevels + 1];
     if (col) {
-        // terms m = hi-1 down to lo; b(m+1) at m = Nz-1 is the halo value b(Nz)
-        T bu = C.buoy(i, j, hi);
-        T xu = diff ? C.buoy_diff(i, j, hi, 1, 0) : T(0), yu = diff ? C.buoy_diff(i, j, hi, 0, 1) : T(0);
+        const T *ba = C.ph.buoyancy == OM_BUOYANCY_TRACER ? C.s.btr : C.s.Ttr, *bs = C.s.Str;
+        const bool none = C.ph.buoyancy == OM_BUOYANCY_NONE;   // (an anomaly of zeros)
+        const bool eos = C.ph.buoyancy == OM_BUOYANCY_LINEAR_EOS;
+#pragma unroll
+        for (int q = 0; q <= kHyLevels; ++q) {
+            const int64_t lev = (int64_t)max(hi - q, lo) * C.g.sz - back;
+            bq[q] = none ? T(0) : at(ba, lev, here);
+            if (diff) {
+                xq[q] = none ? T(0) : bq[q] - at(ba, lev, left);
+                yq[q] = none ? T(0) : bq[q] - at(ba, lev, below);
+            }
+        }
+        if (eos) {
+            // Ctx::buoy and Ctx::buoy_diff from the temperatures above and the salinities
+#pragma unroll
+            for (int q = 0; q <= kHyLevels; ++q) {
+                const int64_t lev = (int64_t)max(hi - q, lo) * C.g.sz - back;
+                const T s0 = at(bs, lev, here);
+                if (diff) {
+                    const T sx = s0 - at(bs, lev, left), sy = s0 - at(bs, lev, below);
+                    xq[q] = C.ph.g * (C.ph.alpha * xq[q] - C.ph.beta * sx);
+                    yq[q] = C.ph.g * (C.ph.alpha * yq[q] - C.ph.beta * sy);
+                }
+                bq[q] = C.ph.g * (C.ph.alpha * bq[q] - C.ph.beta * s0);
+            }
+        }
+        // running sums of the terms ½(b(m) + b(m+1))·Δzᶠ(m+1), m = hi − 1 − q, in place
+        T rp = T(0), rx = T(0), ry = T(0);
 #pragma unroll
         for (int q = 0; q < kHyLevels; ++q) {
             const int m = hi - 1 - q;
-            if (m < lo) break;
-            const T bm = C.buoy(i, j, m);
-            rp += (T(0.5) * (bm + bu)) * C.g.dzf[m + 1];
-            tp[q] = rp;
-            bu = bm;
+            const T dz = C.g.dzf[max(m, 0) + 1];
+            const bool in = m >= lo;
+            const T r = rp + (T(0.5) * (bq[q + 1] + bq[q])) * dz;
+            bq[q] = rp = in ? r : rp;
             if (diff) {
-                const T xm = C.buoy_diff(i, j, m, 1, 0), ym = C.buoy_diff(i, j, m, 0, 1);
-                rx += (T(0.5) * (xm + xu)) * C.g.dzf[m + 1];
-                ry += (T(0.5) * (ym + yu)) * C.g.dzf[m + 1];
-                tx[q] = rx;
-                ty[q] = ry;
-                xu = xm;
-                yu = ym;
+                const T x = rx + (T(0.5) * (xq[q + 1] + xq[q])) * dz, y = ry + (T(0.5) * (yq[q + 1] + yq[q])) * dz;
+                xq[q] = rx = in ? x : rx;
+                yq[q] = ry = in ? y : ry;
             }
         }
     }
-    tot[0][seg][threadIdx.x] = rp;
-    tot[1][seg][threadIdx.x] = rx;
-    tot[2][seg][threadIdx.x] = ry;
+    if (col) {
+        tot[0][seg][threadIdx.x] = bq[kHyLevels - 1];
+        if (diff) {
+            tot[1][seg][threadIdx.x] = xq[kHyLevels - 1];
+            tot[2][seg][threadIdx.x] = yq[kHyLevels - 1];
+        }
+    }
     __syncthreads();
     if (!col) return;
     T ap = T(0), ax = T(0), ay = T(0);
     for (int s2 = seg + 1; s2 < nseg; ++s2) {
         ap += tot[0][s2][threadIdx.x];
-        ax += tot[1][s2][threadIdx.x];
-        ay += tot[2][s2][threadIdx.x];
+        if (diff) {
+            ax += tot[1][s2][threadIdx.x];
+            ay += tot[2][s2][threadIdx.x];
+        }
     }
 #pragma unroll
     for (int q = 0; q < kHyLevels; ++q) {
         const int m = hi - 1 - q;
         if (m < lo) break;
-        const int64_t o = C.at(i, j, m);
-        C.s.pHY[o] = -(ap + tp[q]);
+        const int64_t lev = (int64_t)m * C.g.sz - back;
+        auto put = [&](T *f, T v) { *reinterpret_cast<T *>(reinterpret_cast<char *>(f + lev) + here) = v; };
+        put(C.s.pHY, -(ap + bq[q]));
         if (diff) {
-            C.s.dxpHY[o] = -(ax + tx[q]);
-            C.s.dypHY[o] = -(ay + ty[q]);
+            put(C.s.dxpHY, -(ax + xq[q]));
+            put(C.s.dypHY, -(ay + yq[q]));
         }
     }
 }
@@ -865,8 +913,7 @@ template <class T> void launch_hydrostatic(const Ctx<T> &C, hipStream_t st) {
         launch_k<KHydrostaticSeg<T>>(dim3((C.g.Nx + 63) / 64, C.g.Ny), blk, 0, st, CtxArgs<T>{C});
         return;
     }
-    dim3 blk(64, 4, 1);
-    launch_k<KHydrostatic<T>>(cell_grid(C.g.Nx, C.g.Ny, 1, blk), blk, 0, st, CtxArgs<T>{C});
+    launch_k<KHydrostatic<T>>(dim3((C.g.Nx + 63) / 64, C.g.Ny), dim3(64, kHyWaves), 0, st, CtxArgs<T>{C});
 }
 template <class T> void launch_rk3(const Ctx<T> &C, T dt, T gamma, T zeta, int first, int nfields, hipStream_t st) {
     dim3 blk(64, 4, 1);
