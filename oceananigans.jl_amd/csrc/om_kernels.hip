@@ -271,8 +271,8 @@ template <class T> __global__ void __launch_bounds__(256) k_closure(Ctx<T> C, in
 // formed, so it is accumulated from the top down without FMA contraction.  A block takes 64 columns of a
 // row and slabs of kHySlab levels: its eight waves form the slab's terms ½(b(k) + b(k+1))·Δzᶠ(k+1) in
 // parallel into LDS, one wave runs the serial sum down them, and all waves store the result.  The
-// serial part is additions from LDS only (128³: 33.8 µs with the loads in the
-// chain of one thread per column, 256 waves on the device, → 14.3 µs).
+// serial part is additions from LDS only (128³: 33.8 µs with the loads in the chain of one thread per
+// column, 256 waves on the device, → 14.3 µs).
 constexpr int kHySlab = 64, kHyWaves = 8;
 template <class T> struct KHydrostatic {
     static constexpr int kThreads = 64 * kHyWaves, kMinBlocks = 1;

@@ -99,7 +99,9 @@ template <class T> __device__ __forceinline__ void stage_small(T *dst, const T *
 // Occupancy: with up to one tracer the FP32 kernel fits 96 VGPRs without spilling, i.e. 5 waves per
 // SIMD (5 blocks per CU, 156 KiB of LDS; 4 waves with the parked values in registers instead: 384
 // against 355 µs at 256 × 256 × 128), with two tracers 128; the hint asks the compiler for that
-// budget.  FP64 needs 182 to 250 VGPRs, 2 waves; a third (168) spills 53 and is slower (268 → 315 µs).
+// budget.  FP64 takes 164 to 246 VGPRs, 2 waves; a third (168)
+// with one tracer spills 38, or 16 with half of the differences parked, and is slower (128³: 208 → 272
+// and 228 µs).
 template <class T, int NT> constexpr int tend_min_blocks() { return sizeof(T) == 4 ? (NT <= 1 ? 5 : 4) : 1; }
 
 template <class T> struct TendTiledArgs {
