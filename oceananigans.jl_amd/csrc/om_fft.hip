@@ -720,15 +720,18 @@ template <class T, bool MIXED> __device__ __forceinline__ void KZPass<T, MIXED>:
 }
 
 // ---------------------------------------------------------------------------------------------
-// Fourier–tridiagonal z solve (Thomas per (kx, ky) column; diagonals from
-// fourier_tridiagonal_poisson_solver.jl:199-229).  One thread per column, the columns ℓ = ky·Ms + kx
-// flattened so that a level of a block's columns is one contiguous run (level k of column ℓ at
-// k·(Ms·Ny) + ℓ; columns with kx ≥ Mx are row padding and are skipped); t[k] kept in LDS.  Each sweep
-// reads its levels in batches of tri_batch (16 FP32, 8 FP64), all
-// loads of a batch issued before its arithmetic, so a column costs 2·Nz/batch memory round
-// trips instead of 2·Nz.  The (0,0) column is singular: its last pivot is a rounding residue and
-// is elided as in the reference; the constant this leaves is removed with the column mean
-// (ϕ -= mean(ϕ), :253).
+// Fourier–tridiagonal z solve per (kx, ky) column (diagonals from
+// fourier_tridiagonal_poisson_solver.jl:199-229).  Two lanes of one wave share a column and eliminate
+// towards its middle level, one from the bottom and one from the top; the middle level's equation
+// closes the two chains and both substitute back outwards.  Columns ℓ = ky·Ms + kx are flattened, so that a level of a block's columns is one
+// contiguous run (level k of column ℓ at k·(Ms·Ny) + ℓ; columns with kx ≥ Mx are row padding, never
+// stored).  The chain's memory round trips bound it: a batch of tri_batch levels (16 FP32, 8 FP64) is
+// loaded while the one before it is eliminated, and with KEEP the eliminated column stays in LDS (else,
+// for columns too long for that, only its ratios do, and its values go through the spectrum's memory).
+// The (0,0) column is singular, and the reference elides its last pivot: the top level's equation is
+// the one that a source with a volume integral leaves unmet.  Here that level's source is replaced by
+// what makes the column solvable, which has the same solution, and the closing pivot is elided;
+// the constant this leaves is removed with the column mean (ϕ -= mean(ϕ), :253).
 // ---------------------------------------------------------------------------------------------
 template <class T> struct TriArgs {
     DevGrid<T> g;
@@ -740,97 +743,276 @@ template <class T> struct TriArgs {
 };
 
 template <class T> constexpr int tri_batch() { return sizeof(T) == 4 ? 16 : 8; }
+// LDS bytes of a block of bw columns
+template <class T> constexpr size_t tri_lds(int Nz, int bw, bool keep) {
+    return ((size_t)Nz * bw * (keep ? 3 : 1) + 2 * (size_t)Nz + 1) * sizeof(T);
+}
 
-// The level coefficients and the spectrum come in as restrict-qualified arguments: the sweeps'
-// stores to S then provably leave them alone, so their (column-uniform) loads stay scalar.
-template <class T>
+template <class T, bool KEEP>
 __global__ void __launch_bounds__(64) k_tridiag(TriArgs<T> A, C2<T> *__restrict__ Sg, const T *__restrict__ dzc,
                                                 const T *__restrict__ idzf) {
-    extern __shared__ unsigned char smem_raw[];
-    T *tt = reinterpret_cast<T *>(smem_raw);   // [Nz][blockDim.x]
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     constexpr int KB = tri_batch<T>();
     const int Ny = A.g.Ny, Nz = A.g.Nz, Mx = A.Mx;
-    const int bw = blockDim.x;
-    const int64_t ncol = (int64_t)A.Ms * Ny;   // columns ℓ = ky·Ms + kx, padding columns kx ≥ Mx skipped
-    const int64_t col = (int64_t)blockIdx.x * bw + threadIdx.x;
-    if (col >= ncol) return;
-    const int j = (int)(col / A.Ms), kx = (int)(col - (int64_t)j * A.Ms);
-    if (kx >= Mx) return;
+    const int bw = blockDim.x >> 1;            // columns of the block
+    C2<T> *ph = reinterpret_cast<C2<T> *>(smem_raw);                  // KEEP: [Nz][bw]
+    T *tt = reinterpret_cast<T *>(ph + (KEEP ? (size_t)Nz * bw : 0));   // [Nz][bw]
+    T *dz = tt + (size_t)Nz * bw;              // [Nz] Δzᶜ
+    T *iz = dz + Nz;                           // [Nz + 1] 1/Δzᶠ, the end faces 0
+    const bool down = (int)threadIdx.x >= bw;   // this lane's chain: from the top
+    const int c = threadIdx.x - (down ? bw : 0);
+    const int64_t ncol = (int64_t)A.Ms * Ny;
+    const int64_t col = min((int64_t)blockIdx.x * bw + c, ncol - 1);   // (lanes past the end repeat the last)
+    const int j = (int)(col / A.Ms), kx = min((int)(col - (int64_t)j * A.Ms), Mx - 1);
+    const bool store = (int64_t)blockIdx.x * bw + c == col && col - (int64_t)j * A.Ms < Mx;
     const T lam = A.lx[kx] + A.ly[j];
-    auto diag = [&](int k) -> T {   // 0-based k
-        const T dz = dzc[k];
-        if (Nz == 1) return -dz * lam;
-        if (k == 0) return -idzf[1] - dz * lam;
-        if (k == Nz - 1) return -idzf[Nz - 1] - dz * lam;
-        return -(idzf[k + 1] + idzf[k]) - dz * lam;
-    };
-    auto off = [&](int k) -> T { return idzf[k + 1]; };   // a[k] = c[k] = 1/Δzᶠ(k+1) (reference q = k+1)
+
     C2<T> *S = Sg + col;
+    const int mid = Nz >> 1;                        // the closing level
+    const int steps = down ? Nz - 1 - mid : mid;    // levels of this chain
+    const int longest = mid, common = Nz - 1 - mid;
+    auto level = [&](int q) -> int { return down ? Nz - 1 - q : q; };
     auto at = [&](int k) -> int64_t { return (int64_t)k * ncol; };
-    // forward sweep: level 0, then full batches of KB levels (loads first), then the rest
-    // (ft_div: IEEE division in FP64, as the reference's Thomas sweep; the hardware reciprocal in
-    // FP32, which shortens the serial chain through β at each level)
-    T beta = diag(0);
-    C2<T> phi;
-    {
-        const C2<T> f = S[0];
-        phi = cmk<T>(ft_div<T>(f.x, beta), ft_div<T>(f.y, beta));
-        S[0] = phi;
-    }
-    auto fwd = [&](int k, const C2<T> &f) {
-        const T c = off(k - 1), a = off(k - 1);
-        const T t = ft_div<T>(c, beta);
-        tt[k * bw + threadIdx.x] = t;
-        beta = diag(k) - a * t;
-        if (fabs(beta) > A.eps10) phi = cmk<T>(ft_div<T>(f.x - a * phi.x, beta), ft_div<T>(f.y - a * phi.y, beta));
+    // a chain longer than its column's half reads a level of the other half, and drops it
+    auto load = [&](C2<T> (&f)[KB], int q0) {
+#pragma unroll
+        for (int u = 0; u < KB; ++u) f[u] = S[at(level(min(q0 + u, longest)))];
+    };
+    // The chain carries each pivot as −(next + excess), where excess = Δz·λ + before·excess_prev / (before +
+    // excess_prev) collects what exceeds the couplings: sums and products of positive numbers, so the
+    // nearly singular columns of the longest waves keep the whole precision that the differences of a
+    // pivot's recurrence lose.
+    // (ft_div: IEEE division in FP64; the hardware reciprocal in FP32, which shortens the serial chain)
+    T excess = T(0);
+    T ratio = T(0);                    // coupling / −pivot of the chain's last level
+    C2<T> phi = cmk<T>(T(0), T(0));    // its right-hand side / pivot
+    // level q with couplings `before` (towards the chain's start) and `next`, and spacing d
+    auto eliminate = [&](int q, const C2<T> &f, T before, T next, T d) {
+        const int k = level(q);
+        excess = d * lam + excess * ratio;
+        const T pivot = next + excess;
+        ratio = ft_div<T>(next, pivot);
+        if (q == 0 || pivot > A.eps10) phi = cmk<T>(ft_div<T>(before * phi.x - f.x, pivot), ft_div<T>(before * phi.y - f.y, pivot));
         else phi = cmk<T>(T(0), T(0));
-        S[at(k)] = phi;
+        tt[k * bw + c] = ratio;
+        if (KEEP) ph[k * bw + c] = phi;
+        else if (store) S[at(k)] = phi;
     };
-    int k = 1;
-    for (; k + KB <= Nz; k += KB) {
-        C2<T> f[KB];
-#pragma unroll
-        for (int u = 0; u < KB; ++u) f[u] = S[at(k + u)];
-#pragma unroll
-        for (int u = 0; u < KB; ++u) fwd(k + u, f[u]);
+    const C2<T> fmid = S[at(mid)];
+    C2<T> f[KB];
+    load(f, 0);
+    for (int k = threadIdx.x; k < Nz; k += blockDim.x) {
+        dz[k] = dzc[k];
+        iz[k] = k == 0 ? T(0) : idzf[k];
     }
-    for (; k < Nz; ++k) fwd(k, S[at(k)]);
-    // backward substitution from level Nz − 2 down, in the same batches; the column's sum is
-    // accumulated on the way (used by the (0,0) column only, top level first)
-    C2<T> colsum = phi;
-    auto bwd = [&](int kk, const C2<T> &p) {
-        const T t = tt[(kk + 1) * bw + threadIdx.x];
-        const C2<T> q = cmk<T>(p.x - t * phi.x, p.y - t * phi.y);
-        S[at(kk)] = q;
-        phi = q;
-        colsum = cadd<T>(colsum, q);
+    if (threadIdx.x == 0) iz[Nz] = T(0);
+    __syncthreads();
+    const bool singular = lam == T(0);   // the (0,0) column
+    if (blockIdx.x == 0) {
+        C2<T> below = cmk<T>(T(0), T(0));   // (its source without the top level, summed by the whole wave)
+        for (int k = threadIdx.x; k < Nz - 1; k += blockDim.x) below = cadd<T>(below, Sg[at(k)]);
+        for (int o = bw; o > 0; o >>= 1) below = cadd<T>(below, cmk<T>(__shfl_xor(below.x, o), __shfl_xor(below.y, o)));
+        if (singular && down) f[0] = cmk<T>(-below.x, -below.y);
+    }
+    for (int q0 = 0; q0 < longest; q0 += KB) {
+        C2<T> nxt[KB];
+        load(nxt, q0 + KB);   // (also beyond the end, repeating a level: where a branch could have left these loads out, the
+                              // waits for the batch at hand would wait for them)
+        // (the batch's coefficients before its arithmetic, whose stores to LDS they could not pass)
+        T w[KB + 1], d[KB];
+#pragma unroll
+        for (int u = 0; u <= KB; ++u) w[u] = iz[down ? Nz - min(q0 + u, Nz) : min(q0 + u, Nz)];
+#pragma unroll
+        for (int u = 0; u < KB; ++u) d[u] = dz[level(min(q0 + u, longest))];
+        if (q0 + KB <= common) {
+#pragma unroll
+            for (int u = 0; u < KB; ++u) eliminate(q0 + u, f[u], w[u], w[u + 1], d[u]);
+        } else {
+#pragma unroll
+            for (int u = 0; u < KB; ++u)
+                if (q0 + u < steps) eliminate(q0 + u, f[u], w[u], w[u + 1], d[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < KB; ++u) f[u] = nxt[u];
+    }
+    // the closing level: its neighbours' chains end in (excess, ratio, phi) of the two lanes
+    C2<T> x;
+    {
+        const T eb = __shfl(excess, c) * __shfl(ratio, c), et = __shfl(excess, c + bw) * __shfl(ratio, c + bw);
+        const C2<T> pb = cmk<T>(__shfl(phi.x, c), __shfl(phi.y, c)), pt = cmk<T>(__shfl(phi.x, c + bw), __shfl(phi.y, c + bw));
+        const T below = iz[mid], above = iz[mid + 1];
+        const T pivot = dz[mid] * lam + (eb + et);
+        if (!singular && pivot > A.eps10)
+            x = cmk<T>(ft_div<T>((below * pb.x - fmid.x) + above * pt.x, pivot), ft_div<T>((below * pb.y - fmid.y) + above * pt.y, pivot));
+        else x = cmk<T>(T(0), T(0));
+    }
+    C2<T> sum = down ? cmk<T>(T(0), T(0)) : x;
+    if (store && !down) S[at(mid)] = x;
+    auto fetch = [&](C2<T> (&p)[KB], int q0) {   // levels q0, q0 − 1, …
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            const int k = level(max(q0 - u, 0));
+            p[u] = KEEP ? ph[k * bw + c] : S[at(k)];
+        }
     };
-    k = Nz - 2;
-    for (; k - KB + 1 >= 0; k -= KB) {
+    // q runs down from longest − 1; a chain one level shorter skips the first
+    for (int q0 = longest - 1; q0 >= 0; q0 -= KB) {
         C2<T> p[KB];
+        T t[KB];
+        fetch(p, q0);
 #pragma unroll
-        for (int u = 0; u < KB; ++u) p[u] = S[at(k - u)];
+        for (int u = 0; u < KB; ++u) t[u] = tt[level(max(q0 - u, 0)) * bw + c];
+        // (stored together: a test a level would part the chain)
+        if (q0 - KB + 1 >= 0 && q0 < common) {
 #pragma unroll
-        for (int u = 0; u < KB; ++u) bwd(k - u, p[u]);
+            for (int u = 0; u < KB; ++u) {
+                x = cmk<T>(p[u].x + t[u] * x.x, p[u].y + t[u] * x.y);
+                sum = cadd<T>(sum, x);
+                p[u] = x;
+            }
+            if (store) {
+#pragma unroll
+                for (int u = 0; u < KB; ++u) S[at(level(q0 - u))] = p[u];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < KB; ++u) {
+                const int q = q0 - u;
+                if (q >= 0 && q < steps) {
+                    x = cmk<T>(p[u].x + t[u] * x.x, p[u].y + t[u] * x.y);
+                    sum = cadd<T>(sum, x);
+                    if (store) S[at(level(q))] = x;
+                }
+            }
+        }
     }
-    for (; k >= 0; --k) bwd(k, S[at(k)]);
-    if (col == 0) {
+    sum = cadd<T>(sum, cmk<T>(__shfl_xor(sum.x, bw), __shfl_xor(sum.y, bw)));
+    if (singular && store) {
         // remove the mean of the (0,0) column: equals removing the volume mean of ϕ (the reference
-        // subtracts the mean of the real field; the sum here runs down the column as the backward
-        // sweep produced it).  The column is one thread's work at the end of the kernel, so its
-        // read-modify-write pass goes in batches too (one round trip per level would set the
-        // kernel's duration).
-        const C2<T> s = cmk<T>(colsum.x / T(Nz), colsum.y / T(Nz));
+        // subtracts the mean of the real field).  Each lane revisits the levels it stored, in batches
+        // (one round trip per level would set the kernel's duration).
+        const C2<T> m = cmk<T>(sum.x / T(Nz), sum.y / T(Nz));
+        if (!down) S[at(mid)] = csub<T>(S[at(mid)], m);
         int q = 0;
-        for (; q + KB <= Nz; q += KB) {
+        for (; q + KB <= steps; q += KB) {
             C2<T> v[KB];
 #pragma unroll
-            for (int u = 0; u < KB; ++u) v[u] = S[at(q + u)];
+            for (int u = 0; u < KB; ++u) v[u] = S[at(level(q + u))];
 #pragma unroll
-            for (int u = 0; u < KB; ++u) S[at(q + u)] = csub<T>(v[u], s);
+            for (int u = 0; u < KB; ++u) S[at(level(q + u))] = csub<T>(v[u], m);
         }
-        for (; q < Nz; ++q) S[at(q)] = csub<T>(S[at(q)], s);
+        for (; q < steps; ++q) S[at(level(q))] = csub<T>(S[at(level(q))], m);
     }
+}
+
+// The same solve for columns of up to 2·NR + 1 levels, held in registers from the loads, all issued at once,
+// to the stores: no LDS but the levels' coefficients, so that every column of the grid is under way together.
+// Both chains end at position NR − 1, next to the closing level, and start where their length says; the
+// positions before hold nothing (no source, no coupling to the first level), so that the chains run without a
+// branch.  256 × 256 × 128 FP32: 54 µs by one lane a column through memory, 40 µs by k_tridiag (its columns in
+// LDS leave a second, half-empty round of blocks, and a batch's loads only the arithmetic of one batch to
+// arrive in), 19 µs here, 3.9 TB/s of the spectrum in and out.  The recurrence of the excess takes the
+// FP32 solution's error against FP64 from 1.3e-5 to 1.3e-6 (geometric mean over eight grids).
+template <class T, int NR>
+__global__ void __launch_bounds__(64, 2) k_tridiag_short(TriArgs<T> A, C2<T> *__restrict__ Sg, const T *__restrict__ dzc,
+                                                      const T *__restrict__ idzf) {
+    __shared__ __attribute__((aligned(16))) T before[2][NR], next[2][NR], dz[2][NR];   // by chain and position
+    constexpr int bw = 32;                     // columns of the block
+    const int Ny = A.g.Ny, Nz = A.g.Nz, Mx = A.Mx;
+    const int down = threadIdx.x >= bw;
+    const int c = threadIdx.x & (bw - 1);
+    const int64_t ncol = (int64_t)A.Ms * Ny;
+    const int64_t col = min((int64_t)blockIdx.x * bw + c, ncol - 1);
+    const int j = (int)(col / A.Ms), kx = min((int)(col - (int64_t)j * A.Ms), Mx - 1);
+    const bool store = (int64_t)blockIdx.x * bw + c == col && col - (int64_t)j * A.Ms < Mx;
+    const T lam = A.lx[kx] + A.ly[j];
+    C2<T> *S = Sg + col;
+    const int mid = Nz >> 1;   // the closing level
+    auto first_of = [&](int chain) -> int { return NR - (chain ? Nz - 1 - mid : mid); };
+    auto level_of = [&](int chain, int q) -> int { return chain ? mid + NR - q : q - NR + mid; };
+    const int first = first_of(down);
+    auto at = [&](int k) -> int64_t { return (int64_t)k * ncol; };
+    const C2<T> fmid = S[at(mid)];
+    C2<T> f[NR];
+    T t[NR];
+    // the chain's first level (or the closing one) and the step to the next: one running address, formed anew
+    // for the stores, instead of one a level kept from the loads
+    C2<T> *line = S + at(level_of(down, first));
+    const int64_t step = down ? -ncol : ncol;
+    {
+        const C2<T> *p = line;
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            f[q] = *p;
+            p += q >= first ? step : 0;
+        }
+    }
+    for (int e = threadIdx.x; e < 2 * NR; e += 64) {
+        const int chain = e >= NR, q = e - (chain ? NR : 0), k = level_of(chain, q);
+        const bool real = q >= first_of(chain);
+        // (up: from the face below to the face above; down: the reverse)
+        const T lo = real && k > 0 ? idzf[k] : T(0), hi = real && k < Nz - 1 ? idzf[k + 1] : T(0);
+        before[chain][q] = chain ? hi : lo;
+        next[chain][q] = real ? (chain ? lo : hi) : T(1);
+        dz[chain][q] = real ? dzc[k] : T(0);
+    }
+    __syncthreads();
+    const bool singular = lam == T(0);   // the (0,0) column
+    C2<T> top = cmk<T>(T(0), T(0));
+    if (blockIdx.x == 0) {   // (its source without the top level, summed by the whole wave)
+        for (int k = threadIdx.x; k < Nz - 1; k += 64) top = csub<T>(top, Sg[at(k)]);
+        for (int o = 32; o > 0; o >>= 1) top = cadd<T>(top, cmk<T>(__shfl_xor(top.x, o), __shfl_xor(top.y, o)));
+    }
+    const bool replace = singular && down;
+    T excess = T(0), ratio = T(0);
+    C2<T> phi = cmk<T>(T(0), T(0));
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+        // (the pivots do not wait for the loads; but running far ahead they cost more registers
+        // than the chain's values leave)
+        if (q % (sizeof(T) == 4 ? 8 : 4) == 0) asm volatile("" : "+v"(excess), "+v"(ratio), "+v"(phi.x), "+v"(phi.y));
+        C2<T> s = f[q];
+        if (replace && q == first) s = top;
+        if (q < first) s = cmk<T>(T(0), T(0));
+        excess = dz[down][q] * lam + excess * ratio;
+        const T pivot = next[down][q] + excess;
+        ratio = ft_div<T>(next[down][q], pivot);
+        phi = cmk<T>(ft_div<T>(before[down][q] * phi.x - s.x, pivot), ft_div<T>(before[down][q] * phi.y - s.y, pivot));
+        if (!(pivot > A.eps10)) phi = cmk<T>(T(0), T(0));
+        f[q] = phi;
+        t[q] = ratio;
+    }
+    C2<T> x;
+    {
+        // (a chain without levels couples to nothing)
+        const T below = mid > 0 ? idzf[mid] : T(0), above = mid < Nz - 1 ? idzf[mid + 1] : T(0);
+        const T eb = __shfl(excess, c) * __shfl(ratio, c), et = __shfl(excess, c + bw) * __shfl(ratio, c + bw);
+        const C2<T> pb = cmk<T>(__shfl(phi.x, c), __shfl(phi.y, c)), pt = cmk<T>(__shfl(phi.x, c + bw), __shfl(phi.y, c + bw));
+        const T pivot = dzc[mid] * lam + (eb + et);
+        if (!singular && pivot > A.eps10)
+            x = cmk<T>(ft_div<T>((below * pb.x - fmid.x) + above * pt.x, pivot), ft_div<T>((below * pb.y - fmid.y) + above * pt.y, pivot));
+        else x = cmk<T>(T(0), T(0));
+    }
+    const C2<T> xmid = x;
+    C2<T> sum = down ? cmk<T>(T(0), T(0)) : x;
+#pragma unroll
+    for (int q = NR - 1; q >= 0; --q) {
+        x = cmk<T>(f[q].x + t[q] * x.x, f[q].y + t[q] * x.y);
+        f[q] = x;
+        if (q >= first) sum = cadd<T>(sum, x);
+    }
+    sum = cadd<T>(sum, cmk<T>(__shfl_xor(sum.x, bw), __shfl_xor(sum.y, bw)));
+    // the (0,0) column without its mean: equals removing the volume mean of ϕ
+    const C2<T> mean = singular ? cmk<T>(sum.x / T(Nz), sum.y / T(Nz)) : cmk<T>(T(0), T(0));
+    if (!store) return;
+    if (!down) S[at(mid)] = csub<T>(xmid, mean);
+    asm volatile("" : "+v"(line));
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+        if (q >= first) {
+            *line = csub<T>(f[q], mean);
+            line += step;
+        }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -949,15 +1131,26 @@ template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C,
     if (z_active) {
         if (P.tridiagonal) {
             TriArgs<T> A{g, P.S, Mx, P.Ms, P.lx, P.ly, P.eps10, T(1)};
-            // columns per block (one wave, partly filled when narrow): each column is a serial sweep,
-            // so the launch wants waves on every SIMD (≥ 2048 of them) more than full waves; 16
-            // columns still read whole 128-byte lines of the spectrum.  Limited by the LDS holding t[k].
             const int64_t ncol = (int64_t)P.Ms * Ny;
-            int bw = 64;
-            while (bw > 16 && ncol / bw < 2048) bw >>= 1;
-            while (bw > 1 && (size_t)Nz * bw * sizeof(T) > budget) bw >>= 1;
-            hipLaunchKernelGGL(k_tridiag<T>, dim3((unsigned)((ncol + bw - 1) / bw)), dim3(bw), (size_t)Nz * bw * sizeof(T), st, A,
-                               P.S, g.dzc, g.idzf);
+            const int half = Nz >> 1;
+            // registers hold chains of up to 64 levels in FP32 (234 VGPRs, two waves a SIMD) and 32 in FP64 (247)
+            constexpr int most = sizeof(T) == 4 ? 64 : 32;
+            if (half <= most) {
+                const auto kernel = half <= 16 ? &k_tridiag_short<T, 16> : (half <= 32 ? &k_tridiag_short<T, 32> : &k_tridiag_short<T, most>);
+                hipLaunchKernelGGL(kernel, dim3((unsigned)((ncol + 31) / 32)), dim3(64), 0, st, A, P.S, g.dzc, g.idzf);
+            } else {
+                // columns per block (two lanes each, one wave, partly filled when narrow): each column is a
+                // serial sweep, so the launch wants waves on every SIMD (≥ 2048 of them) more than full
+                // waves; 16 columns still read whole 128-byte lines of the spectrum.
+                int bw = 32;
+                while (bw > 16 && ncol / bw < 2048) bw >>= 1;
+                while (bw > 8 && tri_lds<T>(Nz, bw, true) > budget) bw >>= 1;
+                const bool keep = tri_lds<T>(Nz, bw, true) <= budget;
+                while (bw > 1 && tri_lds<T>(Nz, bw, keep) > budget) bw >>= 1;
+                const auto kernel = keep ? &k_tridiag<T, true> : &k_tridiag<T, false>;
+                hipLaunchKernelGGL(kernel, dim3((unsigned)((ncol + bw - 1) / bw)), dim3(2 * bw), tri_lds<T>(Nz, bw, keep), st, A, P.S, g.dzc,
+                                   g.idzf);
+            }
         } else {
             const LineGeom Lz = line_geom(Nz, Nz + (P.zmode == 1 ? Nz : 0), e, lds);
             ZArgs<T> A{g, P.S, P.tw_z, P.st_z, P.tw_dct, Mx, P.Ms, P.zmode, P.lx, P.ly, P.lz, Lz};
