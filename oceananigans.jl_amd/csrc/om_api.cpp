@@ -345,6 +345,8 @@ template <class T> struct ModelT : ModelBase {
         g.kfix = nullptr;
         g.kfix_max = 0;
         g.fix_list = nullptr;
+        g.kbot_wide = nullptr;
+        g.near_xy = nullptr;
         g.fix_count = 0;
         if (c.bottom_height) {
             std::vector<int> kb((size_t)g.Nx * g.Ny, 0);
@@ -363,30 +365,33 @@ template <class T> struct ModelT : ModelBase {
             const int R = kImmersedReach, Nx = g.Nx, Ny = g.Ny;
             std::vector<int> wx(kb.size()), kf(kb.size());
             auto wrap = [](int a, int n) { return ((a % n) + n) % n; };
+            std::vector<int> iw(Nx + 2 * R), jw(Ny + 2 * R);   // wrapped columns
+            for (int i = 0; i < Nx + 2 * R; ++i) iw[i] = wrap(i - R, Nx);
+            for (int j = 0; j < Ny + 2 * R; ++j) jw[j] = wrap(j - R, Ny);
             for (int j = 0; j < Ny; ++j)
                 for (int i = 0; i < Nx; ++i) {
                     int m = 0;
-                    for (int d = -R; d <= R; ++d) m = std::max(m, kb[(size_t)wrap(i + d, Nx) + (size_t)Nx * j]);
+                    for (int d = -R; d <= R; ++d) m = std::max(m, kb[(size_t)iw[i + d + R] + (size_t)Nx * j]);
                     wx[(size_t)i + (size_t)Nx * j] = m;
                 }
             int kfm = 0;
             for (int j = 0; j < Ny; ++j)
                 for (int i = 0; i < Nx; ++i) {
                     int m = 0;
-                    for (int d = -R; d <= R; ++d) m = std::max(m, wx[(size_t)i + (size_t)Nx * wrap(j + d, Ny)]);
+                    for (int d = -R; d <= R; ++d) m = std::max(m, wx[(size_t)i + (size_t)Nx * jw[j + d + R]]);
                     const int f = m > 0 ? std::min(g.Nz, m + R) : 0;
                     kf[(size_t)i + (size_t)Nx * j] = f;
                     kfm = std::max(kfm, f);
                 }
             g.kfix = upload(kf);
             g.kfix_max = kfm;
-            // the fix-up launches' blocks: every (block, level) holding a cell below kfix, level-major
-            const int nbx = (Nx + kGenericBlockX - 1) / kGenericBlockX, nby = (Ny + kGenericBlockY - 1) / kGenericBlockY;
+            // the fix-up launches' work: every (tile, level) holding a cell below kfix, level-major
+            const int nbx = (Nx + kFixX - 1) / kFixX, nby = (Ny + kFixY - 1) / kFixY;
             if (nbx > 0xffff || nby > 0x7fff) throw ArgError{"grid too wide for the immersed fix-up list"};
             std::vector<int> bmax((size_t)nbx * nby, 0);
             for (int j = 0; j < Ny; ++j)
                 for (int i = 0; i < Nx; ++i) {
-                    int &m = bmax[(size_t)(i / kGenericBlockX) + (size_t)nbx * (j / kGenericBlockY)];
+                    int &m = bmax[(size_t)(i / kFixX) + (size_t)nbx * (j / kFixY)];
                     m = std::max(m, kf[(size_t)i + (size_t)Nx * j]);
                 }
             std::vector<int2> fl;
@@ -396,6 +401,30 @@ template <class T> struct ModelT : ModelBase {
                         if (bmax[(size_t)bx + (size_t)nbx * by] > k) fl.push_back(make_int2(bx | (by << 16), k));
             g.fix_count = (int)fl.size();
             if (!fl.empty()) g.fix_list = upload(fl);
+            // the bottom with its margin, and the window maxima of the buffer rules (DevGrid::near_xy)
+            const int M = kBottomMargin, Wx = Nx + 2 * M, Wy = Ny + 2 * M;
+            std::vector<int> ix(Wx + 8), jy(Wy + 8);   // wrapped columns of the table's, with 4 more on either side
+            for (int i = 0; i < Wx + 8; ++i) ix[i] = wrap(i - 4 - M, Nx);
+            for (int j = 0; j < Wy + 8; ++j) jy[j] = wrap(j - 4 - M, Ny);
+            std::vector<int> kw((size_t)Wx * Wy);
+            std::vector<int2> nr((size_t)Wx * Wy * 4);
+            for (int j = 0; j < Wy; ++j)
+                for (int i = 0; i < Wx; ++i) {
+                    const size_t c = (size_t)i + (size_t)Wx * j;
+                    kw[c] = kb[(size_t)ix[i + 4] + (size_t)Nx * jy[j + 4]];
+                    for (int d = 0; d < 2; ++d) {
+                        int a[7], m[7];   // the bottoms of columns −3 … 3 along d; m: of each and its left neighbour, the lower
+                        for (int q = 0; q < 7; ++q) {
+                            a[q] = d == 0 ? kb[(size_t)ix[i + q + 1] + (size_t)Nx * jy[j + 4]] : kb[(size_t)ix[i + 4] + (size_t)Nx * jy[j + q + 1]];
+                            m[q] = q > 0 ? std::min(a[q], a[q - 1]) : 0;
+                        }
+                        const int f2 = std::max(std::max(a[1], a[2]), std::max(a[3], a[4])), c2 = std::max(std::max(m[2], m[3]), std::max(m[4], m[5]));
+                        nr[4 * c + 2 * d] = make_int2(std::max(f2, std::max(a[0], a[5])), f2);
+                        nr[4 * c + 2 * d + 1] = make_int2(std::max(c2, std::max(m[1], m[6])), c2);
+                    }
+                }
+            g.kbot_wide = upload(kw);
+            g.near_xy = upload(nr);
         }
         // physics
         ph.advection = c.advection; ph.closure = c.closure; ph.buoyancy = c.buoyancy; ph.coriolis = c.coriolis;
@@ -635,7 +664,7 @@ template <class T> struct ModelT : ModelBase {
     void pressure_correction(T dtau, bool defer = false) {
         if (g.kbot) {   // mask immersed velocities (pressure_correction.jl:7)
             PhaseScope ps(this, OM_PHASE_HALOS);
-            for (int f = 0; f < 3; ++f) launch_mask(g, s.U[f], f + 1, st);
+            launch_mask_velocities(g, s.U, st);
         }
         if (defer && !cg && !tune_refine && poisson_source_reads_no_halo(ctx()))
             u_halo_pending = true;

@@ -20,6 +20,8 @@ template <class T> struct Vec2;
 template <> struct Vec2<float> { using type = float2; };
 template <> struct Vec2<double> { using type = double2; };
 
+constexpr int kBottomMargin = 8;   // a stencil's farthest lookup of the bottom, in columns, and some
+
 // Grid description passed by value to every kernel.
 template <class T> struct DevGrid {
     int Nx, Ny, Nz;
@@ -34,13 +36,19 @@ template <class T> struct DevGrid {
     int stretched;
     const int *kbot;         // immersed bottom: immersed cells per interior column (x fastest), or nullptr
     int kbot_top;            // the largest entry of kbot: no cell at or above this level is immersed
+    // kbot on columns −kBottomMargin .. N + kBottomMargin − 1 of x and y, repeated periodically, so that a
+    // stencil's lookups need no wrap; and for each of these columns, by direction and point (x faces, x
+    // centres, y faces, y centres), the levels below which an inactive node lies among the 6 (x) and
+    // the 4 (y) stencil points around it along the direction (near_{x,y}_immersed_boundary, IB::near)
+    const int *kbot_wide;
+    const int2 *near_xy;
     // Levels per column (x fastest) on which an immersed-boundary rule can apply to a tendency or
     // closure evaluation (an immersed cell within kImmersedReach cells in x, y and z), 0 where none
     // can; elsewhere the evaluation equals that on the grid without the bottom.  nullptr without one.
     const int *kfix;
     int kfix_max;            // the largest entry of kfix
-    // the (64 × 4-column block, level) pairs of the generic kernels' launch that hold a cell below
-    // kfix: x = block x | block y << 16, y = level; the fix-up launches visit only these
+    // the (16 × 4-column tile, level) pairs that hold a cell below kfix, a wave's work each: x = tile x |
+    // tile y << 16, y = level; the generic kernels' fix-up launches visit only these
     const int2 *fix_list;
     int fix_count;
     // per-level AMD ratios, 5 entries for each k = -1 .. Nz at (k + 1)·5: 2Δx/Δᶠz, Δᶠz/2Δx, 2Δy/Δᶠz,

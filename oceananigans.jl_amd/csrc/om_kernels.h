@@ -267,10 +267,8 @@ template <class T> struct IB {
         }
         return i;
     }
-    __device__ __forceinline__ bool immersed(int i, int j, int k) const {
-        if (!g.kbot || k >= g.kbot_top) return false;   // above the highest bottom: no column lookup
-        return k < g.kbot[wrap(i, g.Nx) + g.Nx * wrap(j, g.Ny)];
-    }
+    __device__ __forceinline__ int column(int i, int j) const { return (i + kBottomMargin) + (g.Nx + 2 * kBottomMargin) * (j + kBottomMargin); }
+    __device__ __forceinline__ bool immersed(int i, int j, int k) const { return g.kbot && k < g.kbot_wide[column(i, j)]; }
     __device__ __forceinline__ bool inactive_cell(int i, int j, int k) const { return immersed(i, j, k) || outside(k); }
     template <int LX, int LY, int LZ> __device__ __forceinline__ bool all_inactive(int i, int j, int k, bool under) const {
         bool r = true;
@@ -303,30 +301,37 @@ template <class T> struct IB {
     template <int LX, int LY, int LZ> __device__ __forceinline__ bool zd(int i1, int j1, int k1, int i2, int j2, int k2) const {
         return on() && (iin<LX, LY, LZ>(i1, j1, k1) || iin<LX, LY, LZ>(i2, j2, k2));
     }
-    // near_{x,y,z}_immersed_boundary for `buffer` (immersed_advective_fluxes.jl:127-215): any inactive
-    // node among the 2·buffer stencil points; cell centres for a face interpolation point (cs = false),
-    // faces along d for a centre interpolation point (cs = true)
-    __device__ __forceinline__ bool near(int d, bool cs, int buffer, int i, int j, int k) const {
-        bool r = false;
-        for (int n = 1; n <= 2 * buffer; ++n) {
-            const int c = cs ? n - buffer : n - buffer - 1;
-            const int ii = i + (d == 0 ? c : 0), jj = j + (d == 1 ? c : 0), kk = k + (d == 2 ? c : 0);
-            bool in = inactive_cell(ii, jj, kk);
-            if (cs) in = in && inactive_cell(ii - (d == 0), jj - (d == 1), kk - (d == 2));
-            r = r || in;
+    // near_{x,y,z}_immersed_boundary (immersed_advective_fluxes.jl:127-215) for buffers 3 (x) and 2 (y): any
+    // inactive node among the 2·buffer stencil points; cell centres for a face interpolation point
+    // (cs = false), faces along d for a centre interpolation point (cs = true).  A column's
+    // inactive levels are those below its bottom and those outside a Bounded z, so along x and y the answer
+    // is a comparison with the window's highest bottom (DevGrid::near_xy; a face is inactive below the
+    // lower of its two bottoms), and along z the window's ends decide.  Looking up every point was most
+    // of what the fix-up launches issued: with the tables (and kFixX's tiles) 487 → 155 µs for the
+    // tendencies and 103 → 41 µs for the closure of the 256 × 256 × 128 seamount.
+    struct Near {
+        bool b3, b2;
+    };
+    __device__ __forceinline__ Near near(int d, bool cs, int i, int j, int k) const {
+        if (d == 2) {
+            const int kb = g.kbot_wide[column(i, j)];
+            auto any = [&](int buffer) { return k - buffer + (cs ? 1 : 0) < kb || (g.tz == OM_BOUNDED && k + buffer - 1 >= g.Nz); };
+            return Near{any(3), any(2)};
         }
-        return r;
+        const int2 m = g.near_xy[4 * (int64_t)column(i, j) + 2 * d + (cs ? 1 : 0)];
+        const bool out = outside(k);
+        return Near{k < m.x || out, k < m.y || out};
     }
     // buffer chain WENO5 (0) → WENO3 (1) → Centered(2) (2); `topo` is the choice without an immersed boundary
     __device__ __forceinline__ int bsch(int d, bool cs, int i, int j, int k, int topo) const {
         if (!on()) return topo;
-        if (!near(d, cs, 3, i, j, k)) return 0;
-        return near(d, cs, 2, i, j, k) ? 2 : 1;
+        const Near n = near(d, cs, i, j, k);
+        return !n.b3 ? 0 : (n.b2 ? 2 : 1);
     }
     // advecting velocity: Centered(4) (true) or Centered(2) (false)
     __device__ __forceinline__ bool s4(int d, bool cs, int i, int j, int k, bool topo) const {
         if (!on()) return topo;
-        return !near(d, cs, 3, i, j, k);
+        return !near(d, cs, i, j, k).b3;
     }
 };
 
@@ -764,6 +769,10 @@ inline int march_tiles(int Nx, int Ny, int ex, int ey) { return ((Nx + ex - 1) /
 // grid, after the tiled kernels have covered the rest
 constexpr int kImmersedReach = 5;   // farthest offset of an immersed-boundary query from its cell, plus one
 constexpr int kGenericBlockX = 64, kGenericBlockY = 4;   // block shape of k_tendencies / k_closure
+// A wave's tile of columns in the fix-up launches.  The cells to redo follow the bottom, so narrow tiles
+// fit them better (256 × 256 × 128 seamount: 81 % of the lanes at work; 53 % with the rows of 64 of a
+// full launch), and 16 FP32 values are still half a line.
+constexpr int kFixX = 16, kFixY = 4;
 template <class T> void launch_tendencies(const Ctx<T> &C, hipStream_t st, bool fixup = false);
 // z-marching tendency kernels: WENO(order=5) (om_tend_tiled.hip) and Centered(order=2) with constant or
 // no diffusivity (om_tend_centered.hip), and the configurations they cover
@@ -781,7 +790,9 @@ template <class T> void launch_rk3(const Ctx<T> &C, T dt, T gamma, T zeta, int f
 // wrap = 1: periodic x and y without an immersed bottom; p's halos are not read
 template <class T> void launch_correct(const Ctx<T> &C, T dtp, int phi, hipStream_t st, int wrap = 0);
 // mask_immersed_field! of a field at location loc (0 ccc, 1 fcc, 2 cfc, 3 ccf) on an immersed grid
+// (launch_mask_velocities: u, v and w at theirs)
 template <class T> void launch_mask(const DevGrid<T> &g, T *f, int loc, hipStream_t st);
+template <class T> void launch_mask_velocities(const DevGrid<T> &g, T *const *U, hipStream_t st);
 // conjugate-gradient Poisson solver kernels (om_cg.hip)
 // Grid-wide reductions of the elementwise kernels use kCgRedBlocks blocks (and partial sums per
 // value).  The 7-point operator sweeps take a 64 × 4 tile of columns and a chunk of kchunk levels

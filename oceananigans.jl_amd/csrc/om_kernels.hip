@@ -16,18 +16,21 @@ namespace om {
 // Tendency kernel: one thread per cell computes Gu, Gv, Gw and every tracer tendency.
 // nonhydrostatic_tendency_kernel_functions.jl:71-302
 // ----------------------------------------------------------------------------------------
-// (fixup: the block's columns and level come from the fix-up list, see DevGrid::fix_list)
+// (fixup: each wave's columns and level come from the fix-up list, see DevGrid::fix_list; consecutive
+// entries go to one XCD, whose L2 holds what neighbouring tiles share)
 template <class T> __device__ __forceinline__ void cell_block(const DevGrid<T> &g, int fixup, int &i, int &j, int &k) {
-    int bx = blockIdx.x, by = blockIdx.y;
-    k = blockIdx.z;
     if (fixup) {
-        const int2 e = g.fix_list[blockIdx.x];
-        bx = e.x & 0xffff;
-        by = e.x >> 16;
+        const int lane = threadIdx.x;
+        const int n = xcd_work_item((int)blockIdx.x, (int)gridDim.x) * kGenericBlockY + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+        const int2 e = g.fix_list[min(n, g.fix_count - 1)];
+        i = n < g.fix_count ? (e.x & 0xffff) * kFixX + (lane & (kFixX - 1)) : g.Nx;
+        j = (e.x >> 16) * kFixY + lane / kFixX;
         k = e.y;
+        return;
     }
-    i = bx * blockDim.x + threadIdx.x;
-    j = by * blockDim.y + threadIdx.y;
+    k = blockIdx.z;
+    i = blockIdx.x * blockDim.x + threadIdx.x;
+    j = blockIdx.y * blockDim.y + threadIdx.y;
 }
 
 template <class T> __global__ void __launch_bounds__(256) k_tendencies(Ctx<T> C, int fixup) {
@@ -846,11 +849,13 @@ template <class T> __device__ __forceinline__ void KCorrect<T>::run(const Correc
 
 // mask_immersed_field! (mask_immersed_field.jl:65-80): zero on the immersed periphery of the
 // field's location over its interior indices (k = 0 .. Nz for w on a Bounded z)
-template <class T> __global__ void __launch_bounds__(256) k_mask(DevGrid<T> g, T *f, int loc, int nk) {
+// (consecutive fields at consecutive locations, nk levels each)
+template <class T> __global__ void __launch_bounds__(256) k_mask(DevGrid<T> g, T *f0, T *f1, T *f2, int loc0, int nk) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int j = blockIdx.y * blockDim.y + threadIdx.y;
-    const int k = blockIdx.z;
-    if (i >= g.Nx || j >= g.Ny || k >= nk) return;
+    const int n = blockIdx.z / nk, k = blockIdx.z - n * nk, loc = loc0 + n;
+    if (i >= g.Nx || j >= g.Ny) return;
+    T *f = n == 0 ? f0 : (n == 1 ? f1 : f2);
     const IB<T> ib(g);
     bool z;
     if (loc == 1) z = ib.template iper<1, 0, 0>(i, j, k);
@@ -876,12 +881,12 @@ static inline dim3 cell_grid(int Nx, int Ny, int Nz, dim3 blk) {
     return dim3((Nx + blk.x - 1) / blk.x, (Ny + blk.y - 1) / blk.y, Nz);
 }
 
-// the generic kernels' block shape; the fix-up list is built for it
-static_assert(kGenericBlockX == 64 && kGenericBlockY == 4, "fix-up list geometry");
+static dim3 fix_grid(int count) { return dim3((count + kGenericBlockY - 1) / kGenericBlockY); }
+static_assert(kGenericBlockX == 64 && kFixX * kFixY == 64, "a wave per row of the block, and per entry of the fix-up list");
 template <class T> void launch_tendencies(const Ctx<T> &C, hipStream_t st, bool fixup) {
     dim3 blk(kGenericBlockX, kGenericBlockY, 1);
     if (fixup) {
-        if (C.g.fix_count > 0) hipLaunchKernelGGL(k_tendencies<T>, dim3(C.g.fix_count), blk, 0, st, C, 1);
+        if (C.g.fix_count > 0) hipLaunchKernelGGL(k_tendencies<T>, fix_grid(C.g.fix_count), blk, 0, st, C, 1);
         return;
     }
     hipLaunchKernelGGL(k_tendencies<T>, cell_grid(C.g.Nx, C.g.Ny, C.g.Nz, blk), blk, 0, st, C, 0);
@@ -889,7 +894,7 @@ template <class T> void launch_tendencies(const Ctx<T> &C, hipStream_t st, bool 
 template <class T> void launch_closure(const Ctx<T> &C, hipStream_t st, bool fixup) {
     dim3 blk(kGenericBlockX, kGenericBlockY, 1);
     if (fixup) {
-        if (C.g.fix_count > 0) hipLaunchKernelGGL(k_closure<T>, dim3(C.g.fix_count), blk, 0, st, C, 1);
+        if (C.g.fix_count > 0) hipLaunchKernelGGL(k_closure<T>, fix_grid(C.g.fix_count), blk, 0, st, C, 1);
         return;
     }
     hipLaunchKernelGGL(k_closure<T>, cell_grid(C.g.Nx, C.g.Ny, C.g.Nz, blk), blk, 0, st, C, 0);
@@ -931,11 +936,19 @@ template <class T> void launch_correct(const Ctx<T> &C, T dtp, int phi, hipStrea
     launch_k<KCorrect<T>>(cell_grid(C.g.Nx, C.g.Ny, (C.g.Nz + kCorrectLevels - 1) / kCorrectLevels, blk), blk, 0, st,
                           CorrectArgs<T>{C, dtp, phi, wrap});
 }
+// levels that hold a masked node: up to the highest immersed cell and its upper face
+template <class T> static int mask_levels(const DevGrid<T> &g) { return std::min(g.kbot_top + 1, g.tz == OM_BOUNDED ? g.Nz + 1 : g.Nz); }
 template <class T> void launch_mask(const DevGrid<T> &g, T *f, int loc, hipStream_t st) {
-    if (!g.kbot) return;
-    const int nk = (loc == 3 && g.tz == OM_BOUNDED) ? g.Nz + 1 : g.Nz;
+    if (!g.kbot || !g.kbot_top) return;
+    const int nk = std::min(mask_levels(g), loc == 3 ? g.Nz + 1 : g.Nz);
     dim3 blk(64, 4, 1);
-    hipLaunchKernelGGL(k_mask<T>, cell_grid(g.Nx, g.Ny, nk, blk), blk, 0, st, g, f, loc, nk);
+    hipLaunchKernelGGL(k_mask<T>, cell_grid(g.Nx, g.Ny, nk, blk), blk, 0, st, g, f, (T *)nullptr, (T *)nullptr, loc, nk);
+}
+template <class T> void launch_mask_velocities(const DevGrid<T> &g, T *const *U, hipStream_t st) {
+    if (!g.kbot || !g.kbot_top) return;
+    const int nk = mask_levels(g);   // (u and v have a halo level above Nz, where nothing is masked)
+    dim3 blk(64, 4, 1);
+    hipLaunchKernelGGL(k_mask<T>, cell_grid(g.Nx, g.Ny, 3 * nk, blk), blk, 0, st, g, U[0], U[1], U[2], 1, nk);
 }
 template <class T> void launch_divergence(const Ctx<T> &C, T *out, hipStream_t st) {
     dim3 blk(64, 4, 1);
@@ -974,6 +987,7 @@ template <class T> void launch_halos(const DevGrid<T> &g, const HaloJob<T> &J, h
     template void launch_rk3<T>(const Ctx<T> &, T, T, T, int, int, hipStream_t);                    \
     template void launch_correct<T>(const Ctx<T> &, T, int, hipStream_t, int);                          \
     template void launch_mask<T>(const DevGrid<T> &, T *, int, hipStream_t);                           \
+    template void launch_mask_velocities<T>(const DevGrid<T> &, T *const *, hipStream_t);              \
     template void launch_divergence<T>(const Ctx<T> &, T *, hipStream_t);                          \
     template void launch_halos<T>(const DevGrid<T> &, const HaloJob<T> &, hipStream_t);
 // Each precision is compiled in its own object: FP64 without FMA contraction (the reference's
