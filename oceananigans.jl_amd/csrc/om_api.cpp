@@ -186,10 +186,12 @@ template <class T> struct ModelT : ModelBase {
     bool cg = false;
     double *cg_r = nullptr, *cg_b = nullptr;       // residual and right-hand side (FP64, padded layout)
     double *cg_x = nullptr, *cg_p = nullptr, *cg_q = nullptr;   // iterate, search direction, A·p (FP64)
+    double *cg_pold = nullptr;                     // the search direction before it
     T *cg_z = nullptr;                             // preconditioned residual (model precision)
     T *cg_t = nullptr;                             // Thomas-sweep ratios of the columnwise preconditioner
     double *diag_partial = nullptr, *diag_out = nullptr, *diag_host = nullptr;   // diagnostics reductions
     double *cg_partial = nullptr, *cg_out = nullptr, *cg_host = nullptr;
+    double *cg_dots = nullptr, *cg_pq = nullptr;   // partial sums of z·r and of the direction sweep
     int cg_iterations = 0;
     double cg_res_last = 0, cg_true_res_last = 0;
     int cg_unconverged = 0;            // solves of the current call that stopped at maxiter above tolerance
@@ -530,8 +532,12 @@ template <class T> struct ModelT : ModelBase {
             cg = true;
             cg_r = field_origin(dalloc<double>(fsize)); cg_b = field_origin(dalloc<double>(fsize));
             cg_x = field_origin(dalloc<double>(fsize)); cg_p = field_origin(dalloc<double>(fsize));
+            cg_pold = field_origin(dalloc<double>(fsize));
             cg_q = field_origin(dalloc<double>(fsize)); cg_z = field_origin(dalloc<T>(fsize));
-            cg_partial = dalloc<double>((size_t)cg_partials_needed(g.Nx, g.Ny, g.Nz));
+            const size_t np = cg_partials_needed(g.Nx, g.Ny, g.Nz);
+            cg_partial = dalloc<double>(3 * np);
+            cg_dots = cg_partial + np;
+            cg_pq = cg_dots + np;
             cg_out = dalloc<double>(kCgSlots);
             if (cg_precond() == OM_PRECOND_COLUMNWISE_TRIDIAGONAL) cg_t = dalloc<T>((size_t)g.Nx * g.Ny * g.Nz);
             if (cg_precond() == OM_PRECOND_LEARNED) {
@@ -709,8 +715,7 @@ template <class T> struct ModelT : ModelBase {
     // zero-mean gauge; x holds the initial guess, cg_b the right-hand side.  ρ, p·Ap and the gauge
     // sums stay on the device (the kernels that use them form α, β and the means); the host reads
     // the norm once per iteration for the convergence test.
-    double cg_read_slot(int slot) {
-        HIPCHECK(hipMemcpyAsync(cg_host, cg_out + slot, sizeof(double), hipMemcpyDeviceToHost, st));
+    double cg_norm2() {   // the gauge sweep's norm, which it leaves in host memory
         HIPCHECK(hipStreamSynchronize(st));
         return cg_host[0];
     }
@@ -851,8 +856,8 @@ template <class T> struct ModelT : ModelBase {
         // with the FFT or learned preconditioner the gauge sweeps also write its source r V⁻¹
         T *const fsrc = (pk == OM_PRECOND_FFT || pk == OM_PRECOND_LEARNED) ? rhs_dense : nullptr;
         // the loop's first VolumeInverseNorm (step 0: no update, so p, q and the scalars are not read)
-        cg_gauge_norm(g, x, cg_p, cg_r, cg_q, cg_out, 0, 0, ncell, fsrc, cg_partial, cg_out + kCgSlotGauge, st);
-        double res = std::sqrt(cg_read_slot(kCgSlotGauge));
+        cg_gauge_norm(g, x, cg_p, cg_r, cg_q, cg_out, cg_pq, 0, 0, ncell, fsrc, cg_partial, cg_out + kCgSlotGauge, cg_host, st);
+        double res = std::sqrt(cg_norm2());
         int64_t it = 0;
         // flexible CG for the learned preconditioner (a nonlinear map): β = zₖ·(rₖ − rₖ₋₁) / (zₖ₋₁·rₖ₋₁);
         // three iterations in a row that do not bring ‖V⁻¹r‖ below 0.999 of its best value so far hand
@@ -890,18 +895,17 @@ template <class T> struct ModelT : ModelBase {
                 }
             } else if (pk == OM_PRECOND_COLUMNWISE_TRIDIAGONAL) cg_ct(g, cg_r, cg_z, cg_t, st);
             else cg_copy_r(g, cg_r, cg_z, st);
-            // ρ (and z·r_prev), p·Ap with Σp and Σq, and the gauge sweep's sums of x and r stay on the
-            // device (kCgSlot*): α, β and the gauge means are formed by the kernels that use them, and
-            // the host reads one norm per iteration
+            // the scalars stay on the device: β, α and the gauge means are formed, from the partial sums
+            // of the launch before, by the kernels that use them, and the host reads one norm per iteration
             const int itp = (int)(it & 1);
-            if (flex && it > 0) cg_dot2(g, cg_z, cg_r, cg_rprev, cg_partial, cg_out + cg_slot_rho(itp), st);
-            else cg_dot_zr(g, cg_z, cg_r, cg_partial, cg_out + cg_slot_rho(itp), st);
-            cg_update_p(g, cg_p, cg_z, cg_out, it == 0 ? 0 : 2 + itp, (flex && it > 0) ? 1 : 0, st);   // with p's halos
+            if (flex && it > 0) cg_dot2(g, cg_z, cg_r, cg_rprev, cg_dots, st);
+            else cg_dot_zr(g, cg_z, cg_r, cg_dots, st);
+            std::swap(cg_p, cg_pold);
+            cg_direction(g, cg_z, cg_pold, cg_p, cg_q, cg_dots, cg_out, 2 + itp, it == 0 ? 1 : 0, (flex && it > 0) ? 1 : 0, cg_pq, st);
             if (flex) cg_copy_d(g, cg_r, cg_rprev, st);
-            cg_apply(g, cg_p, cg_q, cg_partial, cg_out + kCgSlotPQ, st);
             // x += αp, r −= αq, the zero-mean gauge and the norm in one sweep
-            cg_gauge_norm(g, x, cg_p, cg_r, cg_q, cg_out, itp, 1, ncell, fsrc, cg_partial, cg_out + kCgSlotGauge, st);
-            res = std::sqrt(cg_read_slot(kCgSlotGauge));
+            cg_gauge_norm(g, x, cg_p, cg_r, cg_q, cg_out, cg_pq, itp, 1, ncell, fsrc, cg_partial, cg_out + kCgSlotGauge, cg_host, st);
+            res = std::sqrt(cg_norm2());
             it += 1;
             if (!std::isfinite(res)) break;   // reported as not converged; iterating on cannot recover
             // a learned correction that sends the flexible iteration off (‖V⁻¹r‖ a thousand times its

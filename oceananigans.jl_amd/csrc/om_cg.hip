@@ -35,6 +35,33 @@ __device__ __forceinline__ double block_sum(double v) {
     return s;
 }
 
+// Totals over N values' partial sums (value v at v·nper), in every thread of a kRedThreads block.  Each
+// block of a kernel that needs a reduction's result forms it anew, in one order, from the partials of the
+// launch before: a few loads, where a launch of its own would cost 6 µs and a gap.
+template <int N> __device__ __forceinline__ void partial_totals(const double *__restrict__ partial, int nper, double (&total)[N]) {
+    __shared__ double wsum[N][kRedThreads / 64];
+    double acc[N];
+#pragma unroll
+    for (int v = 0; v < N; ++v) acc[v] = 0;
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nper; b += kRedThreads) {
+#pragma unroll
+        for (int v = 0; v < N; ++v) acc[v] += partial[v * nper + b];
+    }
+#pragma unroll
+    for (int v = 0; v < N; ++v) {
+        for (int o = 32; o > 0; o >>= 1) acc[v] += __shfl_down(acc[v], o, 64);
+        if ((threadIdx.x & 63) == 0) wsum[v][threadIdx.x >> 6] = acc[v];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < N; ++v) {
+        total[v] = 0;
+        for (int w = 0; w < kRedThreads / 64; ++w) total[v] += wsum[v][w];
+    }
+    __syncthreads();
+}
+
 // The interior cells one thread visits.  A work unit is a 64-cell segment of one x row, taken by
 // one wave with a cell per lane: the unit's row (j, k) comes from scalar arithmetic and its
 // accesses are contiguous.  The waves of the grid take the units in turn, two per pass, so the
@@ -67,86 +94,64 @@ template <class T> __device__ __forceinline__ double active(const DevGrid<T> &g,
     return IB<T>(g).inactive_cell(i, j, k) ? 0.0 : 1.0;
 }
 
-// The immersed-boundary predicates of the 7-point operator at any level of one column, from the
-// bottom indices of the column and of its four horizontal neighbours, loaded once (the rules of
-// IB::iin, grid_fitted_immersed_boundaries.jl / immersed_boundary_grid.jl).  Without an immersed
-// bottom every index is INT_MIN, which makes every immersed predicate false.
+// The immersed-boundary rules of the 7-point operator at the levels 0 ≤ k < Nz of one column
+// (conditional_differences.jl:15-44 with IB::iin): the ∂ across a face next to an immersed cell vanishes,
+// and the δ of fluxes next to an inactive face, which only an immersed cell has, whose fluxes vanish
+// already.  So each of the six fluxes is zero below a level: the higher bottom of the two columns for
+// x and y, the cell's own bottom for the face above it, and one level more for the face below.  (In a
+// Periodic z the cell below level 0 counts as immersed, as IB::immersed has it.)
 template <class T> struct ColumnMask {
-    int c, xm, xp, ym, yp;
-    int Nz;
-    bool bounded;
-    __device__ __forceinline__ ColumnMask(const DevGrid<T> &g, int i, int j) : Nz(g.Nz), bounded(g.tz == OM_BOUNDED) {
+    int xm, xp, ym, yp, zm, zp;   // the first level with a flux; zp: the first active cell
+    __device__ __forceinline__ ColumnMask(const DevGrid<T> &g, int i, int j) {
         if (g.kbot) {
-            auto kb = [&](int ii, int jj) { return g.kbot[IB<T>::wrap(ii, g.Nx) + g.Nx * IB<T>::wrap(jj, g.Ny)]; };
-            c = kb(i, j);
-            xm = kb(i - 1, j);
-            xp = kb(i + 1, j);
-            ym = kb(i, j - 1);
-            yp = kb(i, j + 1);
+            const IB<T> ib(g);
+            auto kb = [&](int ii, int jj) { return g.kbot_wide[ib.column(ii, jj)]; };
+            zp = kb(i, j);
+            xm = max(zp, kb(i - 1, j));
+            xp = max(zp, kb(i + 1, j));
+            ym = max(zp, kb(i, j - 1));
+            yp = max(zp, kb(i, j + 1));
+            zm = zp > 0 || g.tz != OM_BOUNDED ? zp + 1 : 0;
         } else {
-            c = xm = xp = ym = yp = INT_MIN;
+            xm = xp = ym = yp = zm = zp = 0;
         }
     }
-    // (bitwise & and | throughout: the predicates are cheap and evaluating all of them keeps the
-    // sweep free of branches)
-    __device__ __forceinline__ bool outside(int k) const { return bounded & ((k < 0) | (k >= Nz)); }
-    __device__ __forceinline__ bool inactive(int kb, int k) const { return (k < kb) | outside(k); }
-    // immersed_inactive_node of a cell centre, of the x or y face between two cells, and of the
-    // z face below level k
-    __device__ __forceinline__ bool iin(int kb, int k) const { return inactive(kb, k) & !outside(k); }
-    __device__ __forceinline__ bool iin_face(int ka, int kb, int k) const {
-        return inactive(ka, k) & inactive(kb, k) & !outside(k);
-    }
-    __device__ __forceinline__ bool iin_zface(int k) const {
-        return inactive(c, k) & inactive(c, k - 1) & !(outside(k) & outside(k - 1));
-    }
+    __device__ __forceinline__ bool active(int k) const { return k >= zp; }
 };
 
 // V∇²ᶜᶜᶜ at level k of a column (conjugate_gradient_poisson_solver.jl:62-66) in FP64 from the seven
-// stencil values.  On an immersed grid the inner ∂ vanishes across a face next to an immersed cell
-// and the outer δ next to an immersed inactive face (conditional_differences.jl:15-44).
+// stencil values.  The level's metrics come from restrict-qualified tables, so that a sweep's stores
+// leave them scalar loads: as vector loads, each waited for, they drained a sweep's batches of loads.
 template <class T>
-__device__ __forceinline__ double vlap_col(const DevGrid<T> &g, const ColumnMask<T> &m, int k, double c0, double xm, double xp,
-                                           double ym, double yp, double zm, double zp) {
+__device__ __forceinline__ double vlap_col(const DevGrid<T> &g, const T *__restrict__ dzc, const double *__restrict__ idzf,
+                                           const ColumnMask<T> &m, int k, double c0, double xm, double xp, double ym, double yp,
+                                           double zm, double zp) {
     const double idx = 1.0 / (double)g.dx, idy = 1.0 / (double)g.dy;
-    const double Ax = (double)g.dy * (double)g.dzc[k], Ay = (double)g.dx * (double)g.dzc[k];
+    const double dz = (double)dzc[k], fm = idzf[k], fp = idzf[k + 1];
+    const double Ax = (double)g.dy * dz, Ay = (double)g.dx * dz;
     const double Az = (double)g.dx * (double)g.dy;
-    double gxp = (xp - c0) * idx, gxm = (c0 - xm) * idx;
-    double gyp = (yp - c0) * idy, gym = (c0 - ym) * idy;
+    const double gxp = k < m.xp ? 0.0 : (xp - c0) * idx, gxm = k < m.xm ? 0.0 : (c0 - xm) * idx;
+    const double gyp = k < m.yp ? 0.0 : (yp - c0) * idy, gym = k < m.ym ? 0.0 : (c0 - ym) * idy;
     // 1 / (double)Δzᶠ from the grid's FP64 table: the same correctly rounded quotient as dividing here
-    double gzp = (zp - c0) * g.idzf64[k + 1], gzm = (c0 - zm) * g.idzf64[k];
-    const bool ic = m.iin(m.c, k);
-    gxp = (ic | m.iin(m.xp, k)) ? 0.0 : gxp;
-    gxm = (ic | m.iin(m.xm, k)) ? 0.0 : gxm;
-    gyp = (ic | m.iin(m.yp, k)) ? 0.0 : gyp;
-    gym = (ic | m.iin(m.ym, k)) ? 0.0 : gym;
-    gzp = (ic | m.iin(m.c, k + 1)) ? 0.0 : gzp;
-    gzm = (ic | m.iin(m.c, k - 1)) ? 0.0 : gzm;
-    const bool ox = m.iin_face(m.c, m.xm, k) | m.iin_face(m.xp, m.c, k);
-    const bool oy = m.iin_face(m.c, m.ym, k) | m.iin_face(m.yp, m.c, k);
-    const bool oz = m.iin_zface(k) | m.iin_zface(k + 1);
-    const double tx = ox ? 0.0 : Ax * gxp - Ax * gxm;
-    const double ty = oy ? 0.0 : Ay * gyp - Ay * gym;
-    const double tz = oz ? 0.0 : Az * gzp - Az * gzm;
-    return (tx + ty) + tz;
+    const double gzp = k < m.zp ? 0.0 : (zp - c0) * fp, gzm = k < m.zm ? 0.0 : (c0 - zm) * fm;
+    return ((Ax * gxp - Ax * gxm) + (Ay * gyp - Ay * gym)) + (Az * gzp - Az * gzm);
 }
 
 // ---------------------------------------------------------------------------------------------
 // Sweeps of the 7-point operator.  A block takes a 64 × 4 tile of columns and a chunk of levels
 // (cg_stencil_shape); each thread marches up its column with the values at k − 1, k and k + 1 in
 // registers, so a level costs five loads (the level above and the four horizontal neighbours),
-// and the immersed-boundary rules use the five bottom indices of ColumnMask.  Blocks are dealt to
+// and the immersed-boundary rules are six comparisons (ColumnMask).  Blocks are dealt to
 // the XCDs in contiguous runs of work items (xcd_work_item), the chunks of one tile consecutive.
-//   STENCIL_APPLY     q = V∇²p; partial sums of p·q, Σp and Σq
 //   STENCIL_RESIDUAL  r = b − V∇²x, through the initial VolumeInverseNorm; partial sums of (r V⁻¹)²
 //   STENCIL_TRUE      e = b − V∇²x; partial sums of e
 //   STENCIL_ENERGY    partial sums of −d·V∇²d and, when gout is given, gout = −2·s·active·V∇²d
 // ---------------------------------------------------------------------------------------------
-enum { STENCIL_APPLY = 0, STENCIL_RESIDUAL = 1, STENCIL_TRUE = 2, STENCIL_ENERGY = 3 };
+enum { STENCIL_RESIDUAL = 1, STENCIL_TRUE = 2, STENCIL_ENERGY = 3 };
 
 template <class T, int MODE>
 __global__ void __launch_bounds__(kCgStTx * kCgStTy)
-    k_cg_stencil(DevGrid<T> g, const double *__restrict__ src, const double *__restrict__ b, double *__restrict__ out,
+    k_cg_stencil(DevGrid<T> g, const T *__restrict__ dzc, const double *__restrict__ idzf, const double *__restrict__ src, const double *__restrict__ b, double *__restrict__ out,
                  float *__restrict__ gout, double gscale, double *__restrict__ partial, int kchunk, int ntx) {
     const int a = threadIdx.x & (kCgStTx - 1), c = threadIdx.x / kCgStTx;
     const int item = xcd_work_item((int)blockIdx.x, (int)gridDim.x);
@@ -155,23 +160,19 @@ __global__ void __launch_bounds__(kCgStTx * kCgStTy)
     const int ty = tile / ntx, tx = tile - ty * ntx;
     const int i = tx * kCgStTx + a, j = ty * kCgStTy + c;
     const int k0 = chunk * kchunk, k1 = min(k0 + kchunk, g.Nz);
-    double acc = 0, accp = 0, accq = 0;   // (STENCIL_APPLY: p·q, Σp, Σq)
+    double acc = 0;
     if (i < g.Nx && j < g.Ny) {
         const ColumnMask<T> m(g, i, j);
         const int64_t col = idx3(i, j, 0, g.sy, g.sz), sy = g.sy, sz = g.sz;
         const double *s = src + col;
         auto emit = [&](int k, double c0, double v) {
             const int64_t o = col + (int64_t)k * sz;
-            if (MODE == STENCIL_APPLY) {
-                out[o] = v;
-                acc += c0 * v;
-                accp += c0;
-                accq += v;
-            } else if (MODE == STENCIL_RESIDUAL) {
+            if (MODE == STENCIL_RESIDUAL) {
                 const double rv = b[o] - v;
-                const double rs = rv * (double)(T(1) / vol(g, k));
+                const T V = g.Az * dzc[k];
+                const double rs = rv * (double)(T(1) / V);
                 acc += rs * rs;
-                out[o] = rs * (double)vol(g, k);
+                out[o] = rs * (double)V;
             } else if (MODE == STENCIL_TRUE) {
                 const double e = b[o] - v;
                 out[o] = e;
@@ -179,7 +180,7 @@ __global__ void __launch_bounds__(kCgStTx * kCgStTy)
             } else {
                 acc -= c0 * v;
                 if (gout) {
-                    const double act = m.inactive(m.c, k) ? 0.0 : 1.0;
+                    const double act = m.active(k) ? 1.0 : 0.0;
                     gout[(int64_t)i + (int64_t)g.Nx * ((int64_t)j + (int64_t)g.Ny * k)] = (float)(-2.0 * gscale * act * v);
                 }
             }
@@ -198,7 +199,7 @@ __global__ void __launch_bounds__(kCgStTx * kCgStTy)
             }
 #pragma unroll
             for (int u = 0; u < kCgStBatch; ++u) {
-                const double v = vlap_col(g, m, k + u, c0, xm[u], xp[u], ym[u], yp[u], zm, zc[u]);
+                const double v = vlap_col(g, dzc, idzf, m, k + u, c0, xm[u], xp[u], ym[u], yp[u], zm, zc[u]);
                 emit(k + u, c0, v);
                 zm = c0;
                 c0 = zc[u];
@@ -207,22 +208,150 @@ __global__ void __launch_bounds__(kCgStTx * kCgStTy)
         for (; k < k1; ++k) {
             const int64_t o = (int64_t)k * sz;
             const double zp = s[o + sz];
-            const double v = vlap_col(g, m, k, c0, s[o - 1], s[o + 1], s[o - sy], s[o + sy], zm, zp);
+            const double v = vlap_col(g, dzc, idzf, m, k, c0, s[o - 1], s[o + 1], s[o - sy], s[o + sy], zm, zp);
             emit(k, c0, v);
             zm = c0;
             c0 = zp;
         }
     }
     const double sum = block_sum(acc);
-    if (MODE == STENCIL_APPLY) {
-        const double sp = block_sum(accp), sq = block_sum(accq);
-        if (threadIdx.x == 0) {
-            partial[blockIdx.x] = sum;
-            partial[gridDim.x + blockIdx.x] = sp;
-            partial[2 * gridDim.x + blockIdx.x] = sq;
+    if (threadIdx.x == 0) partial[blockIdx.x] = sum;
+}
+
+// The search direction and its image in one sweep: p = z (FIRST) or p = z + β p_old, q = V∇²p,
+// partial sums of p·q, Σp and Σq.  ρ = z·r (and z·r_prev for the flexible form) comes from the dot's
+// partial sums, β = ρ / ρ_prev or (ρ − z·r_prev) / ρ_prev; block 0 keeps ρ in the iteration's slot
+// (cg_slot_rho; `it` is any number of the iteration's parity).
+// HBM bounds it, so p is formed from z and p_old where the operator needs it instead of being stored by
+// one sweep and read by the next: 236 instead of 302 MB at 256 × 256 × 128 in FP32.  A block marches up a
+// 64 × 8 tile of columns (two rows a thread, cg_direction_shape's chunk of levels) with a level of p
+// and its one-cell rim in LDS, alternating between two buffers so that a level costs one barrier; the
+// loads of kCgStBatch levels are issued while the batch before them is worked on.  256 × 256 × 128 FP32: 55 µs,
+// 4.3 TB/s, where the two sweeps took 35 and 49.  (62 µs with the prefetch under a condition, 77 with the
+// levels' metrics as vector loads besides.)
+// Neighbours across the domain's edges are read by wrapped index (x, y; z by its topology, the
+// one-layer copy of a Bounded z being the cell itself), so p has no halos.  p_old is another buffer than p.
+template <class T, bool FIRST>
+__global__ void __launch_bounds__(kRedThreads)
+    k_cg_direction(DevGrid<T> g, const T *__restrict__ dzc, const double *__restrict__ idzf, const T *__restrict__ z, const double *__restrict__ pold, double *__restrict__ p,
+                   double *__restrict__ q, const double *__restrict__ dots, double *__restrict__ sc, int it, int flex,
+                   double *__restrict__ partial, int kchunk, int ntx) {
+    constexpr int TX = kCgDirX, TY = kCgDirY, U = kCgStBatch;
+    static_assert(TX == 64 && TY == 8 && kRedThreads == 256, "two rows of 64 a wave; the rim is one element a thread");
+    __shared__ double tile[2][TY + 2][TX + 2];
+    const int a = threadIdx.x & (TX - 1), c = threadIdx.x / TX;
+    const int item = xcd_work_item((int)blockIdx.x, (int)gridDim.x);
+    const int nch = (g.Nz + kchunk - 1) / kchunk;
+    const int column = item / nch, chunk = item - column * nch;
+    const int ty = column / ntx, tx = column - ty * ntx;
+    const int i0 = tx * TX, j0 = ty * TY;
+    const int k0 = chunk * kchunk, k1 = min(k0 + kchunk, g.Nz);
+    // element offsets within a level (a scalar level origin is added; 8 bytes each, a level under 4 GB) by position in the tile; what lies past the
+    // domain's edge reads the wrapped cell (or, further on, one that nobody uses)
+    auto offset = [&](int x, int y) -> uint32_t {
+        const int i = i0 + x, j = j0 + y;
+        const int iw = i < 0 ? g.Nx - 1 : (i >= g.Nx ? 0 : i), jw = j < 0 ? g.Ny - 1 : (j >= g.Ny ? 0 : j);
+        return (uint32_t)jw * (uint32_t)g.sy + (uint32_t)iw;
+    };
+    const uint32_t own0 = offset(a, c), own1 = offset(a, c + TY / 2);
+    // the rim: rows −1 and TY, then columns −1 and TX
+    const int e = threadIdx.x;
+    const bool rim = e < 2 * TX + 2 * TY;
+    const int rx = e < 2 * TX ? a : (e < 2 * TX + TY ? -1 : TX);
+    const int ry = e < 2 * TX ? (e < TX ? -1 : TY) : (e - 2 * TX) & (TY - 1);
+    const uint32_t orim = rim ? offset(rx, ry) : own0;   // (no load is predicated)
+    struct Pair {
+        T z;
+        double p;
+    };
+    struct Level {
+        Pair up0, up1, rim;   // the thread's columns one level up, and its share of the rim
+    };
+    auto load = [&](int k, uint32_t o) -> Pair {
+        const T *zk = z + (int64_t)k * g.sz;
+        const double *pk = pold + (int64_t)k * g.sz;
+        Pair v{*reinterpret_cast<const T *>(reinterpret_cast<const char *>(zk) + o * (uint32_t)sizeof(T)), 0.0};
+        if (!FIRST) v.p = *reinterpret_cast<const double *>(reinterpret_cast<const char *>(pk) + o * 8u);
+        return v;
+    };
+    const bool zper = g.tz == OM_PERIODIC;
+    auto above = [&](int k) -> int { return k < g.Nz - 1 ? k + 1 : (zper ? 0 : g.Nz - 1); };
+    auto fetch = [&](Level (&v)[U], int k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kk = min(k + u, k1 - 1), ka = above(kk);
+            v[u].up0 = load(ka, own0);
+            v[u].up1 = load(ka, own1);
+            v[u].rim = load(kk, orim);
         }
-    } else if (threadIdx.x == 0) {
+        __builtin_amdgcn_sched_barrier(0);   // (all issued before what follows)
+    };
+    const int kb = k0 > 0 ? k0 - 1 : (zper ? g.Nz - 1 : 0);
+    const Pair m0 = load(kb, own0), m1 = load(kb, own1), s0 = load(k0, own0), s1 = load(k0, own1);
+    Level now[U];
+    fetch(now, k0);
+
+    double beta = 0.0;
+    if (!FIRST || blockIdx.x == 0) {
+        double rho[2] = {0, 0};
+        if (flex) partial_totals<2>(dots, kRedBlocks, rho);
+        else {
+            double one[1];
+            partial_totals<1>(dots, kRedBlocks, one);
+            rho[0] = one[0];
+        }
+        if (!FIRST) {
+            const double prev = sc[cg_slot_rho(it - 1)];
+            beta = flex ? (rho[0] - rho[1]) / prev : rho[0] / prev;
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) sc[cg_slot_rho(it)] = rho[0];
+    }
+    auto dir = [&](const Pair &v) -> double { return FIRST ? (double)v.z : (double)v.z + beta * v.p; };
+
+    const int i = i0 + a, ja = j0 + c, jb = ja + TY / 2;
+    const bool in0 = i < g.Nx && ja < g.Ny, in1 = i < g.Nx && jb < g.Ny;
+    const ColumnMask<T> mask0(g, in0 ? i : 0, in0 ? ja : 0), mask1(g, in1 ? i : 0, in1 ? jb : 0);
+    double acc = 0, accp = 0, accq = 0;
+    double zm0 = dir(m0), zm1 = dir(m1), c0 = dir(s0), c1 = dir(s1);
+    for (int k = k0; k < k1; k += U) {
+        Level next[U];
+        fetch(next, k + U);   // (also beyond the end, repeating a level: where a branch could have left these loads
+                              // out, the waits for the batch at hand would wait for them)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kk = k + u;
+            if (kk < k1) {
+                double (&P)[TY + 2][TX + 2] = tile[kk & 1];
+                P[c + 1][a + 1] = c0;
+                P[c + TY / 2 + 1][a + 1] = c1;
+                if (rim) P[ry + 1][rx + 1] = dir(now[u].rim);
+                __syncthreads();   // (a level later this buffer's readers are done: they have passed the next barrier)
+                auto emit = [&](bool in, const ColumnMask<T> &m, int y, uint32_t o, double &zm, double &cc, const Pair &up) {
+                    const double zp = dir(up);
+                    if (in) {
+                        const double v = vlap_col(g, dzc, idzf, m, kk, cc, P[y + 1][a], P[y + 1][a + 2], P[y][a + 1], P[y + 2][a + 1], zm, zp);
+                        char *pk = reinterpret_cast<char *>(p + (int64_t)kk * g.sz), *qk = reinterpret_cast<char *>(q + (int64_t)kk * g.sz);
+                        *reinterpret_cast<double *>(pk + o * 8u) = cc;
+                        *reinterpret_cast<double *>(qk + o * 8u) = v;
+                        acc += cc * v;
+                        accp += cc;
+                        accq += v;
+                    }
+                    zm = cc;
+                    cc = zp;
+                };
+                emit(in0, mask0, c, own0, zm0, c0, now[u].up0);
+                emit(in1, mask1, c + TY / 2, own1, zm1, c1, now[u].up1);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) now[u] = next[u];
+    }
+    const double sum = block_sum(acc), sp = block_sum(accp), sq = block_sum(accq);
+    if (threadIdx.x == 0) {
         partial[blockIdx.x] = sum;
+        partial[gridDim.x + blockIdx.x] = sp;
+        partial[2 * gridDim.x + blockIdx.x] = sq;
     }
 }
 
@@ -246,15 +375,57 @@ template <class T> __global__ void __launch_bounds__(256) k_cg_xio(DevGrid<T> g,
 
 // b = active · divᶜᶜᶜ(U) · V (solve_for_pressure.jl:44-50), or b = rhs · V for a given dense rhs
 // (solve!(x, ::ConjugateGradientPoissonSolver, b) takes the caller's right-hand side as it is)
+// A thread takes kSourceLevels levels of one column of a 64 × 4 tile, all loads first; the conditional
+// δ of the divergence (Ctx::divU) vanishes below a level for each axis: between two faces one of which
+// is inactive, i.e. below the lower of its two columns' bottoms, and within an immersed cell.
+// (128 → 32 µs for the 256 × 256 × 128 seamount: 167 MB at 5.2 TB/s.)
+constexpr int kSourceLevels = 8;
 template <class T> __global__ void __launch_bounds__(256) k_cg_source(Ctx<T> C, const T *__restrict__ dense_rhs, double *__restrict__ b) {
     const DevGrid<T> &g = C.g;
-    for_cells(g, [&](int i, int j, int k, int64_t o, int64_t t) {
-        T d;
-        if (dense_rhs) d = dense_rhs[t];
-        else d = C.divU(i, j, k, i + 1, j + 1);
-        const T act = (!dense_rhs && IB<T>(g).inactive_cell(i, j, k)) ? T(0) : T(1);
-        b[o] = (double)((act * d) * vol(g, k));
-    });
+    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, k0 = blockIdx.z * kSourceLevels;
+    if (i >= g.Nx || j >= g.Ny) return;
+    int bottom = 0, bx = 0, by = 0;
+    if (g.kbot && !dense_rhs) {
+        const IB<T> ib(g);
+        auto kb = [&](int ii, int jj) { return g.kbot_wide[ib.column(ii, jj)]; };
+        bottom = kb(i, j);
+        bx = min(bottom, max(kb(i - 1, j), kb(i + 1, j)));
+        by = min(bottom, max(kb(i, j - 1), kb(i, j + 1)));
+    }
+    const int64_t o = idx3(i, j, 0, g.sy, g.sz);
+    const T *__restrict__ u = C.s.U[0] + o, *__restrict__ v = C.s.U[1] + o, *__restrict__ w = C.s.U[2] + o;
+    T d[kSourceLevels];
+    if (dense_rhs) {
+#pragma unroll
+        for (int q = 0; q < kSourceLevels; ++q)
+            d[q] = dense_rhs[(int64_t)i + (int64_t)g.Nx * (j + (int64_t)g.Ny * min(k0 + q, g.Nz - 1))];
+    } else {
+        T u0[kSourceLevels], u1[kSourceLevels], v0[kSourceLevels], v1[kSourceLevels], ww[kSourceLevels + 1];
+#pragma unroll
+        for (int q = 0; q < kSourceLevels; ++q) {
+            const int64_t level = (int64_t)min(k0 + q, g.Nz - 1) * g.sz;
+            u0[q] = u[level]; u1[q] = u[level + 1];
+            v0[q] = v[level]; v1[q] = v[level + g.sy];
+            ww[q] = w[level];
+        }
+        ww[kSourceLevels] = w[(int64_t)min(k0 + kSourceLevels, g.Nz) * g.sz];
+        // (the face above the topmost level, where the chunk ends before its batch)
+        const T top = w[(int64_t)g.Nz * g.sz];
+#pragma unroll
+        for (int q = 0; q < kSourceLevels; ++q) {
+            const int k = min(k0 + q, g.Nz - 1);
+            const T w1 = k == g.Nz - 1 ? top : ww[q + 1];
+            const T sx = C.flx() || k < bx ? T(0) : C.Axc(k) * u1[q] - C.Axc(k) * u0[q];
+            const T sy = C.fly() || k < by ? T(0) : C.Ayc(k) * v1[q] - C.Ayc(k) * v0[q];
+            const T sz = C.flz() || k < bottom ? T(0) : g.Az * w1 - g.Az * ww[q];
+            d[q] = C.iVc(k) * ((sx + sy) + sz);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kSourceLevels; ++q) {
+        const int k = k0 + q;
+        if (k < g.Nz) b[o + (int64_t)k * g.sz] = (double)(((k < bottom ? T(0) : T(1)) * d[q]) * vol(g, k));
+    }
 }
 
 // DiagonallyDominantPreconditioner (conjugate_gradient_poisson_solver.jl:256-296); r has its halos
@@ -345,35 +516,6 @@ template <class T> __global__ void __launch_bounds__(256) k_cg_dot_zr(DevGrid<T>
     if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
-// p = z (first iteration, it = 0) or p = z + β p with β = ρ / ρ_prev, or the flexible form
-// β = (ρ − z·r_prev) / ρ_prev, from the iteration's scalars on the device (cg_slot_rho); `it` is the
-// iteration index or any number of its parity that is nonzero after the first iteration.  The
-// cells next to the domain's faces also write p's one-layer halos (the fill of cg_halo_r: periodic
-// x and y, z by its topology), which the operator sweep that follows reads.
-template <class T>
-__global__ void __launch_bounds__(256) k_cg_update_p(DevGrid<T> g, double *__restrict__ p, const T *__restrict__ z,
-                                                     const double *__restrict__ sc, int it, int flex) {
-    const int first = it == 0;
-    double beta = 0.0;
-    if (!first) {
-        const double rho = sc[cg_slot_rho(it)], prev = sc[cg_slot_rho(it - 1)];
-        beta = flex ? (rho - sc[cg_slot_rho(it) + 1]) / prev : rho / prev;
-    }
-    const int64_t xs = g.Nx, ys = (int64_t)g.Ny * g.sy, zs = (int64_t)g.Nz * g.sz;
-    const bool zper = g.tz == OM_PERIODIC;
-    for_cells(g, [&](int i, int j, int k, int64_t o, int64_t t) {
-        const double pv = first ? (double)z[o] : (double)z[o] + beta * p[o];
-        p[o] = pv;
-        if (i == 0) p[o + xs] = pv;
-        if (i == g.Nx - 1) p[o - xs] = pv;
-        if (j == 0) p[o + ys] = pv;
-        if (j == g.Ny - 1) p[o - ys] = pv;
-        if (k == 0) p[zper ? o + zs : o - g.sz] = pv;
-        if (k == g.Nz - 1) p[zper ? o - zs : o + g.sz] = pv;
-    });
-}
-
-
 // The gauge and norm sweep (conjugate_gradient_poisson_solver.jl:87-96, then the VolumeInverseNorm
 // of :13-34): x ← (x − mean x)·active, r ← (r − mean r)·active, partial sums of (r V⁻¹)², and of the
 // new x and r (the next iteration's means start from them).  With `dense`, the FFT preconditioner's
@@ -381,19 +523,22 @@ __global__ void __launch_bounds__(256) k_cg_update_p(DevGrid<T> g, double *__res
 //   step = false: the solve's first sweep, means 0 (no update);
 //   step = true:  the iteration's update x += α p, r −= α q comes first, α = ρ / p·Ap, and the means
 //                 of the updated x and r come from sums taken before it: Σx + α Σp and Σr − α Σq
-//                 (Σx, Σr from the previous sweep, Σp, Σq from the operator sweep).  This is the
+//                 (Σx, Σr from the previous sweep; p·q, Σp, Σq from the direction sweep's `pq` partial
+//                 sums, npq of each).  This is the
 //                 same mean the reference takes after the update, summed in another order, so
 //                 the update and the gauge share one pass over x, p, r and q.
 template <class T>
 __global__ void __launch_bounds__(256) k_cg_gauge_norm(DevGrid<T> g, double *__restrict__ x, const double *__restrict__ p,
                                                        double *__restrict__ r, const double *__restrict__ q,
-                                                       const double *__restrict__ sc, int it, int step, double ncell,
-                                                       T *__restrict__ dense, double *partial) {
+                                                       const double *__restrict__ sc, const double *__restrict__ pq, int npq, int it,
+                                                       int step, double ncell, T *__restrict__ dense, double *partial) {
     double alpha = 0.0, mx = 0.0, mr = 0.0;
     if (step) {
-        alpha = sc[cg_slot_rho(it)] / sc[kCgSlotPQ];
-        mx = (sc[kCgSlotGauge + 1] + alpha * sc[kCgSlotPQ + 1]) / ncell;
-        mr = (sc[kCgSlotGauge + 2] - alpha * sc[kCgSlotPQ + 2]) / ncell;
+        double s[3];
+        partial_totals<3>(pq, npq, s);
+        alpha = sc[cg_slot_rho(it)] / s[0];
+        mx = (sc[kCgSlotGauge + 1] + alpha * s[1]) / ncell;
+        mr = (sc[kCgSlotGauge + 2] - alpha * s[2]) / ncell;
     }
     double acc = 0, sx = 0, sr = 0;
     for_cells(g, [&](int i, int j, int k, int64_t o, int64_t t) {
@@ -536,13 +681,23 @@ template <class T> __global__ void __launch_bounds__(256) k_ln_err(DevGrid<T> g,
     });
 }
 
-// out[v] = Σ partial[v·nper + b] over b < nper, in a fixed order
-static __global__ void __launch_bounds__(kRedThreads) k_cg_finish(const double *partial, int nvals, int nper, double *out) {
-    for (int v = 0; v < nvals; ++v) {
-        double acc = 0;
-        for (int b = threadIdx.x; b < nper; b += kRedThreads) acc += partial[v * nper + b];
-        const double s = block_sum(acc);
+// out[v] = Σ partial[v·nper + b] over b < nper, v < nvals ≤ 3, in a fixed order (the values' loads
+// together: one block's latency bounds it).  host (or null): the first value also goes to host memory,
+// which spares the host's read a copy.
+static __global__ void __launch_bounds__(kRedThreads) k_cg_finish(const double *__restrict__ partial, int nvals, int nper,
+                                                                  double *__restrict__ out, double *__restrict__ host) {
+    double acc[3] = {0, 0, 0};
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nper; b += kRedThreads) {
+#pragma unroll
+        for (int v = 0; v < 3; ++v) acc[v] += v < nvals ? partial[v * nper + b] : 0.0;
+    }
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+        if (v == nvals) break;
+        const double s = block_sum(acc[v]);
         if (threadIdx.x == 0) out[v] = s;
+        if (host && v == 0 && threadIdx.x == 0) *host = s;
     }
 }
 
@@ -586,10 +741,9 @@ template <class T, int MODE>
 static void cg_stencil(const DevGrid<T> &g, const double *src, const double *b, double *out, float *gout, double gscale,
                        double *partial, double *outv, hipStream_t st) {
     const CgStencilShape s = cg_stencil_shape(g.Nx, g.Ny, g.Nz);
-    hipLaunchKernelGGL((k_cg_stencil<T, MODE>), dim3(s.nblocks), dim3(kCgStTx * kCgStTy), 0, st, g, src, b, out, gout, gscale,
+    hipLaunchKernelGGL((k_cg_stencil<T, MODE>), dim3(s.nblocks), dim3(kCgStTx * kCgStTy), 0, st, g, g.dzc, g.idzf64, src, b, out, gout, gscale,
                        partial, s.kchunk, s.ntx);
-    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, MODE == STENCIL_APPLY ? 3 : 1, s.nblocks,
-                       outv);
+    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 1, s.nblocks, outv, (double *)nullptr);
 }
 
 template <class T> void cg_scale(const DevGrid<T> &g, T *f, T s, int mode, hipStream_t st) {
@@ -602,7 +756,8 @@ template <class T> void cg_xio(const DevGrid<T> &g, T *f, double *x, T s, int st
     hipLaunchKernelGGL(k_cg_xio<T>, red_grid(), red_blk(), 0, st, g, f, x, s, store);
 }
 template <class T> void cg_source(const Ctx<T> &C, const T *dense_rhs, double *b, hipStream_t st) {
-    hipLaunchKernelGGL(k_cg_source<T>, red_grid(), red_blk(), 0, st, C, dense_rhs, b);
+    const dim3 grid((C.g.Nx + 63) / 64, (C.g.Ny + 3) / 4, (C.g.Nz + kSourceLevels - 1) / kSourceLevels);
+    hipLaunchKernelGGL(k_cg_source<T>, grid, dim3(64, 4), 0, st, C, dense_rhs, b);
 }
 template <class T> void cg_residual(const DevGrid<T> &g, const double *x, const double *b, double *r, double *partial, double *out,
                                     hipStream_t st) {
@@ -623,7 +778,7 @@ template <class T> void cg_ct(const DevGrid<T> &g, const double *r, T *z, T *t, 
 }
 template <class T> void ln_scales(const DevGrid<T> &g, const double *r, const T *z, double *partial, double *out, hipStream_t st) {
     hipLaunchKernelGGL(k_ln_scales<T>, red_grid(), red_blk(), 0, st, g, r, z, partial);
-    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 3, kRedBlocks, out);
+    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 3, kRedBlocks, out, (double *)nullptr);
 }
 template <class T> void ln_input(const DevGrid<T> &g, const double *r, const T *z, double isr, double isz, float *in3, hipStream_t st) {
     hipLaunchKernelGGL(k_ln_input<T>, red_grid(), red_blk(), 0, st, g, r, z, isr, isz, in3);
@@ -637,15 +792,13 @@ template <class T> void ln_correct(const DevGrid<T> &g, T *z, const float *out, 
 template <class T> void cg_copy_d(const DevGrid<T> &g, const double *src, double *dst, hipStream_t st) {
     hipLaunchKernelGGL(k_cg_copy_d<T>, red_grid(), red_blk(), 0, st, g, src, dst);
 }
-template <class T> void cg_dot2(const DevGrid<T> &g, const T *z, const double *r, const double *rp, double *partial, double *out,
-                                hipStream_t st) {
+template <class T> void cg_dot2(const DevGrid<T> &g, const T *z, const double *r, const double *rp, double *partial, hipStream_t st) {
     hipLaunchKernelGGL(k_cg_dot2<T>, red_grid(), red_blk(), 0, st, g, z, r, rp, partial);
-    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 2, kRedBlocks, out);
 }
 template <class T> void ln_target(const DevGrid<T> &g, const double *xf, const double *xk, const float *in3k, double isz, float *tgt,
                                   double *partial, double *out, hipStream_t st) {
     hipLaunchKernelGGL(k_ln_target<T>, red_grid(), red_blk(), 0, st, g, xf, xk, in3k, isz, tgt, partial);
-    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 2, kRedBlocks, out);
+    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 2, kRedBlocks, out, (double *)nullptr);
 }
 template <class T> void ln_center(const DevGrid<T> &g, float *tgt, float mean, hipStream_t st) {
     hipLaunchKernelGGL(k_ln_center<T>, red_grid(), red_blk(), 0, st, g, tgt, mean);
@@ -662,21 +815,22 @@ template <class T> void ln_mask(const DevGrid<T> &g, float *mask, hipStream_t st
 template <class T> void cg_copy_r(const DevGrid<T> &g, const double *r, T *z, hipStream_t st) {
     hipLaunchKernelGGL(k_cg_copy_r<T>, red_grid(), red_blk(), 0, st, g, r, z);
 }
-template <class T> void cg_dot_zr(const DevGrid<T> &g, const T *z, const double *r, double *partial, double *out, hipStream_t st) {
+template <class T> void cg_dot_zr(const DevGrid<T> &g, const T *z, const double *r, double *partial, hipStream_t st) {
     hipLaunchKernelGGL(k_cg_dot_zr<T>, red_grid(), red_blk(), 0, st, g, z, r, partial);
-    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 1, kRedBlocks, out);
 }
-template <class T> void cg_update_p(const DevGrid<T> &g, double *p, const T *z, const double *sc, int it, int flex, hipStream_t st) {
-    hipLaunchKernelGGL(k_cg_update_p<T>, red_grid(), red_blk(), 0, st, g, p, z, sc, it, flex);
-}
-template <class T> void cg_apply(const DevGrid<T> &g, const double *p, double *q, double *partial, double *out, hipStream_t st) {
-    cg_stencil<T, STENCIL_APPLY>(g, p, (const double *)nullptr, q, (float *)nullptr, 0.0, partial, out, st);
+template <class T> void cg_direction(const DevGrid<T> &g, const T *z, const double *pold, double *p, double *q, const double *dots,
+                                     double *sc, int it, int first, int flex, double *partial, hipStream_t st) {
+    const CgStencilShape s = cg_direction_shape(g.Nx, g.Ny, g.Nz);
+    const auto kernel = first ? &k_cg_direction<T, true> : &k_cg_direction<T, false>;
+    hipLaunchKernelGGL(kernel, dim3(s.nblocks), red_blk(), 0, st, g, g.dzc, g.idzf64, z, pold, p, q, dots, sc, it, flex, partial, s.kchunk,
+                       s.ntx);
 }
 template <class T> void cg_gauge_norm(const DevGrid<T> &g, double *x, const double *p, double *r, const double *q,
-                                      const double *sc, int it, int step, double ncell, T *dense, double *partial, double *out,
-                                      hipStream_t st) {
-    hipLaunchKernelGGL(k_cg_gauge_norm<T>, red_grid(), red_blk(), 0, st, g, x, p, r, q, sc, it, step, ncell, dense, partial);
-    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 3, kRedBlocks, out);
+                                      const double *sc, const double *pq, int it, int step, double ncell, T *dense, double *partial,
+                                      double *out, double *host, hipStream_t st) {
+    const int npq = cg_direction_shape(g.Nx, g.Ny, g.Nz).nblocks;
+    hipLaunchKernelGGL(k_cg_gauge_norm<T>, red_grid(), red_blk(), 0, st, g, x, p, r, q, sc, pq, npq, it, step, ncell, dense, partial);
+    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 3, kRedBlocks, out, host);
 }
 template <class T> void cg_true_residual(const DevGrid<T> &g, const double *x, const double *b, double *e, double *partial,
                                          double *out, hipStream_t st) {
@@ -685,7 +839,7 @@ template <class T> void cg_true_residual(const DevGrid<T> &g, const double *x, c
 template <class T> void cg_gauged_norm(const DevGrid<T> &g, const double *e, double mean, double *partial, double *out,
                                        hipStream_t st) {
     hipLaunchKernelGGL(k_cg_gauged_norm<T>, red_grid(), red_blk(), 0, st, g, e, mean, partial);
-    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 1, kRedBlocks, out);
+    hipLaunchKernelGGL(k_cg_finish, dim3(1), red_blk(), 0, st, (const double *)partial, 1, kRedBlocks, out, (double *)nullptr);
 }
 
 #define OM_CG_INSTANTIATE(T)                                                                                     \
@@ -704,18 +858,18 @@ template <class T> void cg_gauged_norm(const DevGrid<T> &g, const double *e, dou
     template void ln_x0<T>(const DevGrid<T> &, const double *, const T *, double, double, void *, hipStream_t);     \
     template void ln_correct<T>(const DevGrid<T> &, T *, const float *, double, hipStream_t);                    \
     template void cg_copy_d<T>(const DevGrid<T> &, const double *, double *, hipStream_t);                       \
-    template void cg_dot2<T>(const DevGrid<T> &, const T *, const double *, const double *, double *, double *, hipStream_t); \
+    template void cg_dot2<T>(const DevGrid<T> &, const T *, const double *, const double *, double *, hipStream_t); \
     template void ln_target<T>(const DevGrid<T> &, const double *, const double *, const float *, double, float *, double *, \
                                double *, hipStream_t);                                                            \
     template void ln_center<T>(const DevGrid<T> &, float *, float, hipStream_t);                                 \
     template void ln_mask<T>(const DevGrid<T> &, float *, hipStream_t);                                          \
     template void ln_energy<T>(const DevGrid<T> &, const float *, const float *, double *, double, float *, double *, double *, \
                                hipStream_t);                                                                      \
-    template void cg_dot_zr<T>(const DevGrid<T> &, const T *, const double *, double *, double *, hipStream_t);  \
-    template void cg_update_p<T>(const DevGrid<T> &, double *, const T *, const double *, int, int, hipStream_t); \
-    template void cg_apply<T>(const DevGrid<T> &, const double *, double *, double *, double *, hipStream_t);   \
+    template void cg_dot_zr<T>(const DevGrid<T> &, const T *, const double *, double *, hipStream_t);  \
+    template void cg_direction<T>(const DevGrid<T> &, const T *, const double *, double *, double *, const double *, double *, int, int, int, \
+                                  double *, hipStream_t);                                                        \
     template void cg_gauge_norm<T>(const DevGrid<T> &, double *, const double *, double *, const double *,      \
-                                   const double *, int, int, double, T *, double *, double *, hipStream_t);     \
+                                   const double *, const double *, int, int, double, T *, double *, double *, double *, hipStream_t); \
     template void cg_true_residual<T>(const DevGrid<T> &, const double *, const double *, double *, double *,   \
                                       double *, hipStream_t);                                                    \
     template void cg_gauged_norm<T>(const DevGrid<T> &, const double *, double, double *, double *, hipStream_t);

@@ -256,17 +256,6 @@ template <class T> struct IB {
     __device__ __forceinline__ explicit IB(const DevGrid<T> &gg) : g(gg) {}
     __device__ __forceinline__ bool on() const { return g.kbot != nullptr; }
     __device__ __forceinline__ bool outside(int k) const { return g.tz == OM_BOUNDED && (k < 0 || k >= g.Nz); }
-    // periodic wrap of a column index into [0, n): one add or subtract for the stencil offsets
-    // (|offset| < n), an integer remainder only for points further out (grids narrower than a stencil)
-    static __device__ __forceinline__ int wrap(int i, int n) {
-        if (i < 0) i += n;
-        else if (i >= n) i -= n;
-        if ((unsigned)i >= (unsigned)n) {
-            i %= n;
-            if (i < 0) i += n;
-        }
-        return i;
-    }
     __device__ __forceinline__ int column(int i, int j) const { return (i + kBottomMargin) + (g.Nx + 2 * kBottomMargin) * (j + kBottomMargin); }
     __device__ __forceinline__ bool immersed(int i, int j, int k) const { return g.kbot && k < g.kbot_wide[column(i, j)]; }
     __device__ __forceinline__ bool inactive_cell(int i, int j, int k) const { return immersed(i, j, k) || outside(k); }
@@ -817,15 +806,30 @@ inline CgStencilShape cg_stencil_shape(int Nx, int Ny, int Nz) {
     s.nblocks = tiles * nch;
     return s;
 }
-inline int cg_partials_needed(int Nx, int Ny, int Nz) {
-    return std::max(4 * kCgRedBlocks, 3 * cg_stencil_shape(Nx, Ny, Nz).nblocks);
+// The direction sweep's tile and chunk: about kCgDirBlocks blocks (two per CU, all resident at once: 160 VGPRs
+// allow three) where the grid allows chunks of eight levels or more (a chunk reads two levels beyond its own).
+constexpr int kCgDirX = 64, kCgDirY = 8, kCgDirBlocks = 512;
+inline CgStencilShape cg_direction_shape(int Nx, int Ny, int Nz) {
+    CgStencilShape s;
+    s.ntx = (Nx + kCgDirX - 1) / kCgDirX;
+    s.nty = (Ny + kCgDirY - 1) / kCgDirY;
+    const int tiles = s.ntx * s.nty;
+    int nch = std::max(1, std::min((Nz + 7) / 8, kCgDirBlocks / tiles));
+    s.kchunk = (Nz + nch - 1) / nch;
+    nch = (Nz + s.kchunk - 1) / s.kchunk;
+    s.nblocks = tiles * nch;
+    return s;
+}
+// One of a solver's three sets of partial sums: the sweep that reads one set writes another.
+inline size_t cg_partials_needed(int Nx, int Ny, int Nz) {
+    return (size_t)std::max(4 * kCgRedBlocks, std::max(cg_stencil_shape(Nx, Ny, Nz).nblocks, 3 * cg_direction_shape(Nx, Ny, Nz).nblocks));
 }
 // The iteration's scalars stay on the device, in the solver's reduction-output array: slots 0-3
-// hold results the host reads; ρ of iteration k (and, for flexible CG, z·r_prev after it) sit at
-// cg_slot_rho(k) by the parity of k, so that ρ_prev is still there; then p·Ap with the sums of p
-// and A·p, and the gauge sweep's ‖V⁻¹r‖² with the sums of x and r.  The update kernels form α, β and
-// the gauge means from them.
-constexpr int kCgSlotRho = 8, kCgSlotPQ = 12, kCgSlotGauge = 16, kCgSlots = 24;   // PQ: p·Ap, Σp, Σq; Gauge: ‖V⁻¹r‖², Σx, Σr
+// hold results the host reads; ρ of iteration k sits at
+// cg_slot_rho(k) by the parity of k, so that ρ_prev is still there; then the gauge sweep's ‖V⁻¹r‖²
+// with the sums of x and r.  The sweeps form α, β and the gauge means from them and from the partial
+// sums of the launch before.
+constexpr int kCgSlotRho = 8, kCgSlotGauge = 16, kCgSlots = 24;   // Gauge: ‖V⁻¹r‖², Σx, Σr
 __host__ __device__ inline int cg_slot_rho(int it) { return kCgSlotRho + 2 * (it & 1); }
 template <class T> void cg_scale(const DevGrid<T> &g, T *f, T s, int mode, hipStream_t st);
 template <class T> void cg_gather(const DevGrid<T> &g, const double *x, T *dense, hipStream_t st);
@@ -842,7 +846,7 @@ template <class T> void ln_input(const DevGrid<T> &g, const double *r, const T *
 template <class T> void ln_x0(const DevGrid<T> &g, const double *r, const T *z, double isr, double isz, void *x0, hipStream_t st);
 template <class T> void ln_correct(const DevGrid<T> &g, T *z, const float *out, double sz, hipStream_t st);
 template <class T> void cg_copy_d(const DevGrid<T> &g, const double *src, double *dst, hipStream_t st);
-template <class T> void cg_dot2(const DevGrid<T> &g, const T *z, const double *r, const double *rp, double *partial, double *out,
+template <class T> void cg_dot2(const DevGrid<T> &g, const T *z, const double *r, const double *rp, double *partial,
                                 hipStream_t st);
 template <class T> void ln_target(const DevGrid<T> &g, const double *xf, const double *xk, const float *in3k, double isz, float *tgt,
                                   double *partial, double *out, hipStream_t st);
@@ -854,16 +858,18 @@ template <class T> void ln_energy(const DevGrid<T> &g, const float *y, const flo
                                   double *partial, double *out, hipStream_t st);
 // ColumnwiseTridiagonalPreconditioner: z = Lz⁻¹ r per column; t is an Nx·Ny·Nz scratch array
 template <class T> void cg_ct(const DevGrid<T> &g, const double *r, T *z, T *t, hipStream_t st);
-template <class T> void cg_dot_zr(const DevGrid<T> &g, const T *z, const double *r, double *partial, double *out, hipStream_t st);
-template <class T> void cg_update_p(const DevGrid<T> &g, double *p, const T *z, const double *sc, int it, int flex, hipStream_t st);
-template <class T> void cg_apply(const DevGrid<T> &g, const double *p, double *q, double *partial, double *out, hipStream_t st);
+template <class T> void cg_dot_zr(const DevGrid<T> &g, const T *z, const double *r, double *partial, hipStream_t st);
+// p = z (first) or z + β p_old, q = V∇²p, with ρ from the dot's partial sums; partial sums of p·q, Σp, Σq (p
+// and p_old, dots and partial: different buffers)
+template <class T> void cg_direction(const DevGrid<T> &g, const T *z, const double *pold, double *p, double *q, const double *dots,
+                                     double *sc, int it, int first, int flex, double *partial, hipStream_t st);
 // The gauge and norm sweep (step = 0: the solve's first; step = 1: with the iteration's update of
-// x and r folded in); writes ‖V⁻¹r‖², Σx, Σr to out.  dense: also write r V⁻¹ in FP32 cell order,
+// x and r folded in, from the direction sweep's partial sums pq); writes ‖V⁻¹r‖², Σx, Σr to out and the
+// first to host memory too.  dense: also write r V⁻¹ in FP32 cell order,
 // the FFT preconditioner's source (may be null).
 template <class T> void cg_gauge_norm(const DevGrid<T> &g, double *x, const double *p, double *r, const double *q,
-                                      const double *sc, int it, int step, double ncell, T *dense, double *partial, double *out,
-                                      hipStream_t st);
-// (the p update also fills p's one-layer halos)
+                                      const double *sc, const double *pq, int it, int step, double ncell, T *dense, double *partial,
+                                      double *out, double *host, hipStream_t st);
 template <class T> void cg_true_residual(const DevGrid<T> &g, const double *x, const double *b, double *e, double *partial,
                                          double *out, hipStream_t st);
 template <class T> void cg_gauged_norm(const DevGrid<T> &g, const double *e, double mean, double *partial, double *out,
