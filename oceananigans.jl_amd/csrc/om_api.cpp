@@ -630,6 +630,8 @@ template <class T> struct ModelT : ModelBase {
             if (g.kbot) launch_tendencies(C, st, true);   // cells within reach of the immersed bottom
         } else if (tune_tendency_kernel == 0 && centered_tendencies_supported(C)) {
             launch_tend_centered(C, tune_kchunk, st);
+        } else if (tune_tendency_kernel == 0 && flat_tendencies_supported(C)) {
+            launch_tend_flat(C, st);
         } else {
             launch_tendencies(C, st);
         }

@@ -769,6 +769,9 @@ template <class T> bool centered_tendencies_supported(const Ctx<T> &C);
 template <class T> void launch_tend_centered(const Ctx<T> &C, int kchunk, hipStream_t st);
 template <class T> bool tiled_tendencies_supported(const Ctx<T> &C);
 template <class T> void launch_tend_tiled(const Ctx<T> &C, int kchunk, hipStream_t st);
+// Flat z, Periodic x and y, no immersed bottom (om_kernels.hip)
+template <class T> bool flat_tendencies_supported(const Ctx<T> &C);
+template <class T> void launch_tend_flat(const Ctx<T> &C, hipStream_t st);
 template <class T> void launch_closure(const Ctx<T> &C, hipStream_t st, bool fixup = false);
 // z-marching LDS-tiled eddy viscosity / diffusivity kernel (om_closure_tiled.hip)
 template <class T> bool tiled_closure_supported(const Ctx<T> &C);

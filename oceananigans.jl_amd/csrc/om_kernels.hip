@@ -154,6 +154,101 @@ template <class T> __global__ void __launch_bounds__(256) k_tendencies(Ctx<T> C,
 }
 
 // ----------------------------------------------------------------------------------------
+// The same tendencies on a Flat z with Periodic x and y, without an immersed bottom: a block evaluates
+// one field (blockIdx.z) on 15 × 15 cells, each of its 256 threads one x-face and one y-face flux of it,
+// which the cells difference from LDS, so every flux is evaluated once where k_tendencies evaluates it
+// twice.  On a small grid a launch lasts as long as one wave, and that is mostly the fetching of its
+// instructions, so one loop body serves both directions of every field, by pointers and strides.  128 × 128
+// FP64: 17 µs in k_tendencies, 14 with each field's two fluxes spelled out, 4.7 here.  The fluxes are
+// those of Ctx (F_Uu … F_cy), operand for operand: the same bits in FP64.
+// ----------------------------------------------------------------------------------------
+constexpr int kFlatTile = 15;
+template <class T, int ADV> __global__ void __launch_bounds__(256) k_tend_flat(Ctx<T> C) {
+    __shared__ T fx[2][256], fy[2][256];   // advective, viscous / diffusive
+    const int tid = threadIdx.x, a = tid & 15, b = tid >> 4, field = blockIdx.z;
+    const int ic = blockIdx.x * kFlatTile + a, jc = blockIdx.y * kFlatTile + b;
+    const int i = min(ic, C.g.Nx), j = min(jc, C.g.Ny);   // (the last cells' far faces are the last evaluated)
+    constexpr int k = 0;
+    const bool clo = C.ph.closure != OM_CLOSURE_NONE;
+    // (the pointer tables with compile-time indices, as in k_tendencies)
+    const T *psi = C.s.U[0];
+#pragma unroll
+    for (int f = 1; f < kMaxFields; ++f) if (f == field) psi = C.s.U[f];
+    const int64_t o = C.at(i, j, k);
+    // u and v are carried by velocities interpolated along their own axis; w and tracers by the velocity
+    // at the face
+    const bool own = field < 2;
+    const int64_t along = field == 0 ? 1 : C.g.sy;
+    const T *const u = C.s.U[0] + o, *const v = C.s.U[1] + o;
+    const T Ax = field == 2 && ADV == OM_ADV_CENTERED2 ? C.Axf(k) : C.Axc(k), Ay = field == 2 && ADV == OM_ADV_CENTERED2 ? C.Ayf(k) : C.Ayc(k);
+    psi += o;
+    T ax = T(0), ay = T(0);
+#pragma unroll 1
+    for (int d = 0; d < 2; ++d) {
+        const T *vel = d ? v : u;
+        const int64_t st = d ? C.g.sy : 1;
+        const T A = d ? Ay : Ax;
+        T F;
+        if (ADV == OM_ADV_CENTERED2) {
+            const T vf = own ? T(0.5) * (vel[-along] + vel[0]) : vel[0];
+            F = A * vf * (T(0.5) * (psi[-st] + psi[0]));
+        } else {
+            const T ut = own ? cen4<T>(A * vel[-2 * along], A * vel[-along], A * vel[0], A * vel[along]) : A * vel[0];
+            F = ut * weno5<T>(psi[-3 * st], psi[-2 * st], psi[-st], psi[0], psi[st], psi[2 * st], ut > T(0));
+        }
+        if (d) ay = F;
+        else ax = F;
+    }
+    T vx = T(0), vy = T(0);
+    if (clo) {
+        if (field == 0) {   // x: at centre i − 1, y: at edge j
+            vx = C.Axc(k) * C.f_ux(i - 1, j, k);
+            vy = C.Ayc(k) * C.f_uy(i, j, k);
+        } else if (field == 1) {
+            vx = C.Axc(k) * C.f_uy(i, j, k);
+            vy = C.Ayc(k) * C.f_vy(i, j - 1, k);
+        } else if (field == 2) {
+            vx = C.Axf(k) * C.f_uz(i, j, k);
+            vy = C.Ayf(k) * C.f_vz(i, j, k);
+        } else {
+#pragma unroll
+            for (int n = 0; n < kMaxTracers; ++n) {
+                if (field != 3 + n) continue;
+                vx = C.Axc(k) * C.q_x(n, C.s.U[3 + n], i, j, k);
+                vy = C.Ayc(k) * C.q_y(n, C.s.U[3 + n], i, j, k);
+            }
+        }
+    }
+    fx[0][tid] = ax;
+    fy[0][tid] = ay;
+    if (clo) { fx[1][tid] = vx; fy[1][tid] = vy; }
+    __syncthreads();
+    if (a >= kFlatTile || b >= kFlatTile || ic >= C.g.Nx || jc >= C.g.Ny) return;
+    const T iV = field == 2 ? C.iVf(k) : C.iVc(k);
+    T G = T(0);
+    G -= iV * (((fx[0][tid + 1] - fx[0][tid]) + (fy[0][tid + 16] - fy[0][tid])) + T(0));
+    if (C.ph.coriolis && field < 2) {
+        const T *o = C.s.U[1 - field];
+        const T A = field == 0 ? C.Ayc(k) : C.Axc(k);
+        auto q = [&](int ii, int jj) { return A * C.ld(o, ii, jj, k); };
+        const T I = field == 0 ? T(0.5) * (T(0.5) * (q(i - 1, j) + q(i, j)) + T(0.5) * (q(i - 1, j + 1) + q(i, j + 1)))
+                               : T(0.5) * (T(0.5) * (q(i, j - 1) + q(i + 1, j - 1)) + T(0.5) * (q(i, j) + q(i + 1, j)));
+        const T cor = (T(0.5) * (C.ph.f + C.ph.f)) * I * recip<T>(A);
+        G = field == 0 ? G + cor : G - cor;
+    }
+    if (C.ph.hydrostatic && field < 2) {
+        const T *d = field == 0 ? C.s.dxpHY : C.s.dypHY;
+        const T dp = d ? C.ld(d, i, j, k) : C.ld(C.s.pHY, i, j, k) - (field == 0 ? C.ld(C.s.pHY, i - 1, j, k) : C.ld(C.s.pHY, i, j - 1, k));
+        G -= dp * (field == 0 ? C.g.idx : C.g.idy);
+    }
+    if (clo) G -= iV * (((fx[1][tid + 1] - fx[1][tid]) + (fy[1][tid + 16] - fy[1][tid])) + T(0));
+    T *out = C.s.Gn[0];
+#pragma unroll
+    for (int f = 1; f < kMaxFields; ++f) if (f == field) out = C.s.Gn[f];
+    out[C.at(i, j, k)] = G;
+}
+
+// ----------------------------------------------------------------------------------------
 // Eddy viscosity / diffusivity (AMD: anisotropic_minimum_dissipation.jl:161-358;
 // Smagorinsky-Lilly: smagorinsky.jl:90-104, lilly_coefficient.jl:129-142)
 // ----------------------------------------------------------------------------------------
@@ -891,6 +986,17 @@ template <class T> void launch_tendencies(const Ctx<T> &C, hipStream_t st, bool 
     }
     hipLaunchKernelGGL(k_tendencies<T>, cell_grid(C.g.Nx, C.g.Ny, C.g.Nz, blk), blk, 0, st, C, 0);
 }
+template <class T> bool flat_tendencies_supported(const Ctx<T> &C) {
+    const DevGrid<T> &g = C.g;
+    const int halo = C.ph.advection == OM_ADV_WENO5 ? 3 : 1;
+    return (C.ph.advection == OM_ADV_WENO5 || C.ph.advection == OM_ADV_CENTERED2) && g.tx == OM_PERIODIC && g.ty == OM_PERIODIC &&
+           g.tz == OM_FLAT && !g.kbot && g.Hx >= halo && g.Hy >= halo;
+}
+template <class T> void launch_tend_flat(const Ctx<T> &C, hipStream_t st) {
+    const dim3 grid((C.g.Nx + kFlatTile - 1) / kFlatTile, (C.g.Ny + kFlatTile - 1) / kFlatTile, 3 + C.ph.n_tracers);
+    const auto kernel = C.ph.advection == OM_ADV_WENO5 ? &k_tend_flat<T, OM_ADV_WENO5> : &k_tend_flat<T, OM_ADV_CENTERED2>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, C);
+}
 template <class T> void launch_closure(const Ctx<T> &C, hipStream_t st, bool fixup) {
     dim3 blk(kGenericBlockX, kGenericBlockY, 1);
     if (fixup) {
@@ -982,6 +1088,8 @@ template <class T> void launch_halos(const DevGrid<T> &g, const HaloJob<T> &J, h
 
 #define OM_INSTANTIATE(T)                                                                           \
     template void launch_tendencies<T>(const Ctx<T> &, hipStream_t, bool);                         \
+    template bool flat_tendencies_supported<T>(const Ctx<T> &);                                    \
+    template void launch_tend_flat<T>(const Ctx<T> &, hipStream_t);                                \
     template void launch_closure<T>(const Ctx<T> &, hipStream_t, bool);                            \
     template void launch_hydrostatic<T>(const Ctx<T> &, hipStream_t);                              \
     template void launch_rk3<T>(const Ctx<T> &, T, T, T, int, int, hipStream_t);                    \
