@@ -258,6 +258,7 @@ template <class T> struct ModelT : ModelBase {
     ~ModelT() override {
         if (st) (void)hipStreamSynchronize(st);
         if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
+        for (hipGraphExec_t x : single_exec) if (x) (void)hipGraphExecDestroy(x);
         for (void *p : allocs) (void)hipFree(p);
         if (cg_host) (void)hipHostFree(cg_host);
         if (diag_host) (void)hipHostFree(diag_host);
@@ -279,9 +280,33 @@ template <class T> struct ModelT : ModelBase {
             if (allocs[q] == p) { HIPCHECK(hipFree(p)); allocs.erase(allocs.begin() + q); return; }
     }
     template <class U> const U *upload(const std::vector<U> &h) {
-        U *d = dalloc<U>(h.size());
-        HIPCHECK(hipMemcpy(d, h.data(), h.size() * sizeof(U), hipMemcpyHostToDevice));
-        return d;
+        // small tables are gathered into blocks, copied together by flush_uploads (an allocation, a memset and
+        // a copy of each were a third of a small model's construction); 256 bytes of zeros behind each
+        const size_t bytes = h.size() * sizeof(U), span = (bytes + 256 + 255) & ~(size_t)255;
+        if (span > kStageBlock) {
+            U *d = dalloc<U>(h.size());
+            HIPCHECK(hipMemcpy(d, h.data(), bytes, hipMemcpyHostToDevice));
+            return d;
+        }
+        if (!stage_dev || staged.size() + span > kStageBlock) {
+            flush_uploads();
+            void *p = nullptr;
+            HIPCHECK(hipMalloc(&p, kStageBlock));
+            allocs.push_back(p);
+            stage_dev = static_cast<char *>(p);
+        }
+        const size_t at = staged.size();
+        staged.resize(at + span, 0);
+        memcpy(staged.data() + at, h.data(), bytes);
+        return reinterpret_cast<U *>(stage_dev + at);
+    }
+    static constexpr size_t kStageBlock = 128 * 1024;
+    std::vector<char> staged;       // the current block's tables on the host
+    char *stage_dev = nullptr;      // and its memory on the device
+    void flush_uploads() {
+        if (!staged.empty()) HIPCHECK(hipMemcpy(stage_dev, staged.data(), staged.size(), hipMemcpyHostToDevice));
+        staged.clear();
+        stage_dev = nullptr;
     }
 
     // Field layout: rows of sy elements (pnx rounded up to 128 bytes), planes of sz = sy·pny, and a
@@ -525,6 +550,7 @@ template <class T> struct ModelT : ModelBase {
                 refop.idzf = upload(idzf);
             }
         }
+        flush_uploads();   // (every table is made above; kernels that read them are launched below)
         diag_partial = dalloc<double>(3 * 1024);
         diag_out = dalloc<double>(4);
         HIPCHECK(hipHostMalloc((void **)&diag_host, 4 * sizeof(double), hipHostMallocDefault));
@@ -1000,8 +1026,22 @@ template <class T> struct ModelT : ModelBase {
     int swap_parity = 0;   // parity of the G⁻/Gⁿ exchanges so far
     bool capturable() const { return !cg; }
     int launch_version = 0;   // changes with every change of a launch choice (tuning, autotuner)
+    // Steps taken one at a time (a call per iteration): one step exchanges G⁻/Gⁿ an odd number of times, so
+    // there is a graph for each buffer assignment.  Captured when Δt has stayed the same for
+    // kSingleStepsBefore calls: capturing costs about as much as the launches of that many small steps, so a
+    // Δt that changes from call to call never pays for it.  (A step of 30 launches on a small grid:
+    // 152 → 130 µs in FP64 128 × 128, 214 → 174 in FP32 32³.)
+    static constexpr int kSingleStepsBefore = 6;
+    hipGraphExec_t single_exec[2] = {nullptr, nullptr};
+    double single_dt = 0;   // Δt of the single steps so far, and of the graphs
+    int single_steps = 0;   // their number
+    void drop_single() {
+        for (hipGraphExec_t &x : single_exec)
+            if (x) { HIPCHECK(hipGraphExecDestroy(x)); x = nullptr; }
+    }
     void drop_graph() {
         ++launch_version;
+        drop_single();
         if (graph_exec) { HIPCHECK(hipGraphExecDestroy(graph_exec)); graph_exec = nullptr; }
     }
     void capture(double dt) {
@@ -1019,9 +1059,38 @@ template <class T> struct ModelT : ModelBase {
         graph_dt = dt;
         graph_parity = swap_parity;
     }
+    void single_step(double dt) {
+        if (single_dt != dt) {
+            drop_single();
+            single_dt = dt;
+            single_steps = 0;
+        }
+        if (single_steps < kSingleStepsBefore) {
+            ++single_steps;
+            time_step(dt);
+            return;
+        }
+        hipGraphExec_t &exec = single_exec[swap_parity];
+        if (exec) {
+            for (int q = 0; q < 3; ++q) cache_previous_tendencies();   // the step's exchanges
+        } else {
+            const bool pt = phase_timing;
+            phase_timing = false;
+            hipGraph_t gr = nullptr;
+            HIPCHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+            step_launches(dt);
+            HIPCHECK(hipStreamEndCapture(st, &gr));
+            phase_timing = pt;
+            HIPCHECK(hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0));
+            HIPCHECK(hipGraphDestroy(gr));
+        }
+        HIPCHECK(hipGraphLaunch(exec, st));
+        step_clock(dt);
+    }
     // enqueue (without waiting) up to two steps of Δt; returns the number of steps issued
     int issue_steps(double dt, int left, bool use_graph) {
-        if (!use_graph || !capturable() || iteration == 0 || left < 2) { time_step(dt); return 1; }
+        if (!use_graph || !capturable() || iteration == 0) { time_step(dt); return 1; }
+        if (left < 2) { single_step(dt); return 1; }
         if (!graph_exec || graph_dt != dt) capture(dt);
         if (graph_parity != swap_parity) { time_step(dt); return 1; }
         HIPCHECK(hipGraphLaunch(graph_exec, st));
