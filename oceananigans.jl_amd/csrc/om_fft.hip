@@ -745,7 +745,7 @@ template <class T> struct TriArgs {
 template <class T> constexpr int tri_batch() { return sizeof(T) == 4 ? 16 : 8; }
 // LDS bytes of a block of bw columns
 template <class T> constexpr size_t tri_lds(int Nz, int bw, bool keep) {
-    return ((size_t)Nz * bw * (keep ? 3 : 1) + 2 * (size_t)Nz + 1) * sizeof(T);
+    return ((size_t)Nz * bw * (keep ? 3 : 1) + (keep ? 2 * (size_t)Nz + 1 : 0)) * sizeof(T);
 }
 
 template <class T, bool KEEP>
@@ -757,8 +757,10 @@ __global__ void __launch_bounds__(64) k_tridiag(TriArgs<T> A, C2<T> *__restrict_
     const int bw = blockDim.x >> 1;            // columns of the block
     C2<T> *ph = reinterpret_cast<C2<T> *>(smem_raw);                  // KEEP: [Nz][bw]
     T *tt = reinterpret_cast<T *>(ph + (KEEP ? (size_t)Nz * bw : 0));   // [Nz][bw]
-    T *dz = tt + (size_t)Nz * bw;              // [Nz] Δzᶜ
-    T *iz = dz + Nz;                           // [Nz + 1] 1/Δzᶠ, the end faces 0
+    T *dz = tt + (size_t)Nz * bw;              // KEEP: [Nz] Δzᶜ
+    T *iz = dz + Nz;                           // and [Nz + 1] 1/Δzᶠ, the end faces 0
+    auto spacing = [&](int k) -> T { return KEEP ? dz[k] : dzc[k]; };
+    auto coupling = [&](int k) -> T { return KEEP ? iz[k] : (k == 0 || k == Nz ? T(0) : idzf[k]); };
     const bool down = (int)threadIdx.x >= bw;   // this lane's chain: from the top
     const int c = threadIdx.x - (down ? bw : 0);
     const int64_t ncol = (int64_t)A.Ms * Ny;
@@ -801,11 +803,13 @@ __global__ void __launch_bounds__(64) k_tridiag(TriArgs<T> A, C2<T> *__restrict_
     const C2<T> fmid = S[at(mid)];
     C2<T> f[KB];
     load(f, 0);
-    for (int k = threadIdx.x; k < Nz; k += blockDim.x) {
-        dz[k] = dzc[k];
-        iz[k] = k == 0 ? T(0) : idzf[k];
+    if (KEEP) {
+        for (int k = threadIdx.x; k < Nz; k += blockDim.x) {
+            dz[k] = dzc[k];
+            iz[k] = k == 0 ? T(0) : idzf[k];
+        }
+        if (threadIdx.x == 0) iz[Nz] = T(0);
     }
-    if (threadIdx.x == 0) iz[Nz] = T(0);
     __syncthreads();
     const bool singular = lam == T(0);   // the (0,0) column
     if (blockIdx.x == 0) {
@@ -821,9 +825,9 @@ __global__ void __launch_bounds__(64) k_tridiag(TriArgs<T> A, C2<T> *__restrict_
         // (the batch's coefficients before its arithmetic, whose stores to LDS they could not pass)
         T w[KB + 1], d[KB];
 #pragma unroll
-        for (int u = 0; u <= KB; ++u) w[u] = iz[down ? Nz - min(q0 + u, Nz) : min(q0 + u, Nz)];
+        for (int u = 0; u <= KB; ++u) w[u] = coupling(down ? Nz - min(q0 + u, Nz) : min(q0 + u, Nz));
 #pragma unroll
-        for (int u = 0; u < KB; ++u) d[u] = dz[level(min(q0 + u, longest))];
+        for (int u = 0; u < KB; ++u) d[u] = spacing(level(min(q0 + u, longest)));
         if (q0 + KB <= common) {
 #pragma unroll
             for (int u = 0; u < KB; ++u) eliminate(q0 + u, f[u], w[u], w[u + 1], d[u]);
@@ -840,8 +844,8 @@ __global__ void __launch_bounds__(64) k_tridiag(TriArgs<T> A, C2<T> *__restrict_
     {
         const T eb = __shfl(excess, c) * __shfl(ratio, c), et = __shfl(excess, c + bw) * __shfl(ratio, c + bw);
         const C2<T> pb = cmk<T>(__shfl(phi.x, c), __shfl(phi.y, c)), pt = cmk<T>(__shfl(phi.x, c + bw), __shfl(phi.y, c + bw));
-        const T below = iz[mid], above = iz[mid + 1];
-        const T pivot = dz[mid] * lam + (eb + et);
+        const T below = coupling(mid), above = coupling(mid + 1);
+        const T pivot = spacing(mid) * lam + (eb + et);
         if (!singular && pivot > A.eps10)
             x = cmk<T>(ft_div<T>((below * pb.x - fmid.x) + above * pt.x, pivot), ft_div<T>((below * pb.y - fmid.y) + above * pt.y, pivot));
         else x = cmk<T>(T(0), T(0));

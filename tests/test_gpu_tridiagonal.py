@@ -13,7 +13,7 @@ import oceananigans_mi355x as om
 pytestmark = pytest.mark.gpu
 
 SIZES = [(8, 6, 1), (8, 6, 2), (6, 8, 3), (16, 16, 15), (16, 16, 16), (40, 6, 17), (32, 8, 31), (33, 9, 32), (32, 10, 33), (48, 20, 34), (8, 8, 64),
-         (34, 12, 65), (70, 66, 67), (16, 8, 341), (16, 4, 342), (8, 4, 700)]
+         (34, 12, 65), (70, 66, 67), (16, 8, 341), (16, 4, 342), (8, 4, 700), (4, 4, 3000), (4, 3, 8192)]
 
 
 @pytest.mark.parametrize("ft", [np.float32, np.float64])
