@@ -218,7 +218,7 @@ template <class T> struct ModelT : ModelBase {
     bool chunks_chosen = false;        // by the caller or the autotuner: choose_chunks leaves them
     int cus = 256;                     // compute units of the device
     int tune_learned_iterations = 0;   // leading CG iterations that apply the learned correction (0: all)
-    int tune_step_graphs = 1;          // om_time_step replays captured two-step graphs
+    int tune_step_graphs = 1;          // om_time_step replays captured steps
     int tune_refine = 0;               // FP64 iterative refinement of FFT / Fourier–tridiagonal solves
     RefineOp refop{};                  // the solver's operator for the refinement residual
     T *ref_r = nullptr, *ref_d = nullptr;   // dense residual and correction
@@ -1447,8 +1447,8 @@ int om_time_step(om_model_t *m, double dt, int32_t nsteps) {
         M->evused = 0;
         M->cg_unconverged = 0;
         HIPCHECK(hipEventRecord(M->ev0, M->st));
-        // pairs of steps replay the model's captured two-step graph (the same launches, so the
-        // same results) unless phases are being timed or the graph form is switched off
+        // pairs of steps replay the model's captured two-step graph, repeated single steps a one-step
+        // graph (the same launches, so the same results), unless phases are being timed or the graph form is switched off
         const bool graphs = M->tune_step_graphs && !M->phase_timing;
         for (int left = nsteps; left > 0;) left -= M->issue_steps(dt, left, graphs);
         HIPCHECK(hipEventRecord(M->ev1, M->st));
