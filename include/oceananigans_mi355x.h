@@ -304,9 +304,9 @@ int om_last_step_timing(const om_model_t *m, double *ms_total, double *ms_per_ph
                                         already) or an immersed bottom. */
 #define OM_TUNE_STEP_GRAPHS 4      /* 1 (default): om_time_step advances pairs of steps by replaying the
                                        model's two-step launch sequence captured once into a hipGraph
-                                       (the same launches; recaptured after a change of Δt or of a
-                                       launch choice), and single steps likewise once Δt has stayed
-                                       the same for several of them; 0: every launch issued directly.  Phase timing
+                                       (the same launches, whatever Δt; recaptured after a change of a
+                                       launch choice), and single steps likewise after the first
+                                       few of them; 0: every launch issued directly.  Phase timing
                                        and the conjugate-gradient solver always launch directly. */
 #define OM_TUNE_CONV_TILED 5       /* convolutions of the learned preconditioner: 1 (default) input tiles
                                        staged in LDS; 0 the input read per tap.  Identical results. */

@@ -550,6 +550,7 @@ template <class T> struct ModelT : ModelBase {
                 refop.idzf = upload(idzf);
             }
         }
+        step_times = const_cast<T *>(upload(std::vector<T>(4)));   // (among the tables: an allocation less)
         flush_uploads();   // (every table is made above; kernels that read them are launched below)
         diag_partial = dalloc<double>(3 * 1024);
         diag_out = dalloc<double>(4);
@@ -695,7 +696,8 @@ template <class T> struct ModelT : ModelBase {
         compute_tendencies();
     }
     // defer: called inside a time step, whose update_state fills the velocity halos next
-    void pressure_correction(T dtau, bool defer = false) {
+    // at: where a captured step finds max(ε, Δτ) (StepScalar)
+    void pressure_correction(T dtau, bool defer = false, const T *at = nullptr) {
         if (g.kbot) {   // mask immersed velocities (pressure_correction.jl:7)
             PhaseScope ps(this, OM_PHASE_HALOS);
             launch_mask_velocities(g, s.U, st);
@@ -704,8 +706,7 @@ template <class T> struct ModelT : ModelBase {
             u_halo_pending = true;
         else
             halos_prognostic(0x7u, true);
-        const T eps = std::numeric_limits<T>::epsilon();
-        const T dtp = dtau > eps ? dtau : eps;
+        const T dtp = pressure_time(dtau);
         if (cg) {
             // solve_for_pressure.jl:149-161: warm start from p·Δt★, b = active·δ·V, solve V∇²ϕ = b;
             // then U −= ∇ϕ and p = ϕ / max(eps, Δt) (pressure_correction.jl:82-106)
@@ -720,22 +721,22 @@ template <class T> struct ModelT : ModelBase {
             halos_aux({s.pNHS});
             {
                 PhaseScope ps(this, OM_PHASE_CORRECTION);
-                launch_correct(ctx(), T(1), 1, st);
+                launch_correct(ctx(), StepScalar<T>(T(1)), 1, st);
                 cg_scale(g, s.pNHS, dtp, 1, st);
             }
             return;
         }
         {
             PhaseScope ps(this, OM_PHASE_POISSON);
-            launch_poisson(P, ctx(), (const T *)nullptr, s.pNHS, 0, dtp, st);
-            if (tune_refine) refine(s.pNHS, g.sy, g.sz, nullptr, (double)dtp);
+            launch_poisson(P, ctx(), (const T *)nullptr, s.pNHS, 0, StepScalar<T>(dtp, at), st);
+            if (tune_refine) refine(s.pNHS, g.sy, g.sz, nullptr, StepScalar<T>(dtp, at));
         }
         // periodic x and y without an immersed bottom or a refinement pass: the correction reads
         // p's neighbours across the edges by wrapped index, and p's halo fill joins the next
         // halo launch (update_state's), one launch fewer per substage
         const bool wrap = !tune_refine && !g.kbot && g.tx == OM_PERIODIC && g.ty == OM_PERIODIC;
         if (!wrap) halos_aux({s.pNHS});
-        { PhaseScope ps(this, OM_PHASE_CORRECTION); launch_correct(ctx(), dtp, 0, st, wrap ? 1 : 0); }
+        { PhaseScope ps(this, OM_PHASE_CORRECTION); launch_correct(ctx(), StepScalar<T>(dtp, at), 0, st, wrap ? 1 : 0); }
         p_halo_pending = wrap;
     }
 
@@ -899,7 +900,7 @@ template <class T> struct ModelT : ModelBase {
         while (it < maxiter && !(res <= tol)) {
             if (pk == OM_PRECOND_DIAGONALLY_DOMINANT) { cg_halo_r(g, cg_r, st); cg_dd(g, cg_r, cg_z, st); }
             else if (pk == OM_PRECOND_FFT || pk == OM_PRECOND_LEARNED) {
-                launch_poisson(P, ctx(), rhs_dense, cg_z, 0, T(1), st);   // source written by the last gauge sweep
+                launch_poisson(P, ctx(), rhs_dense, cg_z, 0, StepScalar<T>(T(1)), st);   // source written by the last gauge sweep
                 const bool log_this = logging && it < log_iters;
                 const bool learn_this = pk == OM_PRECOND_LEARNED && !fallback &&
                                         (tune_learned_iterations == 0 || it < tune_learned_iterations);
@@ -955,11 +956,16 @@ template <class T> struct ModelT : ModelBase {
         cg_gauged_norm(g, cg_q, emean, cg_partial, cg_out, st);
         cg_true_res_last = std::sqrt(cg_read(1));
     }
-    void rk3_substep(double dt, T gamma, T zeta, bool first, bool defer = false) {
+    static T substep_time(double dt, T gamma, T zeta, bool first) { return first ? (T)(dt * (double)gamma) : (T)(dt * (double)(gamma + zeta)); }
+    static T pressure_time(T dtau) {
+        const T eps = std::numeric_limits<T>::epsilon();
+        return dtau > eps ? dtau : eps;
+    }
+    // times: of a captured step, Δt (its first number) and the substep's max(ε, Δτ) (at `which`) in device memory
+    void rk3_substep(double dt, T gamma, T zeta, bool first, bool defer = false, const T *times = nullptr, int which = 0) {
         const T kdt = (T)dt;
-        const T dtau = first ? (T)(dt * (double)gamma) : (T)(dt * (double)(gamma + zeta));
-        { PhaseScope ps(this, OM_PHASE_RK_UPDATE); launch_rk3(ctx(), kdt, gamma, zeta, first ? 1 : 0, nf, st); }
-        pressure_correction(dtau, defer);
+        { PhaseScope ps(this, OM_PHASE_RK_UPDATE); launch_rk3(ctx(), StepScalar<T>(kdt, times), gamma, zeta, first ? 1 : 0, nf, st); }
+        pressure_correction(substep_time(dt, gamma, zeta, first), defer, times ? times + which : nullptr);
     }
     void set_refinement(int on) {
         if (on && (cg || g.kbot)) throw ArgError{"iterative refinement applies to the FFT and Fourier-tridiagonal solvers on a grid without an immersed bottom"};
@@ -970,9 +976,9 @@ template <class T> struct ModelT : ModelBase {
         tune_refine = on;
     }
     // one refinement step of the solution p (strides psy, psz) of L p = b (b64, or ∇·U / divisor)
-    void refine(T *p, int64_t psy, int64_t psz, const double *b64, double divisor) {
+    void refine(T *p, int64_t psy, int64_t psz, const double *b64, StepScalar<T> divisor) {
         launch_poisson_residual(ctx(), refop, p, psy, psz, b64, divisor, ref_r, st);
-        launch_poisson(P, ctx(), ref_r, ref_d, 1, T(1), st);
+        launch_poisson(P, ctx(), ref_r, ref_d, 1, StepScalar<T>(T(1)), st);
         launch_add_correction(g, p, psy, psz, ref_d, st);
     }
     void cache_previous_tendencies() {
@@ -983,16 +989,17 @@ template <class T> struct ModelT : ModelBase {
     }
     // RK3 coefficients (runge_kutta_3.jl:36-48)
     static constexpr double kG1 = 8.0 / 15, kG2 = 5.0 / 12, kG3 = 3.0 / 4, kZ2 = -17.0 / 60, kZ3 = -5.0 / 12;
-    // the device work of one time step: every launch depends only on Δt and the buffer assignment
-    void step_launches(double dt) {
+    // the device work of one time step: every launch depends only on Δt (by value, or through `times` in device
+    // memory) and the buffer assignment
+    void step_launches(double dt, const T *times = nullptr) {
         const T g1 = T(kG1), g2 = T(kG2), g3 = T(kG3), z2 = T(kZ2), z3 = T(kZ3);
-        rk3_substep(dt, g1, T(0), true, true);
+        rk3_substep(dt, g1, T(0), true, true, times, 1);
         cache_previous_tendencies();
         update_state();
-        rk3_substep(dt, g2, z2, false, true);
+        rk3_substep(dt, g2, z2, false, true, times, 2);
         cache_previous_tendencies();
         update_state();
-        rk3_substep(dt, g3, z3, false, true);
+        rk3_substep(dt, g3, z3, false, true, times, 3);
         cache_previous_tendencies();
         update_state();
     }
@@ -1016,84 +1023,76 @@ template <class T> struct ModelT : ModelBase {
         step_clock(dt);
     }
 
-    // ---- captured steps: two time steps recorded once into a hipGraph and replayed.  Two steps
-    // return G⁻/Gⁿ to the buffers they started in (three exchanges per step), so a replay is valid
-    // whenever the exchange parity matches the one at capture.  CG solves read scalars on the
-    // host and are never captured.
+    // ---- captured steps, recorded once into a hipGraph and replayed: two time steps, which return G⁻/Gⁿ to
+    // the buffers they started in (three exchanges per step), so that a replay is valid whenever the exchange
+    // parity matches the one at capture; and, for steps taken one at a time (a call per iteration), one step
+    // for each of the two buffer assignments.  CG solves read scalars on the host and are never captured.
+    // A captured step reads Δt and the substeps' times from device memory, written by a launch before the
+    // replay whenever they change, so that a graph serves every Δt.  (Two captures cost 110 µs at 128² in
+    // FP64 and 280 at 32³ in FP32, as much as seven and ten replays gain; with a graph for each Δt, changed every ten
+    // calls as a wizard does, a single step took 137 and 239 µs, launched directly 127 and 220, and
+    // takes 112 and 193 here, changed at every call 114 and 196.)
     hipGraphExec_t graph_exec = nullptr;
-    double graph_dt = 0;
     int graph_parity = 0;
     int swap_parity = 0;   // parity of the G⁻/Gⁿ exchanges so far
     bool capturable() const { return !cg; }
     int launch_version = 0;   // changes with every change of a launch choice (tuning, autotuner)
-    // Steps taken one at a time (a call per iteration): one step exchanges G⁻/Gⁿ an odd number of times, so
-    // there is a graph for each buffer assignment.  Captured when Δt has stayed the same for
-    // kSingleStepsBefore calls: capturing costs about as much as the launches of that many small steps, so a
-    // Δt that changes from call to call never pays for it.  (A step of 30 launches on a small grid:
-    // 152 → 130 µs in FP64 128 × 128, 214 → 174 in FP32 32³.)
+    // Single steps before the first capture, which a program of only a few would not earn back.  (From
+    // 64³ on the device is the slower side, and a replay takes as long as the direct launches: 273 µs.)
     static constexpr int kSingleStepsBefore = 6;
     hipGraphExec_t single_exec[2] = {nullptr, nullptr};
-    double single_dt = 0;   // Δt of the single steps so far, and of the graphs
-    int single_steps = 0;   // their number
-    void drop_single() {
-        for (hipGraphExec_t &x : single_exec)
-            if (x) { HIPCHECK(hipGraphExecDestroy(x)); x = nullptr; }
-    }
+    int single_steps = 0;
+    T *step_times = nullptr;     // device: Δt, max(ε, Δτ) of the three substeps
+    double step_times_dt = NAN;  // the Δt they belong to
     void drop_graph() {
         ++launch_version;
-        drop_single();
-        if (graph_exec) { HIPCHECK(hipGraphExecDestroy(graph_exec)); graph_exec = nullptr; }
+        single_steps = 0;
+        for (hipGraphExec_t *x : {&graph_exec, &single_exec[0], &single_exec[1]})
+            if (*x) { HIPCHECK(hipGraphExecDestroy(*x)); *x = nullptr; }
     }
-    void capture(double dt) {
-        drop_graph();
+    void capture(hipGraphExec_t &exec, int steps, double dt) {
         const bool pt = phase_timing;
         phase_timing = false;
         hipGraph_t gr = nullptr;
         HIPCHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        step_launches(dt);
-        step_launches(dt);
+        for (int q = 0; q < steps; ++q) step_launches(dt, step_times);
         HIPCHECK(hipStreamEndCapture(st, &gr));
         phase_timing = pt;
-        HIPCHECK(hipGraphInstantiate(&graph_exec, gr, nullptr, nullptr, 0));
+        HIPCHECK(hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0));
         HIPCHECK(hipGraphDestroy(gr));
-        graph_dt = dt;
-        graph_parity = swap_parity;
+    }
+    void replay(hipGraphExec_t exec, double dt) {
+        if (step_times_dt != dt) {
+            const T g1 = T(kG1), g2 = T(kG2), g3 = T(kG3), z2 = T(kZ2), z3 = T(kZ3);
+            launch_step_times(StepTimes<T>{{(T)dt, pressure_time(substep_time(dt, g1, T(0), true)),
+                                            pressure_time(substep_time(dt, g2, z2, false)), pressure_time(substep_time(dt, g3, z3, false))}},
+                              step_times, st);
+            step_times_dt = dt;
+        }
+        HIPCHECK(hipGraphLaunch(exec, st));
     }
     void single_step(double dt) {
-        if (single_dt != dt) {
-            drop_single();
-            single_dt = dt;
-            single_steps = 0;
-        }
         if (single_steps < kSingleStepsBefore) {
             ++single_steps;
             time_step(dt);
             return;
         }
         hipGraphExec_t &exec = single_exec[swap_parity];
-        if (exec) {
-            for (int q = 0; q < 3; ++q) cache_previous_tendencies();   // the step's exchanges
-        } else {
-            const bool pt = phase_timing;
-            phase_timing = false;
-            hipGraph_t gr = nullptr;
-            HIPCHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            step_launches(dt);
-            HIPCHECK(hipStreamEndCapture(st, &gr));
-            phase_timing = pt;
-            HIPCHECK(hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0));
-            HIPCHECK(hipGraphDestroy(gr));
-        }
-        HIPCHECK(hipGraphLaunch(exec, st));
+        if (exec) for (int q = 0; q < 3; ++q) cache_previous_tendencies();   // the step's exchanges
+        else capture(exec, 1, dt);                                           // (makes them)
+        replay(exec, dt);
         step_clock(dt);
     }
     // enqueue (without waiting) up to two steps of Δt; returns the number of steps issued
     int issue_steps(double dt, int left, bool use_graph) {
         if (!use_graph || !capturable() || iteration == 0) { time_step(dt); return 1; }
         if (left < 2) { single_step(dt); return 1; }
-        if (!graph_exec || graph_dt != dt) capture(dt);
+        if (!graph_exec) {
+            capture(graph_exec, 2, dt);
+            graph_parity = swap_parity;
+        }
         if (graph_parity != swap_parity) { time_step(dt); return 1; }
-        HIPCHECK(hipGraphLaunch(graph_exec, st));
+        replay(graph_exec, dt);
         step_clock(dt);
         step_clock(dt);
         return 2;
@@ -1496,10 +1495,10 @@ int om_poisson_solve(om_model_t *m, const double *rhs, double *phi) {
             M->cg_solve();
             cg_gather(M->g, M->cg_x, M->phi_dense, M->st);
         } else {
-            launch_poisson(M->P, M->ctx(), M->rhs_dense, M->phi_dense, 1, (TT)1, M->st);
+            launch_poisson(M->P, M->ctx(), M->rhs_dense, M->phi_dense, 1, om::StepScalar<TT>((TT)1), M->st);
             if (M->tune_refine) {
                 HIPCHECK(hipMemcpyAsync(M->ref_b64, rhs, n * sizeof(double), hipMemcpyHostToDevice, M->st));
-                M->refine(M->phi_dense, M->g.Nx, (int64_t)M->g.Nx * M->g.Ny, M->ref_b64, 1.0);
+                M->refine(M->phi_dense, M->g.Nx, (int64_t)M->g.Nx * M->g.Ny, M->ref_b64, om::StepScalar<TT>((TT)1));
             }
         }
         HIPCHECK(hipStreamSynchronize(M->st));

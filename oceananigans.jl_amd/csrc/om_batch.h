@@ -21,6 +21,8 @@
 #include <type_traits>
 #include <vector>
 
+#include "om_internal.h"
+
 namespace om {
 
 struct Blk {
@@ -35,7 +37,6 @@ template <class A> struct BatchEntry {
 // The arguments of a kind that declares kArgsInMemory are read where the launch put them (the
 // kernel-argument segment, or the batch's table), in the constant address space, so that the kind may
 // read them again (ConstArgs) instead of holding them all in scalar registers.
-#define OM_CONSTANT __attribute__((address_space(4)))
 template <class K, class = void> struct ArgsInMemory { static constexpr bool value = false; };
 template <class K> struct ArgsInMemory<K, std::enable_if_t<K::kArgsInMemory>> { static constexpr bool value = true; };
 

@@ -483,7 +483,7 @@ template <class T> struct XBwdArgs {
     T *out;            // field interior view (strided) or dense array
     int dense;
     T scale;           // 1 / (Nx · Ny · Nz-normalisations)
-    T divisor;         // the written value is (x · scale) / divisor
+    StepScalar<T> divisor;   // the written value is (x · scale) / divisor
     // even Nx: take X_0 and X_{Nx/2} as real, which they are but for rounding.  Their imaginary parts
     // hold the forward passes' rounding, amplified at the longest y and z waves by the inverse
     // Laplacian, and would enter the output as a ±1 wave along x (a u error of 4e-6 of max |u| at
@@ -501,6 +501,7 @@ template <class T, bool MIXED> struct KXBwd {
 };
 template <class T, bool MIXED> __device__ __forceinline__ void KXBwd<T, MIXED>::run(const XBwdArgs<T> &A, const Blk &B) {
     extern __shared__ unsigned char smem_raw[];
+    const T divisor = A.divisor.get();
     const int Nx = A.g.Nx, Ny = A.g.Ny;
     const bool half = (Nx & 1) == 0;
     const int M = half ? Nx / 2 : Nx;
@@ -559,7 +560,7 @@ template <class T, bool MIXED> __device__ __forceinline__ void KXBwd<T, MIXED>::
             T x;
             if (half) { const C2<T> zz = z[r * ld + (i >> 1)]; x = (i & 1) ? zz.y : zz.x; }
             else x = z[r * ld + i].x;
-            dst[i] = ft_div<T>(x * A.scale, A.divisor);   // IEEE in FP64; FP32 by the reciprocal of the divisor
+            dst[i] = ft_div<T>(x * A.scale, divisor);   // IEEE in FP64; FP32 by the reciprocal of the divisor
         }
     }
 }
@@ -1024,7 +1025,7 @@ __global__ void __launch_bounds__(64, 2) k_tridiag_short(TriArgs<T> A, C2<T> *__
 // ---------------------------------------------------------------------------------------------
 template <class T>
 __global__ void __launch_bounds__(256) k_poisson_residual(Ctx<T> C, RefineOp L, const T *p, int64_t psy, int64_t psz,
-                                                          const double *b64, double idiv, T *r) {
+                                                          const double *b64, StepScalar<T> divisor, T *r) {
     const DevGrid<T> &g = C.g;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int j = blockIdx.y * blockDim.y + threadIdx.y;
@@ -1042,7 +1043,7 @@ __global__ void __launch_bounds__(256) k_poisson_residual(Ctx<T> C, RefineOp L, 
         if (!C.fly()) b += ((double)C.ld(C.s.U[1], i, jp, k) - (double)C.ld(C.s.U[1], i, j, k)) * (double)g.idy;
         if (!C.flz())
             b += ((double)C.ld(C.s.U[2], i, j, k + 1) - (double)C.ld(C.s.U[2], i, j, k)) * (L.ihz2 < 0 ? L.idzc[k] : (double)g.idzc[k]);
-        b *= idiv;
+        b *= 1.0 / (double)divisor.get();
     }
     auto P = [&](int ii, int jj, int kk) -> double { return (double)p[(int64_t)ii + psy * jj + psz * kk]; };
     const double pc = P(i, j, k);
@@ -1074,9 +1075,9 @@ __global__ void __launch_bounds__(256) k_add_correction(DevGrid<T> g, T *p, int6
 }
 
 template <class T> void launch_poisson_residual(const Ctx<T> &C, const RefineOp &L, const T *p, int64_t psy, int64_t psz,
-                                                const double *b64, double divisor, T *r, hipStream_t st) {
+                                                const double *b64, StepScalar<T> divisor, T *r, hipStream_t st) {
     const dim3 blk(64, 4, 1), grid((C.g.Nx + 63) / 64, (C.g.Ny + 3) / 4, C.g.Nz);
-    hipLaunchKernelGGL(k_poisson_residual<T>, grid, blk, 0, st, C, L, p, psy, psz, b64, 1.0 / divisor, r);
+    hipLaunchKernelGGL(k_poisson_residual<T>, grid, blk, 0, st, C, L, p, psy, psz, b64, divisor, r);
 }
 template <class T> void launch_add_correction(const DevGrid<T> &g, T *p, int64_t psy, int64_t psz, const T *d, hipStream_t st) {
     const dim3 blk(64, 4, 1), grid((g.Nx + 63) / 64, (g.Ny + 3) / 4, g.Nz);
@@ -1099,7 +1100,7 @@ static LineGeom line_geom(int n, int tables, size_t e, size_t &lds) {
 }
 
 template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C, const T *src, T *out, int dense_out,
-                                       T divisor, hipStream_t st) {
+                                       StepScalar<T> divisor, hipStream_t st) {
     const DevGrid<T> &g = C.g;
     const size_t e = sizeof(C2<T>);
     const size_t budget = 64 * 1024;
@@ -1173,16 +1174,16 @@ template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C,
 
 #ifndef OM_ONLY_DOUBLE
 template void launch_poisson_residual<float>(const Ctx<float> &, const RefineOp &, const float *, int64_t, int64_t,
-                                             const double *, double, float *, hipStream_t);
+                                             const double *, StepScalar<float>, float *, hipStream_t);
 template void launch_add_correction<float>(const DevGrid<float> &, float *, int64_t, int64_t, const float *, hipStream_t);
-template void launch_poisson<float>(const PoissonPlan<float> &, const Ctx<float> &, const float *, float *, int, float,
+template void launch_poisson<float>(const PoissonPlan<float> &, const Ctx<float> &, const float *, float *, int, StepScalar<float>,
                                     hipStream_t);
 #endif
 #ifndef OM_ONLY_FLOAT
 template void launch_poisson_residual<double>(const Ctx<double> &, const RefineOp &, const double *, int64_t, int64_t,
-                                              const double *, double, double *, hipStream_t);
+                                              const double *, StepScalar<double>, double *, hipStream_t);
 template void launch_add_correction<double>(const DevGrid<double> &, double *, int64_t, int64_t, const double *, hipStream_t);
-template void launch_poisson<double>(const PoissonPlan<double> &, const Ctx<double> &, const double *, double *, int, double,
+template void launch_poisson<double>(const PoissonPlan<double> &, const Ctx<double> &, const double *, double *, int, StepScalar<double>,
                                      hipStream_t);
 #endif
 

@@ -16,6 +16,18 @@ namespace om {
 constexpr int kMaxTracers = OM_MAX_TRACERS;
 constexpr int kMaxFields = OM_MAX_FIELDS;
 
+#define OM_CONSTANT __attribute__((address_space(4)))   // memory that no kernel writes while one reads it so
+
+// A number of the time step: by value, or (a captured step, whose arguments are fixed while Δt changes)
+// at an address of device memory that the stream wrote before.
+template <class T> struct StepScalar {
+    T value;
+    const T *mem;
+    StepScalar(T v, const T *m = nullptr) : value(v), mem(m) {}
+    StepScalar() = default;
+    __device__ __forceinline__ T get() const { return mem ? *(const OM_CONSTANT T *)mem : value; }
+};
+
 template <class T> struct Vec2;
 template <> struct Vec2<float> { using type = float2; };
 template <> struct Vec2<double> { using type = double2; };

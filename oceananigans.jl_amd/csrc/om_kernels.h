@@ -642,7 +642,8 @@ template <class T> struct CtxArgs {
 };
 
 template <class T> struct RKArgs {
-    T dt, gamma, zeta;
+    StepScalar<T> dt;
+    T gamma, zeta;
     int first;
     int nfields;
 };
@@ -777,10 +778,10 @@ template <class T> void launch_closure(const Ctx<T> &C, hipStream_t st, bool fix
 template <class T> bool tiled_closure_supported(const Ctx<T> &C);
 template <class T> void launch_closure_tiled(const Ctx<T> &C, int kchunk, hipStream_t st);
 template <class T> void launch_hydrostatic(const Ctx<T> &C, hipStream_t st);
-template <class T> void launch_rk3(const Ctx<T> &C, T dt, T gamma, T zeta, int first, int nfields, hipStream_t st);
+template <class T> void launch_rk3(const Ctx<T> &C, StepScalar<T> dt, T gamma, T zeta, int first, int nfields, hipStream_t st);
 // U −= dtp·∇p (phi = 0: p is the pressure) or U −= ∇ϕ (phi = 1: ϕ = p·Δt, as the reference stores it)
 // wrap = 1: periodic x and y without an immersed bottom; p's halos are not read
-template <class T> void launch_correct(const Ctx<T> &C, T dtp, int phi, hipStream_t st, int wrap = 0);
+template <class T> void launch_correct(const Ctx<T> &C, StepScalar<T> dtp, int phi, hipStream_t st, int wrap = 0);
 // mask_immersed_field! of a field at location loc (0 ccc, 1 fcc, 2 cfc, 3 ccf) on an immersed grid
 // (launch_mask_velocities: u, v and w at theirs)
 template <class T> void launch_mask(const DevGrid<T> &g, T *f, int loc, hipStream_t st);
@@ -878,15 +879,20 @@ template <class T> void cg_true_residual(const DevGrid<T> &g, const double *x, c
 template <class T> void cg_gauged_norm(const DevGrid<T> &g, const double *e, double mean, double *partial, double *out,
                                        hipStream_t st);
 template <class T> void launch_divergence(const Ctx<T> &C, T *out, hipStream_t st);
+// mem[0 .. 3] ← v: the numbers of a captured step (StepScalar)
+template <class T> struct StepTimes {
+    T v[4];
+};
+template <class T> void launch_step_times(const StepTimes<T> &t, T *mem, hipStream_t st);
 template <class T> void launch_halos(const DevGrid<T> &g, const HaloJob<T> &J, hipStream_t st);
-// Solve ∇²ϕ = source; writes ϕ / divisor into `out` (the nonhydrostatic pressure p/Δt when
-// called from the pressure correction, divisor = 1 otherwise).
 // whether the X-forward pass forms ∇·U of the state without reading a halo
 template <class T> bool poisson_source_reads_no_halo(const Ctx<T> &C) {
     return !C.g.kbot && C.g.tx != OM_FLAT && C.g.ty != OM_FLAT;
 }
+// Solve ∇²ϕ = source; writes ϕ / divisor into `out` (the nonhydrostatic pressure p/Δt when
+// called from the pressure correction, divisor = 1 otherwise).
 template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C, const T *src, T *out, int dense_out,
-                                       T divisor, hipStream_t st);
+                                       StepScalar<T> divisor, hipStream_t st);
 
 // FP64 iterative refinement of a Poisson solve.  Residual r = b − ∇²p in FP64 arithmetic, stored
 // dense in T: ∇² is the operator the FFT / Fourier–tridiagonal solver inverts (periodic x, y;
@@ -899,7 +905,7 @@ struct RefineOp {
     const double *idzc;        // from the configuration's FP64 face heights (stretched z)
 };
 template <class T> void launch_poisson_residual(const Ctx<T> &C, const RefineOp &L, const T *p, int64_t psy, int64_t psz,
-                                                const double *b64, double divisor, T *r, hipStream_t st);
+                                                const double *b64, StepScalar<T> divisor, T *r, hipStream_t st);
 template <class T> void launch_add_correction(const DevGrid<T> &g, T *p, int64_t psy, int64_t psz, const T *d, hipStream_t st);
 
 // diagnostics reductions (om_diagnostics.hip); partial holds 3·1024 doubles, out 3 doubles

@@ -812,6 +812,7 @@ template <class T, int NF> struct KRk3Batched {
 template <class T, int NF> __device__ __forceinline__ void KRk3Batched<T, NF>::run(const RkPack<T> &A, const Blk &B) {
     const Ctx<T> &C = A.C;
     const RKArgs<T> &a = A.a;
+    const T dt = a.dt.get();
     const int i = B.x * blockDim.x + threadIdx.x;
     const int j = B.y * blockDim.y + threadIdx.y;
     const int k = B.z;
@@ -836,8 +837,8 @@ template <class T, int NF> __device__ __forceinline__ void KRk3Batched<T, NF>::r
             if (changed) C.s.Gn[f][o] = g;
         }
         if (f == 2 && bz && k == 0 && C.g.Nz > 1) continue;   // exclude_periphery for w
-        if (a.first) C.s.U[f][o] = Um[f] + a.dt * a.gamma * g;
-        else C.s.U[f][o] = Um[f] + a.dt * (a.gamma * g + a.zeta * Gp[f]);
+        if (a.first) C.s.U[f][o] = Um[f] + dt * a.gamma * g;
+        else C.s.U[f][o] = Um[f] + dt * (a.gamma * g + a.zeta * Gp[f]);
     }
 }
 
@@ -848,6 +849,7 @@ template <class T> struct KRk3 {
 template <class T> __device__ __forceinline__ void KRk3<T>::run(const RkPack<T> &A, const Blk &B) {
     const Ctx<T> &C = A.C;
     const RKArgs<T> &a = A.a;
+    const T dt = a.dt.get();
     const int i = B.x * blockDim.x + threadIdx.x;
     const int j = B.y * blockDim.y + threadIdx.y;
     const int k = B.z;
@@ -865,8 +867,8 @@ template <class T> __device__ __forceinline__ void KRk3<T>::run(const RkPack<T> 
         }
         if (f == 2 && bz && k == 0 && C.g.Nz > 1) continue;   // exclude_periphery for w
         T *U = C.s.U[f];
-        if (a.first) U[o] += a.dt * a.gamma * G;
-        else U[o] += a.dt * (a.gamma * G + a.zeta * C.s.Gm[f][o]);
+        if (a.first) U[o] += dt * a.gamma * G;
+        else U[o] += dt * (a.gamma * G + a.zeta * C.s.Gm[f][o]);
     }
 }
 
@@ -881,7 +883,7 @@ constexpr int kCorrectLevels = 8;
 
 template <class T> struct CorrectArgs {
     Ctx<T> C;
-    T dtp;
+    StepScalar<T> dtp;
     int phi;
     int wrap;   // periodic x and y, no immersed bottom: neighbours across the edges by wrapped index
 };
@@ -891,7 +893,7 @@ template <class T> struct KCorrect {
 };
 template <class T> __device__ __forceinline__ void KCorrect<T>::run(const CorrectArgs<T> &A, const Blk &B) {
     const Ctx<T> &C = A.C;
-    const T dtp = A.dtp;
+    const T dtp = A.dtp.get();
     const int phi = A.phi;
     const int i = B.x * blockDim.x + threadIdx.x;
     const int j = B.y * blockDim.y + threadIdx.y;
@@ -1026,7 +1028,7 @@ template <class T> void launch_hydrostatic(const Ctx<T> &C, hipStream_t st) {
     }
     launch_k<KHydrostatic<T>>(dim3((C.g.Nx + 63) / 64, C.g.Ny), dim3(64, kHyWaves), 0, st, CtxArgs<T>{C});
 }
-template <class T> void launch_rk3(const Ctx<T> &C, T dt, T gamma, T zeta, int first, int nfields, hipStream_t st) {
+template <class T> void launch_rk3(const Ctx<T> &C, StepScalar<T> dt, T gamma, T zeta, int first, int nfields, hipStream_t st) {
     dim3 blk(64, 4, 1);
     const RkPack<T> A{C, RKArgs<T>{dt, gamma, zeta, first, nfields}};
     const dim3 grid = cell_grid(C.g.Nx, C.g.Ny, C.g.Nz, blk);
@@ -1037,7 +1039,7 @@ template <class T> void launch_rk3(const Ctx<T> &C, T dt, T gamma, T zeta, int f
         default: launch_k<KRk3<T>>(grid, blk, 0, st, A);
     }
 }
-template <class T> void launch_correct(const Ctx<T> &C, T dtp, int phi, hipStream_t st, int wrap) {
+template <class T> void launch_correct(const Ctx<T> &C, StepScalar<T> dtp, int phi, hipStream_t st, int wrap) {
     dim3 blk(64, 4, 1);
     launch_k<KCorrect<T>>(cell_grid(C.g.Nx, C.g.Ny, (C.g.Nz + kCorrectLevels - 1) / kCorrectLevels, blk), blk, 0, st,
                           CorrectArgs<T>{C, dtp, phi, wrap});
@@ -1055,6 +1057,13 @@ template <class T> void launch_mask_velocities(const DevGrid<T> &g, T *const *U,
     const int nk = mask_levels(g);   // (u and v have a halo level above Nz, where nothing is masked)
     dim3 blk(64, 4, 1);
     hipLaunchKernelGGL(k_mask<T>, cell_grid(g.Nx, g.Ny, 3 * nk, blk), blk, 0, st, g, U[0], U[1], U[2], 1, nk);
+}
+template <class T> __global__ void k_step_times(StepTimes<T> t, T *mem) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) if ((int)threadIdx.x == q) mem[q] = t.v[q];
+}
+template <class T> void launch_step_times(const StepTimes<T> &t, T *mem, hipStream_t st) {
+    hipLaunchKernelGGL(k_step_times<T>, dim3(1), dim3(64), 0, st, t, mem);
 }
 template <class T> void launch_divergence(const Ctx<T> &C, T *out, hipStream_t st) {
     dim3 blk(64, 4, 1);
@@ -1092,11 +1101,12 @@ template <class T> void launch_halos(const DevGrid<T> &g, const HaloJob<T> &J, h
     template void launch_tend_flat<T>(const Ctx<T> &, hipStream_t);                                \
     template void launch_closure<T>(const Ctx<T> &, hipStream_t, bool);                            \
     template void launch_hydrostatic<T>(const Ctx<T> &, hipStream_t);                              \
-    template void launch_rk3<T>(const Ctx<T> &, T, T, T, int, int, hipStream_t);                    \
-    template void launch_correct<T>(const Ctx<T> &, T, int, hipStream_t, int);                          \
+    template void launch_rk3<T>(const Ctx<T> &, StepScalar<T>, T, T, int, int, hipStream_t);                    \
+    template void launch_correct<T>(const Ctx<T> &, StepScalar<T>, int, hipStream_t, int);                          \
     template void launch_mask<T>(const DevGrid<T> &, T *, int, hipStream_t);                           \
     template void launch_mask_velocities<T>(const DevGrid<T> &, T *const *, hipStream_t);              \
     template void launch_divergence<T>(const Ctx<T> &, T *, hipStream_t);                          \
+    template void launch_step_times<T>(const StepTimes<T> &, T *, hipStream_t);                    \
     template void launch_halos<T>(const DevGrid<T> &, const HaloJob<T> &, hipStream_t);
 // Each precision is compiled in its own object: FP64 without FMA contraction (the reference's
 // rounding: Julia never fuses a*b+c implicitly), FP32 with it.

@@ -353,8 +353,8 @@ class NonhydrostaticModel:
                    step_graphs=None, conv_tiled=None, wgrad_mfma=None):
         """Launch-shape choices: tendency_kernel 'tiled' (default where supported) or 'generic';
         kchunk = z levels per block of the tiled kernel; step_graphs: time_step replays captured
-        hipGraphs of two steps and, after several with one Δt, of single steps (default) or issues every launch; conv_tiled: the learned preconditioner's
-        convolutions with LDS-staged input tiles (default) or not.  Results do not depend on them.
+        hipGraphs of two steps and, after the first few, of single steps (default) or issues every launch;
+        conv_tiled: the learned preconditioner's convolutions with LDS-staged input tiles (default) or not.  Results do not depend on them.
         poisson_refinement: one FP64 iterative-refinement step after each FFT / Fourier–tridiagonal
         Poisson solve (off by default)."""
         if wgrad_mfma is not None:
