@@ -529,7 +529,6 @@ template <class T> struct ModelT : ModelBase {
         P.lx = upload(eigen<T>(g.Nx, hg.Lx, g.tx, 1));
         P.ly = upload(eigen<T>(g.Ny, hg.Ly, g.ty, 1));
         P.lz = upload(eigen<T>(g.Nz, hg.Lz, g.tz, g.tz == OM_BOUNDED ? 2 : 1));
-        P.eps10 = T(10) * std::numeric_limits<T>::epsilon();
         {
             // the inverse squared spacings behind the solver's eigenvalues (eigen(): h = T(L / N))
             auto ih2 = [](T L, int N, int topo) { if (topo == OM_FLAT) return 0.0; const double h = (double)(T)(L / T(N)); return 1.0 / (h * h); };

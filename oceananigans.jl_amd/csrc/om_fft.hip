@@ -14,6 +14,7 @@
 // src/Solvers/fourier_tridiagonal_poisson_solver.jl:231-260, src/Solvers/batched_tridiagonal_solver.jl:211-243.
 #include <hip/hip_runtime.h>
 
+#include <limits>
 #include <stdexcept>
 
 #include "om_internal.h"
@@ -732,16 +733,19 @@ template <class T, bool MIXED> __device__ __forceinline__ void KZPass<T, MIXED>:
 // The (0,0) column is singular, and the reference elides its last pivot: the top level's equation is
 // the one that a source with a volume integral leaves unmet.  Here that level's source is replaced by
 // what makes the column solvable, which has the same solution, and the closing pivot is elided;
-// the constant this leaves is removed with the column mean (ϕ -= mean(ϕ), :253).
+// the constant this leaves is removed with the column mean (ϕ -= mean(ϕ), :253).  No other column
+// loses a level: the reference's pivot guard (10·ε) is there for the rounding of a pivot that is a difference, and in
+// FP32 it also takes the closing level of every column with λ · depth below 1e-6 (a 100 m layer over
+// 2000 km) and with it the column's solution; here pivots are sums of positive numbers.
 // ---------------------------------------------------------------------------------------------
 template <class T> struct TriArgs {
     DevGrid<T> g;
     C2<T> *S;
     int Mx, Ms;
     const T *lx, *ly;
-    T eps10;
-    T zscale;   // (1 / L_backward_norm) applied later; unused here
 };
+// whether a closing pivot can be divided by (0 in the singular column)
+template <class T> __device__ __forceinline__ bool closes(T pivot) { return pivot >= std::numeric_limits<T>::min(); }
 
 template <class T> constexpr int tri_batch() { return sizeof(T) == 4 ? 16 : 8; }
 // LDS bytes of a block of bw columns
@@ -795,8 +799,7 @@ __global__ void __launch_bounds__(64) k_tridiag(TriArgs<T> A, C2<T> *__restrict_
         excess = d * lam + excess * ratio;
         const T pivot = next + excess;
         ratio = ft_div<T>(next, pivot);
-        if (q == 0 || pivot > A.eps10) phi = cmk<T>(ft_div<T>(before * phi.x - f.x, pivot), ft_div<T>(before * phi.y - f.y, pivot));
-        else phi = cmk<T>(T(0), T(0));
+        phi = cmk<T>(ft_div<T>(before * phi.x - f.x, pivot), ft_div<T>(before * phi.y - f.y, pivot));
         tt[k * bw + c] = ratio;
         if (KEEP) ph[k * bw + c] = phi;
         else if (store) S[at(k)] = phi;
@@ -847,7 +850,7 @@ __global__ void __launch_bounds__(64) k_tridiag(TriArgs<T> A, C2<T> *__restrict_
         const C2<T> pb = cmk<T>(__shfl(phi.x, c), __shfl(phi.y, c)), pt = cmk<T>(__shfl(phi.x, c + bw), __shfl(phi.y, c + bw));
         const T below = coupling(mid), above = coupling(mid + 1);
         const T pivot = spacing(mid) * lam + (eb + et);
-        if (!singular && pivot > A.eps10)
+        if (!singular && closes<T>(pivot))
             x = cmk<T>(ft_div<T>((below * pb.x - fmid.x) + above * pt.x, pivot), ft_div<T>((below * pb.y - fmid.y) + above * pt.y, pivot));
         else x = cmk<T>(T(0), T(0));
     }
@@ -983,7 +986,6 @@ __global__ void __launch_bounds__(64, 2) k_tridiag_short(TriArgs<T> A, C2<T> *__
         const T pivot = next[down][q] + excess;
         ratio = ft_div<T>(next[down][q], pivot);
         phi = cmk<T>(ft_div<T>(before[down][q] * phi.x - s.x, pivot), ft_div<T>(before[down][q] * phi.y - s.y, pivot));
-        if (!(pivot > A.eps10)) phi = cmk<T>(T(0), T(0));
         f[q] = phi;
         t[q] = ratio;
     }
@@ -994,7 +996,7 @@ __global__ void __launch_bounds__(64, 2) k_tridiag_short(TriArgs<T> A, C2<T> *__
         const T eb = __shfl(excess, c) * __shfl(ratio, c), et = __shfl(excess, c + bw) * __shfl(ratio, c + bw);
         const C2<T> pb = cmk<T>(__shfl(phi.x, c), __shfl(phi.y, c)), pt = cmk<T>(__shfl(phi.x, c + bw), __shfl(phi.y, c + bw));
         const T pivot = dzc[mid] * lam + (eb + et);
-        if (!singular && pivot > A.eps10)
+        if (!singular && closes<T>(pivot))
             x = cmk<T>(ft_div<T>((below * pb.x - fmid.x) + above * pt.x, pivot), ft_div<T>((below * pb.y - fmid.y) + above * pt.y, pivot));
         else x = cmk<T>(T(0), T(0));
     }
@@ -1135,10 +1137,10 @@ template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C,
     T scale = T(1) / (T(M) * T(Ny));
     if (z_active) {
         if (P.tridiagonal) {
-            TriArgs<T> A{g, P.S, Mx, P.Ms, P.lx, P.ly, P.eps10, T(1)};
+            TriArgs<T> A{g, P.S, Mx, P.Ms, P.lx, P.ly};
             const int64_t ncol = (int64_t)P.Ms * Ny;
             const int half = Nz >> 1;
-            // registers hold chains of up to 64 levels in FP32 (234 VGPRs, two waves a SIMD) and 32 in FP64 (247)
+            // registers hold chains of up to 64 levels in FP32 (241 VGPRs, two waves a SIMD) and 32 in FP64 (247)
             constexpr int most = sizeof(T) == 4 ? 64 : 32;
             if (half <= most) {
                 const auto kernel = half <= 16 ? &k_tridiag_short<T, 16> : (half <= 32 ? &k_tridiag_short<T, 32> : &k_tridiag_short<T, most>);

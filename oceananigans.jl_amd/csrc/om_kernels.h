@@ -693,7 +693,6 @@ template <class T> struct PoissonPlan {
     int zmode;                           // 0 Periodic z, 1 Bounded z via a length-Nz DCT
     int Lz_norm;                         // normalisation of the z transform pair: Nz (Periodic), 2·Nz (Bounded)
     int tridiagonal;                     // Fourier–tridiagonal z solve (stretched z)
-    T eps10;                             // 10·eps(FT): the Thomas pivot guard
 };
 
 // Lines of the FFT passes staged per block: the largest power of two R ≤ 16 with R·n ≤ 4096 whose
