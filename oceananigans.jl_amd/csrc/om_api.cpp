@@ -1306,10 +1306,8 @@ static std::string validate(const om_config_t *c) {
         const int Nz = c->N[2];
         bool ok = om::fft_lines_per_block(xl, xl, e) > 0 && om::fft_lines_per_block(c->N[1], c->N[1], e) > 0;
         const bool z_tridiagonal = c->pressure_solver == OM_SOLVER_FOURIER_TRIDIAGONAL || c->z_faces;
-        if (c->topology[2] != OM_FLAT && !z_tridiagonal) {
-            const int L = (c->topology[2] == OM_BOUNDED && Nz % 2 == 1) ? 2 * Nz : Nz;
-            ok = ok && om::fft_lines_per_block(L, L + (c->topology[2] == OM_BOUNDED && Nz % 2 == 0 ? Nz : 0), e) > 0;
-        }
+        if (c->topology[2] != OM_FLAT && !z_tridiagonal)
+            ok = ok && om::fft_lines_per_block(Nz, om::z_line_tables(Nz, c->topology[2] == OM_BOUNDED), e) > 0;
         if (!ok) return "grid too large for the FFT pressure solver: a line of Nx/2, Ny or Nz points and its tables must fit in 64 KiB of LDS";
     }
     if (c->bottom_height) {

@@ -1159,7 +1159,7 @@ template <class T> void launch_poisson(const PoissonPlan<T> &P, const Ctx<T> &C,
                                    g.idzf);
             }
         } else {
-            const LineGeom Lz = line_geom(Nz, Nz + (P.zmode == 1 ? Nz : 0), e, lds);
+            const LineGeom Lz = line_geom(Nz, z_line_tables(Nz, P.zmode == 1), e, lds);
             ZArgs<T> A{g, P.S, P.tw_z, P.st_z, P.tw_dct, Mx, P.Ms, P.zmode, P.lx, P.ly, P.lz, Lz};
             by_length(KZPass<T, false>(), KZPass<T, true>(), Nz, (P.Ms * Ny + Lz.R - 1) / Lz.R, lds, A);
             scale = T(1) / ((T(M) * T(Ny)) * T(P.Lz_norm));

@@ -708,6 +708,9 @@ inline int fft_lines_per_block(int n, int tables, size_t elem) {
     return 0;
 }
 
+// table entries of a z line: its twiddles and, with Bounded z, the DCT's c_k
+inline int z_line_tables(int Nz, bool bounded) { return bounded ? 2 * Nz : Nz; }
+
 // Levels per block (the z chunk) of a kernel whose blocks march up a tile of columns.  With n =
 // tiles · chunks blocks, m = n / CUs of them per CU and `occ` resident at once, a level of a full CU
 // costs each block one unit of VALU time, a level of a lone block `lat` units of latency, and a block
