@@ -160,11 +160,12 @@ template <class T> __global__ void __launch_bounds__(256) k_tendencies(Ctx<T> C,
 // twice.  On a small grid a launch lasts as long as one wave, and that is mostly the fetching of its
 // instructions, so one loop body serves both directions of every field, by pointers and strides.  128 × 128
 // FP64: 17 µs in k_tendencies, 14 with each field's two fluxes spelled out, 4.7 here.  The fluxes are
-// those of Ctx (F_Uu … F_cy), operand for operand: the same bits in FP64.
+// those of Ctx (F_Uu … F_cy) and the sums those of k_tendencies, operand for operand and expression for
+// expression (which decides the contractions in FP32: a viscous flux takes its area where it is differenced): the same bits.
 // ----------------------------------------------------------------------------------------
 constexpr int kFlatTile = 15;
 template <class T, int ADV> __global__ void __launch_bounds__(256) k_tend_flat(Ctx<T> C) {
-    __shared__ T fx[2][256], fy[2][256];   // advective, viscous / diffusive
+    __shared__ T fx[2][256], fy[2][256];   // advective, viscous / diffusive (not yet times area)
     const int tid = threadIdx.x, a = tid & 15, b = tid >> 4, field = blockIdx.z;
     const int ic = blockIdx.x * kFlatTile + a, jc = blockIdx.y * kFlatTile + b;
     const int i = min(ic, C.g.Nx), j = min(jc, C.g.Ny);   // (the last cells' far faces are the last evaluated)
@@ -202,20 +203,20 @@ template <class T, int ADV> __global__ void __launch_bounds__(256) k_tend_flat(C
     T vx = T(0), vy = T(0);
     if (clo) {
         if (field == 0) {   // x: at centre i − 1, y: at edge j
-            vx = C.Axc(k) * C.f_ux(i - 1, j, k);
-            vy = C.Ayc(k) * C.f_uy(i, j, k);
+            vx = C.f_ux(i - 1, j, k);
+            vy = C.f_uy(i, j, k);
         } else if (field == 1) {
-            vx = C.Axc(k) * C.f_uy(i, j, k);
-            vy = C.Ayc(k) * C.f_vy(i, j - 1, k);
+            vx = C.f_uy(i, j, k);
+            vy = C.f_vy(i, j - 1, k);
         } else if (field == 2) {
-            vx = C.Axf(k) * C.f_uz(i, j, k);
-            vy = C.Ayf(k) * C.f_vz(i, j, k);
+            vx = C.f_uz(i, j, k);
+            vy = C.f_vz(i, j, k);
         } else {
 #pragma unroll
             for (int n = 0; n < kMaxTracers; ++n) {
                 if (field != 3 + n) continue;
-                vx = C.Axc(k) * C.q_x(n, C.s.U[3 + n], i, j, k);
-                vy = C.Ayc(k) * C.q_y(n, C.s.U[3 + n], i, j, k);
+                vx = C.q_x(n, C.s.U[3 + n], i, j, k);
+                vy = C.q_y(n, C.s.U[3 + n], i, j, k);
             }
         }
     }
@@ -233,15 +234,19 @@ template <class T, int ADV> __global__ void __launch_bounds__(256) k_tend_flat(C
         auto q = [&](int ii, int jj) { return A * C.ld(o, ii, jj, k); };
         const T I = field == 0 ? T(0.5) * (T(0.5) * (q(i - 1, j) + q(i, j)) + T(0.5) * (q(i - 1, j + 1) + q(i, j + 1)))
                                : T(0.5) * (T(0.5) * (q(i, j - 1) + q(i + 1, j - 1)) + T(0.5) * (q(i, j) + q(i + 1, j)));
-        const T cor = (T(0.5) * (C.ph.f + C.ph.f)) * I * recip<T>(A);
-        G = field == 0 ? G + cor : G - cor;
+        if (field == 0) G += (T(0.5) * (C.ph.f + C.ph.f)) * I * recip<T>(A);
+        else G -= (T(0.5) * (C.ph.f + C.ph.f)) * I * recip<T>(A);
     }
     if (C.ph.hydrostatic && field < 2) {
         const T *d = field == 0 ? C.s.dxpHY : C.s.dypHY;
         const T dp = d ? C.ld(d, i, j, k) : C.ld(C.s.pHY, i, j, k) - (field == 0 ? C.ld(C.s.pHY, i - 1, j, k) : C.ld(C.s.pHY, i, j - 1, k));
         G -= dp * (field == 0 ? C.g.idx : C.g.idy);
     }
-    if (clo) G -= iV * (((fx[1][tid + 1] - fx[1][tid]) + (fy[1][tid + 16] - fy[1][tid])) + T(0));
+    if (clo) {
+        const T Ax = field == 2 ? C.Axf(k) : C.Axc(k), Ay = field == 2 ? C.Ayf(k) : C.Ayc(k);
+        const T sx = Ax * fx[1][tid + 1] - Ax * fx[1][tid], sy = Ay * fy[1][tid + 16] - Ay * fy[1][tid];
+        G -= iV * ((sx + sy) + T(0));
+    }
     T *out = C.s.Gn[0];
 #pragma unroll
     for (int f = 1; f < kMaxFields; ++f) if (f == field) out = C.s.Gn[f];
