@@ -316,9 +316,10 @@ int om_set_tuning(om_model_t *m, int32_t key, int32_t value);
 int om_get_tuning(const om_model_t *m, int32_t key, int32_t *value);
 
 /* Autotuner (no reference counterpart): times the tiled tendency and closure kernels, each on
- * its own, on the model's current state for z-chunk lengths 4 .. 64 and keeps the fastest for
- * each (OM_TUNE_KCHUNK sets both).  Results do not depend on the choice.  *kchunk (may be NULL)
- * receives the tendency kernel's. */
+ * its own, on the model's current state for z-chunk lengths 1 .. 64 (the tendency kernel's: 4 .. 64)
+ * and keeps the fastest for each, the one in use among them (OM_TUNE_KCHUNK sets both).  Results
+ * do not depend on the choice.  *kchunk (may be NULL) receives the tendency kernel's.  Grids whose
+ * tendency chunk is below 4 by default (some 64^3 cells and fewer) are best left to their default. */
 int om_autotune(om_model_t *m, int32_t *kchunk);
 
 /* Ensembles of independent models (no reference counterpart for NonhydrostaticModel: the
