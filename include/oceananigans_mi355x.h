@@ -286,8 +286,11 @@ int om_set_phase_timing(om_model_t *m, int32_t enable);
 int om_last_step_timing(const om_model_t *m, double *ms_total, double *ms_per_phase, int32_t *launches_per_phase,
                         int32_t nphases);
 
-/* launch-shape choices of this library (no reference counterpart).  Results do not depend on
- * them: every tendency kernel gives identically rounded tendencies. */
+/* launch-shape choices of this library (no reference counterpart).  In FP64 results do not depend on
+ * them: the tendency and closure kernels round identically.  In FP32 they do so too but for one: the
+ * tiled WENO kernel takes a face's area once, after the interpolation of the advecting velocity, so its
+ * momentum tendencies differ from the thread-per-cell kernel's by rounding (2e-7 of the largest value) unless
+ * the areas are powers of two.  Chunks, graphs and the order of launches change no bit. */
 #define OM_TUNE_TENDENCY_KERNEL 0   /* 0: z-marching LDS-tiled tendency and closure kernels where supported
                                        (default); 1: thread-per-cell kernels */
 #define OM_TUNE_KCHUNK          1   /* z levels marched by one block of the tiled kernels (default: by the grid's size;

@@ -61,8 +61,9 @@ template <class T> struct RC {
 // a sum of products p₁ + p₂ + … + pₙ, evaluated left to right, becomes
 // muladd(pₙ, muladd(…, muladd(p₂, p₁))), i.e. the first product rounded on its own and every later
 // one fused into the running sum, and a product a·b·c splits as (a·b, c).  The generic templates
-// below (the FP64 path) spell these fused multiply-adds out and contract nothing else, so that
-// identical inputs give identically rounded values; FP64 smoothness indicators on raw stencil
+// below (the FP64 path: β, WENO3, Centered) spell these fused multiply-adds out and contract nothing else, so that
+// identical inputs give the reference's rounding; weno5<double>'s weights and weighted sum alone
+// round otherwise, and less (see there).  FP64 smoothness indicators on raw stencil
 // values cancel heavily when the values carry a large offset, which makes the order observable.
 
 // Smoothness quadratic form ψ₁(k₀ψ₁ + k₁ψ₂ + k₂ψ₃) + ψ₂(k₃ψ₂ + k₄ψ₃) + ψ₃ψ₃k₅

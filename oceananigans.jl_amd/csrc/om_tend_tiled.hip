@@ -23,7 +23,7 @@
 //
 // The flux formulas, their operand order and the tendency assembly are those of k_tendencies
 // (om_kernels.hip), which follows nonhydrostatic_tendency_kernel_functions.jl:71-302; the two
-// kernels give identically rounded results.
+// kernels give identically rounded results, but in FP32 where areas are no powers of two: acen4 takes them once.
 #include <hip/hip_runtime.h>
 
 #include "om_batch.h"

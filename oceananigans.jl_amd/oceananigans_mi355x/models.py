@@ -354,7 +354,9 @@ class NonhydrostaticModel:
         """Launch-shape choices: tendency_kernel 'tiled' (default where supported) or 'generic';
         kchunk = z levels per block of the tiled kernel; step_graphs: time_step replays captured
         hipGraphs of two steps and, after the first few, of single steps (default) or issues every launch;
-        conv_tiled: the learned preconditioner's convolutions with LDS-staged input tiles (default) or not.  Results do not depend on them.
+        conv_tiled: the learned preconditioner's convolutions with LDS-staged input tiles (default) or not.
+        Results do not depend on them, but for the rounding of FP32 momentum tendencies between the tiled
+        WENO kernel and the generic one (2e-7 of the largest).
         poisson_refinement: one FP64 iterative-refinement step after each FFT / Fourier–tridiagonal
         Poisson solve (off by default)."""
         if wgrad_mfma is not None:
